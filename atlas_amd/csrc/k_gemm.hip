@@ -40,9 +40,11 @@ typedef double d2 __attribute__((ext_vector_type(2)));
 template <typename T> struct Mfma;
 template <> struct Mfma<double> {
   typedef d4 acc_t;
-  typedef d2 vec_t;                 /* one 16-byte global load */
+  typedef d2 vec_t;                 /* one 16-byte load */
+  typedef d2 __attribute__((aligned(8))) uvec_t;   /* the same from any element address */
   static constexpr int VEC = 2;
   static constexpr int BK = 16;     /* 2 x 36 KB LDS: two workgroups per CU */
+  static constexpr int BKS = 16;    /* K slice of the small tiles */
   static constexpr int PADK = 2;    /* LDS row = 18 doubles = 144 B */
   static constexpr int PADR = 2;    /* [k][row] tiles: 130 doubles per k */
   __device__ static acc_t mma(double a, double b, acc_t c) {
@@ -54,8 +56,10 @@ template <> struct Mfma<double> {
 template <> struct Mfma<float> {
   typedef f4 acc_t;
   typedef f4 vec_t;
+  typedef f4 __attribute__((aligned(4))) uvec_t;
   static constexpr int VEC = 4;
   static constexpr int BK = 16;     /* 2 x 20 KB LDS: three workgroups per CU */
+  static constexpr int BKS = 32;
   static constexpr int PADK = 4;    /* LDS row = 20 floats = 80 B */
   static constexpr int PADR = 4;    /* [k][row] tiles: 132 floats per k */
   __device__ static acc_t mma(float a, float b, acc_t c) {
@@ -75,42 +79,44 @@ struct GemmArgs {
   int tri;
   int tiles_m, tiles_n;
   int per_xcd;            /* tiles per XCD slot in the remapped numbering */
-  int vec_a, vec_b;       /* 16-byte vector loads allowed */
   const int *abort_flag;
 };
 
-/* Load one BKxBM (or BKxBN) slice of an operand into registers.
- * KCONT: the operand's K index is contiguous in memory (op(A) with A
- * transposed, or op(B) with B not transposed).  rows = extent in M (or N).
+/* Load one BKxBM (or BKxBN) slice of an operand into registers, by NTH
+ * threads.  KCONT: the operand's K index is contiguous in memory (op(A) with
+ * A transposed, or op(B) with B not transposed).  rows = extent in M (or N).
  * Element (r, k) of the slice lives at P[k + r*ld] when KCONT, else at
- * P[r + k*ld]. */
-template <typename T, bool KCONT, int ROWS, int BK>
+ * P[r + k*ld].  Whole vectors are 16-byte loads whatever the address (the
+ * type says so, uvec_t): an odd leading dimension costs a split cache line
+ * now and then, where element loads took four instructions a vector
+ * (float, T x N, 1511 x 777 x 4001 in 128-tiles: 539 -> 373 us). */
+template <typename T, bool KCONT, int ROWS, int BK, int NTH = NT>
 struct SliceLoader {
   typedef Mfma<T> MF;
   static constexpr int VEC = MF::VEC;
-  static constexpr int NV = ROWS * BK / VEC / NT;   /* vectors per thread */
+  static constexpr int NV = ROWS * BK / VEC / NTH;  /* vectors per thread */
+  static_assert(NV * VEC * NTH == ROWS * BK, "a slice is whole vectors per thread");
   typename MF::vec_t v[NV];
 
-  __device__ void load(const T *P, long ld, int r0, int k0, int rows, int K,
-                       bool vec_ok, int tid) {
+  __device__ void load(const T *P, long ld, int r0, int k0, int rows, int K, int tid) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int lin = tid + NT * i;
+      const int lin = tid + NTH * i;
       int r, k;
       if (KCONT) { r = lin / (BK / VEC); k = (lin % (BK / VEC)) * VEC; }
       else       { k = lin / (ROWS / VEC); r = (lin % (ROWS / VEC)) * VEC; }
       const int gr = r0 + r, gk = k0 + k;
       if (KCONT) {
-        if (vec_ok && gr < rows && gk + VEC <= K) {
-          v[i] = *reinterpret_cast<const typename MF::vec_t *>(P + (size_t)gr * ld + gk);
+        if (gr < rows && gk + VEC <= K) {
+          v[i] = *reinterpret_cast<const typename MF::uvec_t *>(P + (size_t)gr * ld + gk);
         } else {
 #pragma unroll
           for (int e = 0; e < VEC; ++e)
             v[i][e] = (gr < rows && gk + e < K) ? P[(size_t)gr * ld + gk + e] : T(0);
         }
       } else {
-        if (vec_ok && gk < K && gr + VEC <= rows) {
-          v[i] = *reinterpret_cast<const typename MF::vec_t *>(P + (size_t)gk * ld + gr);
+        if (gk < K && gr + VEC <= rows) {
+          v[i] = *reinterpret_cast<const typename MF::uvec_t *>(P + (size_t)gk * ld + gr);
         } else {
 #pragma unroll
           for (int e = 0; e < VEC; ++e)
@@ -129,7 +135,7 @@ struct SliceLoader {
   __device__ void store(T *S, int tid) const {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int lin = tid + NT * i;
+      const int lin = tid + NTH * i;
       if (KCONT) {
         const int r = lin / (BK / VEC), k = (lin % (BK / VEC)) * VEC;
         *reinterpret_cast<typename MF::vec_t *>(S + r * LDK + k) = v[i];
@@ -223,8 +229,8 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(GemmArgs<T> g) {
   const int kt0 = kb / BK, kt1 = (ke + BK - 1) / BK;
 
   if (kt0 < kt1) {
-    la.load(g.A, g.lda, m0, kt0 * BK, g.M, g.K, g.vec_a, tid);
-    lb.load(g.B, g.ldb, n0, kt0 * BK, g.N, g.K, g.vec_b, tid);
+    la.load(g.A, g.lda, m0, kt0 * BK, g.M, g.K, tid);
+    lb.load(g.B, g.ldb, n0, kt0 * BK, g.N, g.K, tid);
     la.store(As[0], tid);
     lb.store(Bs[0], tid);
   }
@@ -239,8 +245,8 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(GemmArgs<T> g) {
   for (int kt = kt0; kt < kt1; ++kt) {
     const int cur = (kt - kt0) & 1;
     if (kt + 1 < kt1) {
-      la.load(g.A, g.lda, m0, (kt + 1) * BK, g.M, g.K, g.vec_a, tid);
-      lb.load(g.B, g.ldb, n0, (kt + 1) * BK, g.N, g.K, g.vec_b, tid);
+      la.load(g.A, g.lda, m0, (kt + 1) * BK, g.M, g.K, tid);
+      lb.load(g.B, g.ldb, n0, (kt + 1) * BK, g.N, g.K, tid);
     }
 #pragma unroll
     for (int kg = 0; kg < BK / 16; ++kg) {
@@ -273,6 +279,144 @@ __global__ __launch_bounds__(NT, 2) void gemm_kernel(GemmArgs<T> g) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         /* acc[i][j] holds D = (C tile)^T: D[n][m] */
+        const int row = m0 + wm + i * 16 + lr;
+        const int col = n0 + wn + j * 16 + MF::drow(lane, r);
+        if (row < g.M && col < g.N) {
+          if (g.tri == KX_LOWER && row < col) continue;
+          if (g.tri == KX_UPPER && row > col) continue;
+          if (g.tri == KX_CLOWER && (row >> 1) < col) continue;
+          if (g.tri == KX_CUPPER && (row >> 1) > col) continue;
+          T *c = g.C + (size_t)col * g.ldc + row;
+          T v = g.alpha * acc[i][j][r];
+          if (g.beta != T(0)) v += g.beta * *c;
+          *c = v;
+        }
+      }
+}
+
+/* The same product in smaller tiles, for shapes whose 128x128 tiles leave
+ * the chip idle: a TS x TS tile per workgroup (64: each of a group's four
+ * wavefronts 32x32; 32: 16x16), and KG groups of four wavefronts that split
+ * the tile's K slices between them in order (group g takes the g-th part)
+ * and add their sums through LDS in the order of the groups, so the result
+ * does not depend on timing and no workspace is needed.  What bounds it: a
+ * tile of a small product is a serial chain of K slices (load, barrier,
+ * MFMAs; ~0.5 us each), so KG shortens the chain and the smaller tile
+ * spreads the MFMAs (FP64: 64 cycles each) over more compute units; the
+ * price is operand traffic (2/TS of a load per FMA), which L2 carries. */
+template <typename T, int TA, int TB, int TS, int KG>
+__global__ __launch_bounds__(NT *KG) void gemm_small_kernel(GemmArgs<T> g) {
+  typedef Mfma<T> MF;
+  typedef typename MF::acc_t acc_t;
+  constexpr int BK = MF::BKS;
+  constexpr int NB = TS / 32;                    /* 16-blocks per wavefront side */
+  constexpr bool A_KCONT = (TA != KX_NOTRANS);
+  constexpr bool B_KCONT = (TB == KX_NOTRANS);
+  typedef SliceLoader<T, A_KCONT, TS, BK> LA;
+  typedef SliceLoader<T, B_KCONT, TS, BK> LB;
+  if (g.abort_flag && *g.abort_flag) return;
+
+  const int bid = blockIdx.x;
+  const int tile = g.tri ? bid : (bid & 7) * g.per_xcd + (bid >> 3);
+  const int ntiles = g.tiles_m * g.tiles_n;
+  if (tile >= ntiles) return;
+  const int per_group = GROUP_M * g.tiles_n;
+  const int first_m = (tile / per_group) * GROUP_M;
+  const int gsz = min(g.tiles_m - first_m, GROUP_M);
+  const int m0 = (first_m + (tile % per_group) % gsz) * TS;
+  const int n0 = ((tile % per_group) / gsz) * TS;
+  if (g.tri == KX_LOWER && m0 + TS - 1 < n0) return;
+  if (g.tri == KX_UPPER && n0 + TS - 1 < m0) return;
+  if (g.tri == KX_CLOWER && ((m0 + TS - 1) >> 1) < n0) return;
+  if (g.tri == KX_CUPPER && n0 + TS - 1 < (m0 >> 1)) return;
+
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x & (NT - 1), grp = threadIdx.x / NT;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int wm = (wave & 1) * (TS / 2), wn = (wave >> 1) * (TS / 2);
+  T *S = (T *)smem + (size_t)grp * 2 * (LA::SIZE + LB::SIZE);
+  T *As = S, *Bs = S + 2 * LA::SIZE;
+
+  acc_t acc[NB][NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+
+  /* every group runs as many steps as the first; one without a slice left
+   * only meets the barriers */
+  const int nk = (g.K + BK - 1) / BK, per = (nk + KG - 1) / KG;
+  const int kt0 = grp * per, kt1 = min(kt0 + per, nk);
+  LA la;
+  LB lb;
+  if (kt0 < kt1) {
+    la.load(g.A, g.lda, m0, kt0 * BK, g.M, g.K, tid);
+    lb.load(g.B, g.ldb, n0, kt0 * BK, g.N, g.K, tid);
+    la.store(As, tid);
+    lb.store(Bs, tid);
+  }
+  __syncthreads();
+  const int kq = (lane >> 4) * 4, lr = lane & 15;
+  for (int st = 0; st < per; ++st) {
+    const int kt = kt0 + st, cur = st & 1;
+    const bool more = kt + 1 < kt1;
+    if (more) {
+      la.load(g.A, g.lda, m0, (kt + 1) * BK, g.M, g.K, tid);
+      lb.load(g.B, g.ldb, n0, (kt + 1) * BK, g.N, g.K, tid);
+    }
+    if (kt < kt1) {
+      const T *a_ = As + cur * LA::SIZE, *b_ = Bs + cur * LB::SIZE;
+#pragma unroll
+      for (int kg = 0; kg < BK / 16; ++kg)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          T a[NB], b[NB];
+#pragma unroll
+          for (int i = 0; i < NB; ++i) {
+            a[i] = a_[LA::at(wm + i * 16 + lr, kg * 16 + kq + s)];
+            b[i] = b_[LB::at(wn + i * 16 + lr, kg * 16 + kq + s)];
+          }
+#pragma unroll
+          for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = MF::mma(b[j], a[i], acc[i][j]);
+        }
+    }
+    if (more) {
+      la.store(As + (cur ^ 1) * LA::SIZE, tid);
+      lb.store(Bs + (cur ^ 1) * LB::SIZE, tid);
+    }
+    __syncthreads();
+  }
+
+  if constexpr (KG > 1) {
+    /* the groups' sums, [group - 1][wavefront][block][lane] (the staging
+     * area, free after the last barrier) */
+    acc_t *red = (acc_t *)smem;
+    constexpr int PER = 4 * NB * NB * 64;
+    if (grp > 0) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          red[(grp - 1) * PER + (wave * NB * NB + i * NB + j) * 64 + lane] = acc[i][j];
+    }
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int q = 0; q < KG - 1; ++q)
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[i][j] += red[q * PER + (wave * NB * NB + i * NB + j) * 64 + lane];
+  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
         const int row = m0 + wm + i * 16 + lr;
         const int col = n0 + wn + j * 16 + MF::drow(lane, r);
         if (row < g.M && col < g.N) {
@@ -330,8 +474,8 @@ __global__ __launch_bounds__(NT, 1) void update_kernel(GemmArgs<T> g) {
 
   LA la;
   LB lb;
-  la.load(g.A, g.lda, m0, 0, g.M, g.K, g.vec_a, tid);
-  lb.load(g.B, g.ldb, n0, 0, g.N, g.K, g.vec_b, tid);
+  la.load(g.A, g.lda, m0, 0, g.M, g.K, tid);
+  lb.load(g.B, g.ldb, n0, 0, g.N, g.K, tid);
   acc_t cv[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -360,8 +504,8 @@ __global__ __launch_bounds__(NT, 1) void update_kernel(GemmArgs<T> g) {
     lb.store(Bs, tid);
     __syncthreads();
     if (k0 + KB < g.K) {
-      la.load(g.A, g.lda, m0, k0 + KB, g.M, g.K, g.vec_a, tid);
-      lb.load(g.B, g.ldb, n0, k0 + KB, g.N, g.K, g.vec_b, tid);
+      la.load(g.A, g.lda, m0, k0 + KB, g.M, g.K, tid);
+      lb.load(g.B, g.ldb, n0, k0 + KB, g.N, g.K, tid);
     }
 #pragma unroll
     for (int kg = 0; kg < KB / 16; ++kg)
@@ -440,8 +584,8 @@ __global__ __launch_bounds__(NT, 1) void update_d_kernel(GemmArgs<double> g) {
 
   LA la;
   LB lb;
-  la.load(g.A, g.lda, m0, 0, g.M, g.K, g.vec_a, tid);
-  lb.load(g.B, g.ldb, n0, 0, g.N, g.K, g.vec_b, tid);
+  la.load(g.A, g.lda, m0, 0, g.M, g.K, tid);
+  lb.load(g.B, g.ldb, n0, 0, g.N, g.K, tid);
   /* the C tile, element r of block (i, j) = C(row, col) as the accumulator
    * holds it: row m0 + wm + 16 i + lr, column n0 + wn + 16 j + drow(r) */
   acc_t cv[4][4];
@@ -467,8 +611,8 @@ __global__ __launch_bounds__(NT, 1) void update_d_kernel(GemmArgs<double> g) {
   for (int kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
     if (kt + 1 < nk) {
-      la.load(g.A, g.lda, m0, (kt + 1) * BK, g.M, g.K, g.vec_a, tid);
-      lb.load(g.B, g.ldb, n0, (kt + 1) * BK, g.N, g.K, g.vec_b, tid);
+      la.load(g.A, g.lda, m0, (kt + 1) * BK, g.M, g.K, tid);
+      lb.load(g.B, g.ldb, n0, (kt + 1) * BK, g.N, g.K, tid);
     }
 #pragma unroll
     for (int s4 = 0; s4 < 4; ++s4) {
@@ -570,8 +714,8 @@ __global__ __launch_bounds__(NT, 1) void update_lp_kernel(GemmArgs<float> g) {
 
   LA la;
   LB lb;
-  la.load(g.A, g.lda, m0, 0, g.M, g.K, g.vec_a, tid);
-  lb.load(g.B, g.ldb, n0, 0, g.N, g.K, g.vec_b, tid);
+  la.load(g.A, g.lda, m0, 0, g.M, g.K, tid);
+  lb.load(g.B, g.ldb, n0, 0, g.N, g.K, tid);
   f4 cv[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -612,8 +756,8 @@ __global__ __launch_bounds__(NT, 1) void update_lp_kernel(GemmArgs<float> g) {
     }
     __syncthreads();
     if (k0 + KB < g.K) {
-      la.load(g.A, g.lda, m0, k0 + KB, g.M, g.K, g.vec_a, tid);
-      lb.load(g.B, g.ldb, n0, k0 + KB, g.N, g.K, g.vec_b, tid);
+      la.load(g.A, g.lda, m0, k0 + KB, g.M, g.K, tid);
+      lb.load(g.B, g.ldb, n0, k0 + KB, g.N, g.K, tid);
     }
 #pragma unroll
     for (int ks = 0; ks < KB / 16; ++ks) {
@@ -646,6 +790,60 @@ __global__ __launch_bounds__(NT, 1) void update_lp_kernel(GemmArgs<float> g) {
     }
 }
 
+template <typename T, int TA, int TB, int TS, int KG>
+hipError_t launch_small(const GemmArgs<T> &g, hipStream_t s) {
+  typedef SliceLoader<T, TA != KX_NOTRANS, TS, Mfma<T>::BKS> LA;
+  typedef SliceLoader<T, TB == KX_NOTRANS, TS, Mfma<T>::BKS> LB;
+  constexpr int stage = KG * 2 * (LA::SIZE + LB::SIZE) * (int)sizeof(T);
+  constexpr int red = (KG - 1) * TS * TS * (int)sizeof(T);
+  constexpr int lds = stage > red ? stage : red;
+  if (lds > 64 * 1024) {
+    hipError_t e = hipFuncSetAttribute((const void *)gemm_small_kernel<T, TA, TB, TS, KG>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((gemm_small_kernel<T, TA, TB, TS, KG>), dim3(8 * g.per_xcd), dim3(NT * KG),
+                     lds, s, g);
+  return hipGetLastError();
+}
+
+template <typename T, int TS, int KG>
+hipError_t launch_small_t(int ta, int tb, GemmArgs<T> &g, hipStream_t s) {
+  g.tiles_m = (g.M + TS - 1) / TS;
+  g.tiles_n = (g.N + TS - 1) / TS;
+  g.per_xcd = (int)(((long)g.tiles_m * g.tiles_n + 7) / 8);
+  if (ta == KX_NOTRANS)
+    return tb == KX_NOTRANS ? launch_small<T, KX_NOTRANS, KX_NOTRANS, TS, KG>(g, s)
+                            : launch_small<T, KX_NOTRANS, KX_TRANS, TS, KG>(g, s);
+  return tb == KX_NOTRANS ? launch_small<T, KX_TRANS, KX_NOTRANS, TS, KG>(g, s)
+                          : launch_small<T, KX_TRANS, KX_TRANS, TS, KG>(g, s);
+}
+
+/* The tile edge for an M x N x K product: 128, 64 or 32.  u(t) is the share
+ * of the last round of 256 compute units that t equal tiles keep busy.  The
+ * 128-tile moves the least data per FMA and wins while its rounds are full
+ * (FP64 4096 x 4096 x 512, u = 1: 285 us, 64-tile 313); where the last
+ * round is nearly empty the 64-tile wins (3000^3, 576 tiles, u = 0.75:
+ * 1256 -> 1015 us), the two being equal near u = 0.85.  Between 64 and 32
+ * the factor 0.8 is what the 32-tile's extra operand traffic costs (FP64
+ * 1000^3: 50 us with 256 64-tiles, 57 with 32-tiles; 1511 x 777 x 4001,
+ * u64 = 0.61: 318 against 235 us; 768^3: 35 against 32).  A short K leaves
+ * little to amortise a larger tile's start (1000 x 1000 x 64: 10 against
+ * 8.6 us).  The K groups: one wavefront group per compute unit cannot hide
+ * its own load latency, so few tiles or a long K take four (FP64 200^3,
+ * 32-tile: 9.5 / 7.5 / 7.2 us with 1 / 2 / 4; 300 x 300 x 4000: 188 / 84 /
+ * 63; was 645 in 128-tiles), and a full chip with a short K one (64-tile,
+ * 8192 x 2048 x 64: 56 / 68 / 111). */
+inline double tile_use(long t) { return (double)t / (256.0 * ((t + 255) / 256)); }
+inline int gemm_tile(int M, int N, int K) {
+  const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+  const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+  const long t32 = (long)((M + 31) / 32) * ((N + 31) / 32);
+  if (t128 >= 256 && tile_use(t128) >= 0.85) return 128;
+  if (K <= 64 && t64 <= 256) return 32;
+  return tile_use(t64) >= 0.8 * tile_use(t32) ? 64 : 32;
+}
+
 template <typename T>
 hipError_t launch_gemm(int ta, int tb, int M, int N, int K, T alpha, const T *A,
                        long lda, const T *B, long ldb, T beta, T *C, long ldc,
@@ -666,9 +864,23 @@ hipError_t launch_gemm(int ta, int tb, int M, int N, int K, T alpha, const T *A,
   const long ntiles = (long)g.tiles_m * g.tiles_n;
   if (ntiles > (1L << 30)) return hipErrorInvalidValue;
   g.per_xcd = (int)((ntiles + 7) / 8);
-  constexpr int VEC = Mfma<T>::VEC;
-  g.vec_a = (((uintptr_t)A % 16) == 0) && (lda % VEC == 0);
-  g.vec_b = (((uintptr_t)B % 16) == 0) && (ldb % VEC == 0);
+  /* an in-place product (C is an operand, within one tile row or column of
+   * 128) and the K bands keep the 128-tile */
+  if (C != A && C != B && !(tri >= KX_KBAND_AL && tri <= KX_KBAND_RBU)) {
+    const int ts = gemm_tile(M, N, K);
+    if (ts == 64) {
+      const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+      if (K <= 128) return launch_small_t<T, 64, 1>(ta, tb, g, s);
+      if (t64 >= 512) return launch_small_t<T, 64, 2>(ta, tb, g, s);
+      return launch_small_t<T, 64, 4>(ta, tb, g, s);
+    }
+    if (ts == 32) {
+      const long t32 = (long)((M + 31) / 32) * ((N + 31) / 32);
+      if (K <= 64) return launch_small_t<T, 32, 1>(ta, tb, g, s);
+      if (K >= 1024 || (t32 <= 256 && K > 128)) return launch_small_t<T, 32, 4>(ta, tb, g, s);
+      return launch_small_t<T, 32, 2>(ta, tb, g, s);
+    }
+  }
   const dim3 grid((unsigned)(8 * g.per_xcd)), block(NT);
   if (tri >= KX_KBAND_AL && tri <= KX_KBAND_RBU) {
     if (ta == KX_NOTRANS && tb == KX_NOTRANS)
@@ -707,8 +919,6 @@ extern "C" hipError_t atlmx_k_supdate(int M, int N, int K, float alpha, const fl
   const long ntiles = (long)g.tiles_m * g.tiles_n;
   if (ntiles > (1L << 30)) return hipErrorInvalidValue;
   g.per_xcd = (int)((ntiles + 7) / 8);
-  g.vec_a = (((uintptr_t)A % 16) == 0) && (lda % 4 == 0);
-  g.vec_b = (((uintptr_t)B % 16) == 0) && (ldb % 4 == 0);
   hipLaunchKernelGGL((update_kernel<float, 32>), dim3((unsigned)(8 * g.per_xcd)), dim3(NT), 0, s,
                      g);
   return hipGetLastError();
@@ -733,8 +943,6 @@ extern "C" hipError_t atlmx_k_dupdate(int tb, int M, int N, int K, double alpha,
   const long ntiles = (long)g.tiles_m * g.tiles_n;
   if (ntiles > (1L << 30)) return hipErrorInvalidValue;
   g.per_xcd = (int)((ntiles + 7) / 8);
-  g.vec_a = (((uintptr_t)A % 16) == 0) && (lda % 2 == 0);
-  g.vec_b = (((uintptr_t)B % 16) == 0) && (ldb % 2 == 0);
   const dim3 grid((unsigned)(8 * g.per_xcd)), block(NT);
   if (tb == KX_NOTRANS)
     hipLaunchKernelGGL(update_d_kernel<KX_NOTRANS>, grid, block, 0, s, g);
@@ -760,8 +968,6 @@ extern "C" hipError_t atlmx_k_supdate_lp(int lp, int M, int N, int K, float alph
   const long ntiles = (long)g.tiles_m * g.tiles_n;
   if (ntiles > (1L << 30)) return hipErrorInvalidValue;
   g.per_xcd = (int)((ntiles + 7) / 8);
-  g.vec_a = (((uintptr_t)A % 16) == 0) && (lda % 4 == 0);
-  g.vec_b = (((uintptr_t)B % 16) == 0) && (ldb % 4 == 0);
   const dim3 grid((unsigned)(8 * g.per_xcd)), block(NT);
   if (lp == 1)
     hipLaunchKernelGGL(update_lp_kernel<1>, grid, block, 0, s, g);
