@@ -12,8 +12,8 @@
  * kernel into a hipGraph.  Running the plan replays that graph on the
  * calling thread's stream.
  *
- * The autotuner times every candidate configuration -- panel width 16 or
- * 32, one to three persistent workgroups per CU; for GEMM the kernel
+ * The autotuner times every candidate configuration of the LU and the GEMM
+ * -- panel width 16 or 32, one to three persistent workgroups per CU; for GEMM the kernel
  * (vector FMAs, or MFMA with one or four wavefronts per 64 x 64 tile) and
  * the workgroups per CU -- on a replica of up to AT_SAMPLE instances drawn evenly from the
  * ordered batch (well-conditioned synthetic data of the same sizes, so
@@ -266,6 +266,20 @@ static void autotune(atlmx_batch *p, const int *h_order, const int *h_n, const i
     free(sn); free(offA); free(hA);
     return;
   }
+  if (p->kind == BK_POSV) {
+    /* one kernel, and as many workgroups as its registers let share a
+     * compute unit (212 in FP64, 157 in FP32): the timing below, on a sample
+     * of 512, had preferred one for orders up to 512 because its largest
+     * instances alone run faster unshared (4000 of order 8..512: FP64 4.2 ms
+     * with one, 2.9 with two; FP32 3.2 / 2.0 / 1.7 with one / two / three).
+     * No more than instances, so that a few spread over all units (256 of
+     * order 512: 0.74 ms with 256 workgroups, 0.99 with 512). */
+    const int grid = (p->dbl ? 2 : 3) * cus;
+    p->nb = 32;
+    p->grid = p->count < grid ? (p->count > 0 ? p->count : 1) : grid;
+    free(sn); free(offA); free(hA);
+    return;
+  }
 
   for (i = 0; i < p->count; ++i)
     mean += (p->kind == BK_GEMM) ? cbrt((double)h_m[i] * h_n[i] * h_k[i]) : h_n[i];
@@ -372,7 +386,7 @@ static void autotune(atlmx_batch *p, const int *h_order, const int *h_n, const i
 
   p->nb = p->kind == BK_GEMM ? 2 : 32;
   p->grid = cus;
-  /* factorizations: panel width 16 or 32 x one to three workgroups per CU;
+  /* LU: panel width 16 or 32 x one to three workgroups per CU;
    * GEMM: the kernel variant (vector FMAs, MFMA with one or four
    * wavefronts per 64 x 64 tile) x workgroups per CU */
   for (c = 0; c < (p->kind == BK_GEMM ? 3 : 2); ++c)

@@ -10,11 +10,10 @@
  * in the order the host planned (largest first), so uneven sizes balance
  * themselves.  A factor+solve instance is one workgroup's work:
  *
- *   posv (lower Cholesky): right-looking, NB-column panels: the diagonal
- *     block is factored in LDS, the panel below is solved row by row
- *     against it, and the lower triangle of the trailing matrix is updated
- *     in 64 x 64 tiles (each thread a 4 x 4 piece, the panel's rows staged
- *     in LDS).  The right-hand sides are solved in LDS.
+ *   posv (lower Cholesky): left-looking, 32-column panels; the panel's
+ *     32-row tiles, the right-hand sides among them, are accumulated from
+ *     the finished columns on the matrix cores and multiplied by the diagonal
+ *     block's inverse.
  *   gesv (LU, partial pivoting): the (n-k) x NB panel lives in LDS while it
  *     is factored with partial pivoting (workgroup arg-max per column, ties
  *     to the lower row, NaN never wins, like cblas_idamax), its interchanges
@@ -47,94 +46,6 @@ __device__ inline float bcast(float v, int src) {
 template <typename T> __device__ inline T dsqrt(T x);
 template <> __device__ inline double dsqrt<double>(double x) { return sqrt(x); }
 template <> __device__ inline float dsqrt<float>(float x) { return sqrtf(x); }
-
-/* C(r0.., c0..) -= P_r(rows r0.., K) * P_c(rows c0.., K)^T for one 64 x 64 tile,
- * restricted to r >= c when lower_only.  P_r, P_c: column-major with ld.
- * mr, mc: rows/cols of the tile inside the matrix. */
-template <typename T>
-__device__ void tile_update_nt(T *C, long ldc, const T *Pr, const T *Pc, long ldp, int K, int mr,
-                               int mc, bool lower_only, int r0, int c0, T *s_a, T *s_b) {
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  T acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = T(0);
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    const int kc = min(16, K - k0);
-    __syncthreads();
-    /* s_a[kk][r] = Pr[r + (k0+kk)*ldp]; s_b[kk][c] likewise */
-    for (int e = tid; e < 16 * TS; e += NT) {
-      const int kk = e / TS, rr = e % TS;
-      s_a[kk * TS + rr] = (kk < kc && rr < mr) ? Pr[(size_t)(k0 + kk) * ldp + rr] : T(0);
-      s_b[kk * TS + rr] = (kk < kc && rr < mc) ? Pc[(size_t)(k0 + kk) * ldp + rr] : T(0);
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int kk = 0; kk < 16; ++kk) {
-      T a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = s_a[kk * TS + ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = s_b[kk * TS + tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = ty * 4 + i, c = tx * 4 + j;
-      if (r < mr && c < mc && (!lower_only || r0 + r >= c0 + c))
-        C[(size_t)c * ldc + r] -= acc[i][j];
-    }
-}
-
-/* C(tile) -= L(rows, K) * U(K, cols): L column-major ld ldl, U column-major ld ldu */
-template <typename T>
-__device__ void tile_update_nn(T *C, long ldc, const T *L, long ldl, const T *U, long ldu, int K,
-                               int mr, int mc, T *s_a, T *s_b) {
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  T acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = T(0);
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    const int kc = min(16, K - k0);
-    __syncthreads();
-    for (int e = tid; e < 16 * TS; e += NT) {
-      const int kk = e / TS, rr = e % TS;
-      s_a[kk * TS + rr] = (kk < kc && rr < mr) ? L[(size_t)(k0 + kk) * ldl + rr] : T(0);
-      /* U(k0+kk, cc): kk fastest for the global read, cc = e / 16 */
-      const int cc = e / 16, k2 = e % 16;
-      s_b[k2 * TS + cc] = (k2 < kc && cc < mc) ? U[(size_t)cc * ldu + k0 + k2] : T(0);
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int kk = 0; kk < 16; ++kk) {
-      T a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = s_a[kk * TS + ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = s_b[kk * TS + tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = ty * 4 + i, c = tx * 4 + j;
-      if (r < mr && c < mc) C[(size_t)c * ldc + r] -= acc[i][j];
-    }
-}
 
 /* ---------------------------------------------------------------------- */
 /* Trailing updates on the matrix cores, one 64 x 64 tile per wavefront    */
@@ -357,105 +268,389 @@ __device__ void wg_trsv(int n, int nrhs, const T *A, long lda, bool lower, bool 
 /* ---------------------------------------------------------------------- */
 /* Cholesky factor + solve of one instance by one workgroup                */
 /* ---------------------------------------------------------------------- */
-template <typename T, int NB>
-__device__ void wg_posv(int n, T *A, long lda, int nrhs, T *B, long ldb, int *info, T *s_d,
-                        T *s_a, T *s_b, T *s_x, int *s_flag) {
-  const int tid = threadIdx.x;
-  for (int k = 0; k < n; k += NB) {
-    const int kb = min(NB, n - k);
-    /* ---- diagonal block: potf2 in LDS (ATL_potrfL.c's leaf, unblocked) ---- */
-    __syncthreads();
-    for (int e = tid; e < NB * NB; e += NT) {
-      const int r = e % NB, c = e / NB;
-      s_d[c * (NB + 1) + r] = (r < kb && c < kb && r >= c) ? A[(size_t)(k + c) * lda + k + r] : T(0);
+/* Left-looking in panels of PB = 32 columns.  Panel k's 32 x 32 row tiles
+ * are each one wavefront's: A's tile less L(rows, 0:k) L(k.., 0:k)^T,
+ * accumulated on the matrix cores from the finished columns, then times the
+ * diagonal block's inverse, and written once -- no tile of the trailing
+ * matrix is read and written again for every panel, as the right-looking
+ * form did.  The right-hand sides are one more row tile, [A; B^T], so the
+ * forward substitution costs no pass of its own.  Products are formed
+ * transposed (D[column][row]): a lane's 16 neighbours run down a column of
+ * A, and an accumulator is itself the operand of the product with the
+ * inverse (its element e on lane group g is the k index drow(e) there).
+ *
+ * What bounds an instance is the chain of panels: the diagonal tile (its
+ * sum split over the four wavefronts), its factor and inverse by wavefront 0
+ * alone, then the tiles below; the other wavefronts accumulate their first
+ * tile meanwhile, and two workgroups share a compute unit (three in FP32).
+ * Panels of 64 columns, which read the finished columns half as often, were
+ * no faster (4000 of order 8..512: 3.02 against 2.85 ms).  FP64, 4000
+ * instances of order 8..512, one right-hand side: 14.4 -> 2.9 ms; 512 of
+ * order 256 with 8: 2.17 -> 0.31 ms.  (Starting the accumulators from A's
+ * tile saves 32 registers but doubles the rounding error: FP32 factors of
+ * order 512 1.1e-7 off against 5.5e-8 with the sum apart, 6.3e-8 before.) */
+constexpr int PB = 32;
+constexpr int PLD = PB + 1;
+
+template <typename T> struct Rng;
+template <> struct Rng<double> {
+  __device__ static double rsq(double d) { return __builtin_amdgcn_rsq(d); }
+  __device__ static bool plain(double d) { return d >= 1e-280 && d <= 1e280; }
+};
+template <> struct Rng<float> {
+  __device__ static float rsq(float d) { return __builtin_amdgcn_rsqf(d); }
+  __device__ static bool plain(float d) { return d >= 1e-30f && d <= 1e30f; }
+};
+
+/* sd = sqrt(d) and ri = 1 / sd (d > 0), each within an ulp: the hardware
+ * reciprocal square root and two coupled Newton steps (one in FP32), a
+ * shorter chain than the library's square root and division; outside the
+ * range where no step can over- or underflow, those. */
+template <typename T>
+__device__ inline void sqrt_inv(T d, T &sd, T &ri) {
+  if (Rng<T>::plain(d)) {
+    T y = Rng<T>::rsq(d), g = d * y, h = T(0.5) * y;
+#pragma unroll
+    for (int it = 0; it < (sizeof(T) == 8 ? 2 : 1); ++it) {
+      const T r = fma(-h, g, T(0.5));
+      g = fma(g, r, g);
+      h = fma(h, r, h);
     }
-    if (tid == 0) *s_flag = 0;
-    __syncthreads();
-    /* wavefront 0 alone, one row per lane in registers: column j's values
-     * reach the other lanes by readlane, so no barrier per column */
-    if (threadIdx.x < 64) {
-      const int lane = threadIdx.x;
-      T a[NB];
+    sd = fma(fma(-g, g, d), h, g);
+    ri = T(2) * h;
+    ri = fma(fma(-ri, sd, T(1)), ri, ri);
+  } else {
+    sd = dsqrt(d);
+    ri = T(1) / sd;
+  }
+}
+
+/* acc[ci][rj] += sum over j in [j0, j1) of Y(16 ci + c, j) X(16 rj + r, j):
+ * lane (li, lk) reads Y(16 ci + li, j + lk) at y[ci][(j + lk) ys] and X
+ * likewise.  j1 - j0 is a multiple of 4 U; the next U steps' operands are
+ * loaded before the current steps' MFMAs. */
+template <typename T, int NC, int RJ, int U>
+__device__ __forceinline__ void panel_acc(typename TMfma<T>::acc_t (&acc)[NC][RJ],
+                                          const T *const (&y)[NC], long ys,
+                                          const T *const (&x)[RJ], long xs, int j0, int j1) {
+  const int lk = (threadIdx.x & 63) >> 4;
+  T yc[U][NC], xc[U][RJ];
+  auto load = [&](int j) {
 #pragma unroll
-      for (int c = 0; c < NB; ++c) a[c] = (lane < kb && c <= lane) ? s_d[c * (NB + 1) + lane] : T(0);
-      int fail = 0;
+    for (int u = 0; u < U; ++u) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        if (j < kb && !fail) {
-          const T d = bcast(a[j], j);
-          if (!(d > T(0))) {
-            fail = j + 1;                         /* uniform: every lane saw the same d */
-          } else {
-            const T sd = dsqrt(d);
-            if (lane == j) a[j] = sd;
-            else if (lane > j) a[j] = a[j] / sd;
+      for (int c = 0; c < NC; ++c) yc[u][c] = y[c][(size_t)(j + 4 * u + lk) * ys];
 #pragma unroll
-            for (int c = j + 1; c < NB; ++c) {
-              const T lcj = bcast(a[j], c);
-              if (lane >= c && lane < kb) a[c] -= a[j] * lcj;
-            }
-          }
-        }
+      for (int r = 0; r < RJ; ++r) xc[u][r] = x[r][(size_t)(j + 4 * u + lk) * xs];
+    }
+  };
+  if (j0 >= j1) return;
+  load(j0);
+  for (int j = j0; j < j1; j += 4 * U) {
+    T ya[U][NC], xa[U][RJ];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) ya[u][c] = yc[u][c];
+#pragma unroll
+      for (int r = 0; r < RJ; ++r) xa[u][r] = xc[u][r];
+    }
+    if (j + 4 * U < j1) load(j + 4 * U);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int r = 0; r < RJ; ++r) acc[c][r] = TMfma<T>::mma(ya[u][c], xa[u][r], acc[c][r]);
+  }
+}
+
+template <typename acc_t, int NC, int RJ>
+__device__ __forceinline__ void zero_tile(acc_t (&t)[NC][RJ]) {
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int r = 0; r < RJ; ++r) t[c][r] = acc_t{0, 0, 0, 0};
+}
+
+/* w <- w inv^T for a tile held as accumulators: out[c][r] = the sum over l of
+ * inv(c, l) w(l, r), the inverse (lower) at s_inv[l PLD + c] in LDS */
+template <typename T, int RJ>
+__device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][RJ],
+                                               const T *s_inv) {
+  typename TMfma<T>::acc_t out[2][RJ];
+  const int lane = threadIdx.x & 63, li = lane & 15;
+  zero_tile(out);
+#pragma unroll
+  for (int l = 0; l < 2; ++l)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 16 * l + TMfma<T>::drow(lane, e);
+#pragma unroll
+      for (int c = l; c < 2; ++c) {                /* inv(c, l) = 0 above the diagonal */
+        const T a = s_inv[row * PLD + 16 * c + li];
+#pragma unroll
+        for (int r = 0; r < RJ; ++r) out[c][r] = TMfma<T>::mma(a, w[l][r][e], out[c][r]);
       }
-      if (lane < kb)
-#pragma unroll
-        for (int c = 0; c < NB; ++c)
-          if (c <= lane) s_d[c * (NB + 1) + lane] = a[c];
-      if (lane == 0) *s_flag = fail;
     }
-    __syncthreads();
-    if (*s_flag) {
-      if (tid == 0) *info = k + *s_flag;
-      return;                               /* ATL_potrfL.c:238-240: stop */
-    }
-    for (int e = tid; e < NB * NB; e += NT) {
-      const int r = e % NB, c = e / NB;
-      if (r < kb && c < kb && r >= c) A[(size_t)(k + c) * lda + k + r] = s_d[c * (NB + 1) + r];
-    }
-    /* ---- panel below: row i solves x L_kk^T = a ---- */
-    for (int i = k + kb + tid; i < n; i += NT) {
-      T x[NB];
 #pragma unroll
-      for (int c = 0; c < NB; ++c) x[c] = (c < kb) ? A[(size_t)(k + c) * lda + i] : T(0);
+  for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int c = 0; c < NB; ++c) {
-        if (c < kb) {
-          T v = x[c];
+    for (int r = 0; r < RJ; ++r) w[c][r] = out[c][r];
+}
+
+/* A scalar, or this lane's number, that the compiler takes for a new value
+ * here: without it the products of lda with dozens of column numbers, and
+ * one 64-bit mask for every lane compare, are computed ahead of the panel
+ * loop and spilled across it (the Cholesky: 252 scalar spills). */
+__device__ __forceinline__ long fresh(long v) {
+  int lo = __builtin_amdgcn_readfirstlane((int)v);   /* a leading dimension: 31 bits */
+  asm volatile("" : "+s"(lo));
+  return lo;
+}
+__device__ __forceinline__ int fresh_lane() {
+  int l = threadIdx.x & 63;
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
+/* Wavefront 0: the Cholesky factor of the 32 x 32 block at s_d[c PLD + r]
+ * (identity beyond the matrix), lanes 0..31 one row each, and its inverse,
+ * lanes 32..63 one column each: both are the same elimination step,
+ * v[c] -= v[j] L(c, j), the inverse's columns starting from the identity's.
+ * Column j's entries reach all lanes by readlane.  Returns 0 or 1 + the
+ * failing column; v holds the row of L or the column of the inverse. */
+template <typename T>
+__device__ __forceinline__ int block_factor(T (&v)[PB], const T *s_d) {
+  const int lane = fresh_lane();
+  int fail = 0;
 #pragma unroll
-          for (int l = 0; l < c; ++l) v -= x[l] * s_d[l * (NB + 1) + c];
-          x[c] = v / s_d[c * (NB + 1) + c];
-        }
+  for (int c = 0; c < PB; ++c)
+    v[c] = lane < PB ? s_d[c * PLD + lane] : (c == lane - PB ? T(1) : T(0));
+#pragma unroll
+  for (int j = 0; j < PB; ++j) {
+    if (!fail) {
+      const T d = bcast(v[j], j);
+      if (!(d > T(0))) {
+        fail = j + 1;                              /* uniform: every lane saw the same d */
+      } else {
+        T sd, ri;
+        sqrt_inv(d, sd, ri);
+        v[j] = lane == j ? sd : v[j] * ri;
+#pragma unroll
+        for (int c = j + 1; c < PB; ++c) v[c] = fma(-v[j], bcast(v[j], c), v[c]);
       }
+    }
+  }
+  return fail;
+}
+
+/* s_blk: 4 blocks of PB x PLD elements, or 2 where LDS is short (split =
+ * false: then wavefront 0 sums the diagonal tile alone); s_x: n x nrhs;
+ * s_ctl: 3 */
+template <typename T>
+__device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, int *info,
+                        T *s_blk, bool split, T *s_x, int *s_ctl) {
+  typedef TMfma<T> MF;
+  typedef typename MF::acc_t acc_t;
+  constexpr int BLK = PB * PLD, UT = 4;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15;
+  T *s_d = s_blk, *s_inv = s_blk + BLK;
+  if (tid == 0) s_ctl[0] = s_ctl[2] = 0;
+  for (int e = tid; e < n * nrhs; e += NT) s_x[e] = B[(size_t)(e / n) * ldb + e % n];
+  __syncthreads();
+
+  for (int k = 0; k < n; k += PB) {
+    const int kb = min(PB, n - k), epoch = k / PB + 1;
+    const long lda = fresh(lda0);
+    const T *yp[2] = {A + min(k + li, n - 1), A + min(k + 16 + li, n - 1)};
+    /* ---- the diagonal tile's sum, split over the wavefronts ---- */
+    if (split || wave == 0) {
+      acc_t acc[2][2];
+      zero_tile(acc);
+      const int w = split ? k / 4 : k;             /* a multiple of 8 */
+      panel_acc<T, 2, 2, 2>(acc, yp, lda, yp, lda, wave * w, wave * w + w);
+      T *sp = s_blk + wave * BLK;
 #pragma unroll
-      for (int c = 0; c < NB; ++c)
-        if (c < kb) A[(size_t)(k + c) * lda + i] = x[c];
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sp[(16 * c + MF::drow(lane, e)) * PLD + 16 * r + li] = acc[c][r][e];
     }
     __syncthreads();
-    /* ---- trailing lower triangle: A22 -= P P^T in 64 x 64 tiles ---- */
-    const int m0 = k + kb, m = n - m0;
-    const int nt = (m + TS - 1) / TS;
-    const T *P = A + (size_t)k * lda;
-    {
-      /* the lower triangle's tiles, wavefront w taking every fourth */
-      const int wave = threadIdx.x >> 6;
+    for (int e = tid; e < PB * PB; e += NT) {
+      const int c = e / PB, r = e % PB;
+      T *o = s_blk + c * PLD + r;
+      T v = r == c ? T(1) : T(0);                  /* beyond the matrix: the identity */
+      if (r < kb && c < kb && r >= c) {
+        T sum = *o;
+        if (split) sum = (sum + o[BLK]) + (o[2 * BLK] + o[3 * BLK]);
+        v = A[(size_t)(k + c) * lda + k + r] - sum;
+      }
+      *o = v;
+    }
+    if (tid == 0) s_ctl[1] = 1;                    /* the next row tile to take */
+    __syncthreads();
+
+    if (wave == 0) {
+      T v[PB];
+      const int fail = block_factor(v, s_d);
+      const long lda = fresh(lda0);
+      const int ln = fresh_lane();
+      if (ln < PB) {
+        if (!fail && ln < kb) {
+#pragma unroll
+          for (int c = 0; c < PB; ++c)
+            if (c <= ln) A[(size_t)(k + c) * lda + k + ln] = v[c];
+        }
+      } else {
+#pragma unroll
+        for (int c = 0; c < PB; ++c) s_inv[(ln - PB) * PLD + c] = v[c];
+      }
+      if (ln == 0) {
+        if (fail) s_ctl[2] = k + fail;
+        __hip_atomic_store(&s_ctl[0], epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
+    /* ---- the row tiles below, and last the right-hand sides' tile; a
+     * wavefront waits for the inverse (wavefront 0 always gets there) only
+     * with its sum complete ---- */
+    const int nt = (n - k + PB - 1) / PB, ntile = nt + (nrhs > 0 ? 1 : 0);
+    for (;;) {
       int t = 0;
-      for (int tj = 0; tj < nt; ++tj)
-        for (int ti = tj; ti < nt; ++ti, ++t) {
-          if ((t & 3) != wave) continue;
-          const int r0 = m0 + ti * TS, c0 = m0 + tj * TS;
-          wave_tile_update<T, NB>(A + (size_t)c0 * lda + r0, lda, P + r0, lda, P + c0, 1, lda,
-                                  kb, min(TS, n - r0), min(TS, n - c0), ti == tj, r0, c0);
-        }
+      if (lane == 0) t = atomicAdd(&s_ctl[1], 1);
+      t = __builtin_amdgcn_readfirstlane(t);
+      if (t >= ntile) break;
+      const long lda = fresh(lda0);
+      if (t < nt) {
+        const int r0 = k + t * PB;                 /* then kb == PB */
+        const int ra = r0 + li, rb = ra + 16;
+        const T *xp[2] = {A + min(ra, n - 1), A + min(rb, n - 1)};
+        acc_t acc[2][2], w[2][2];
+        zero_tile(acc);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)            /* A's tile on its way behind the sum */
+              w[c][r][e] = xp[r][(size_t)(k + 16 * c + MF::drow(lane, e)) * lda];
+        panel_acc<T, 2, 2, UT>(acc, yp, lda, xp, lda, 0, k);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int r = 0; r < 2; ++r) w[c][r] -= acc[c][r];
+        while (__hip_atomic_load(&s_ctl[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < epoch)
+          __builtin_amdgcn_s_sleep(1);
+        if (s_ctl[2]) continue;
+        tile_times_inv<T, 2>(w, s_inv);
+        const long ldc = fresh(lda0);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            T *col = A + (size_t)(k + 16 * c + MF::drow(lane, e)) * ldc;
+            if (ra < n) col[ra] = w[c][0][e];
+            if (rb < n) col[rb] = w[c][1][e];
+          }
+      } else {
+        const T *xp[1] = {s_x + (size_t)min(li, nrhs - 1) * n};
+        acc_t acc[2][1], w[2][1];
+        zero_tile(acc);
+        panel_acc<T, 2, 1, UT>(acc, yp, lda, xp, 1, 0, k);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            /* columns beyond the matrix repeat its last row: dropped */
+            const int j = 16 * c + MF::drow(lane, e);
+            w[c][0][e] = j < kb ? xp[0][k + j] - acc[c][0][e] : T(0);
+          }
+        while (__hip_atomic_load(&s_ctl[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < epoch)
+          __builtin_amdgcn_s_sleep(1);
+        if (s_ctl[2]) continue;
+        tile_times_inv<T, 1>(w, s_inv);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int j = 16 * c + MF::drow(lane, e);
+            if (j < kb && li < nrhs) s_x[(size_t)li * n + k + j] = w[c][0][e];
+          }
+      }
+    }
+    __syncthreads();
+    if (s_ctl[2]) {
+      if (tid == 0) *info = s_ctl[2];
+      return;                               /* ATL_potrfL.c:238-240: stop */
     }
   }
   if (tid == 0) *info = 0;
   if (nrhs <= 0) return;
-  /* ---- potrs: L y = b, L^T x = y, right-hand sides in LDS; the factor
-   * phase's LDS (s_d, s_a, s_b, contiguous) is the solve's staging ---- */
-  __syncthreads();
-  for (int e = tid; e < n * nrhs; e += NT) s_x[e] = B[(size_t)(e / n) * ldb + e % n];
-  wg_trsv(n, nrhs, A, lda, true, false, false, s_x, s_d, s_d + SB * (SB + 1));
-  wg_trsv(n, nrhs, A, lda, true, true, false, s_x, s_d, s_d + SB * (SB + 1));
+
+  /* ---- L^T x = y, blocks from the last: the rows below block k
+   * contribute L(r, c) x(r), split over the wavefronts by 16 rows (lane
+   * group lk takes rows 4 lk + s at step s: four neighbours in memory); then
+   * the 32 x 32 triangle, one unknown per lane, wavefront w solving
+   * right-hand side w in lanes 0..31 and w + 4 in lanes 32..63 ---- */
+  for (int k = (n - 1) / PB * PB; k >= 0; k -= PB) {
+    const long lda = fresh(lda0);
+    const int kb = min(PB, n - k), lane = fresh_lane(), li = lane & 15, lk = lane >> 4;
+    const int ln = lane & (PB - 1), rhs = wave + 4 * (lane / PB);
+    T lc[PB], rd = T(0);
+    if (wave < nrhs) {
+#pragma unroll
+      for (int j = 0; j < PB; ++j)
+        lc[j] = (ln < j && j < kb) ? A[(size_t)(k + ln) * lda + k + j] : T(0);
+      if (ln < kb) rd = T(1) / A[(size_t)(k + ln) * lda + k + ln];
+    }
+    acc_t acc[2] = {acc_t{0, 0, 0, 0}, acc_t{0, 0, 0, 0}};
+    const T *xr = s_x + (size_t)min(li, nrhs - 1) * n;
+    for (int r0 = k + PB + 16 * wave; r0 < n; r0 += 16 * (NT / 64)) {
+      T a[2][4], b[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int r = r0 + 4 * lk + s, rr = min(r, n - 1);
+        a[0][s] = A[(size_t)(k + li) * lda + rr];
+        a[1][s] = A[(size_t)(k + 16 + li) * lda + rr];
+        b[s] = r < n ? xr[r] : T(0);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        acc[0] = MF::mma(a[0][s], b[s], acc[0]);
+        acc[1] = MF::mma(a[1][s], b[s], acc[1]);
+      }
+    }
+    if (li < nrhs) {
+      T *sp = s_blk + wave * MAXR * PB;
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sp[li * PB + 16 * c + MF::drow(lane, e)] = acc[c][e];
+    }
+    __syncthreads();
+    if (wave < nrhs) {
+      T g = T(0);
+      if (rhs < nrhs && ln < kb) {
+        const T *sp = s_blk + rhs * PB + ln;
+        g = s_x[(size_t)rhs * n + k + ln] -
+            ((sp[0] + sp[MAXR * PB]) + (sp[2 * MAXR * PB] + sp[3 * MAXR * PB]));
+      }
+#pragma unroll
+      for (int j = PB - 1; j >= 0; --j) {          /* steps past kb change nothing */
+        const T x = g * rd;                        /* lane j's is x_j */
+        T xj = bcast(x, j);
+        if (nrhs > 4) xj = lane < PB ? xj : bcast(x, PB + j);
+        g = ln == j ? x : fma(-lc[j], xj, g);
+      }
+      if (rhs < nrhs && ln < kb) s_x[(size_t)rhs * n + k + ln] = g;
+    }
+    __syncthreads();
+  }
   for (int e = tid; e < n * nrhs; e += NT) B[(size_t)(e / n) * ldb + e % n] = s_x[e];
 }
 
@@ -815,23 +1010,22 @@ struct BatchArgs {
   int *counter;                  /* zero on entry; left at count + grid */
 };
 
-template <typename T, int NB>
-__global__ __launch_bounds__(NT) void posv_batched_kernel(BatchArgs<T> g) {
+template <typename T>
+__global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 3) void posv_batched_kernel(
+    BatchArgs<T> g, int blocks) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  T *s_d = (T *)smem;                                  /* NB x (NB+1) */
-  T *s_a = s_d + NB * (NB + 1);                        /* 16 x 64 */
-  T *s_b = s_a + 16 * TS;                              /* 16 x 64 */
-  T *s_x = s_b + 16 * TS;                              /* n x nrhs */
-  __shared__ int s_item, s_flag;
+  T *s_blk = (T *)smem;                                /* blocks x PB x PLD */
+  T *s_x = s_blk + blocks * PB * PLD;                  /* n x nrhs */
+  __shared__ int s_item, s_ctl[3];
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) s_item = atomicAdd(g.counter, 1);
     __syncthreads();
-    const int it = s_item;
+    const int it = __builtin_amdgcn_readfirstlane(s_item);   /* scalar: addresses too */
     if (it >= g.count) return;
     const int i = g.order[it];
-    wg_posv<T, NB>(g.n[i], g.A[i], g.lda[i], g.nrhs, g.B ? g.B[i] : nullptr,
-                   g.ldb ? g.ldb[i] : 1, &g.info[i], s_d, s_a, s_b, s_x, &s_flag);
+    wg_posv<T>(g.n[i], g.A[i], g.lda[i], g.nrhs, g.B ? g.B[i] : nullptr, g.ldb ? g.ldb[i] : 1,
+               &g.info[i], s_blk, blocks == 4, s_x, s_ctl);
   }
 }
 
@@ -849,7 +1043,7 @@ __global__ __launch_bounds__(NT) void gesv_batched_kernel(BatchArgs<T> g, int ma
     __syncthreads();
     if (threadIdx.x == 0) s_item = atomicAdd(g.counter, 1);
     __syncthreads();
-    const int it = s_item;
+    const int it = __builtin_amdgcn_readfirstlane(s_item);   /* scalar: addresses too */
     if (it >= g.count) return;
     const int i = g.order[it];
     wg_gesv<T, NB>(g.n[i], g.A[i], g.lda[i], g.ipiv[i], g.nrhs, g.B ? g.B[i] : nullptr,
@@ -883,7 +1077,7 @@ __global__ __launch_bounds__(NT) void gemm_batched_kernel(GemmBatchArgs<T> g) {
     __syncthreads();
     if (tid == 0) s_item = atomicAdd(g.counter, 1);
     __syncthreads();
-    const int it = s_item;
+    const int it = __builtin_amdgcn_readfirstlane(s_item);   /* scalar: addresses too */
     if (it >= total) return;
     /* instance: the last i with tile_start[i] <= it */
     int lo = 0, hi = g.count - 1;
@@ -975,14 +1169,17 @@ __global__ __launch_bounds__(NT) void chol_adjoint_kernel(AdjArgs<T> g) {
   }
 }
 
-template <typename T, int NB>
+template <typename T>
 hipError_t launch_posv(const BatchArgs<T> &g, int maxn, int grid, hipStream_t s) {
-  const size_t lds = sizeof(T) * ((size_t)NB * (NB + 1) + 2 * 16 * TS + (size_t)maxn * MAXR);
-  if (lds > 160 * 1024) return hipErrorInvalidValue;
-  hipError_t e = hipFuncSetAttribute((const void *)posv_batched_kernel<T, NB>,
+  const size_t x = sizeof(T) * (size_t)maxn * g.nrhs, blk = sizeof(T) * PB * PLD;
+  const size_t cap = 160 * 1024 - 64;              /* less the static words */
+  const int blocks = 4 * blk + x <= cap ? 4 : 2;
+  const size_t lds = blocks * blk + x;
+  if (lds > cap) return hipErrorInvalidValue;
+  hipError_t e = hipFuncSetAttribute((const void *)posv_batched_kernel<T>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((posv_batched_kernel<T, NB>), dim3(grid), dim3(NT), lds, s, g);
+  hipLaunchKernelGGL((posv_batched_kernel<T>), dim3(grid), dim3(NT), lds, s, g, blocks);
   return hipGetLastError();
 }
 
@@ -1007,8 +1204,7 @@ hipError_t batch_factor(int kind, int nb, int count, const int *order, const int
   g.count = count; g.order = order; g.n = n; g.A = A; g.lda = lda; g.ipiv = ipiv;
   g.nrhs = nrhs; g.B = B; g.ldb = ldb; g.info = info; g.counter = counter;
   if (kind == 0) {
-    if (nb == 16) return launch_posv<T, 16>(g, maxn, grid, s);
-    if (nb == 32) return launch_posv<T, 32>(g, maxn, grid, s);
+    if (nb == 16 || nb == 32) return launch_posv<T>(g, maxn, grid, s);   /* one panel width */
   } else if (kind == 1 || kind == 2) {      /* 2: solve with A^T */
     if (nb == 16) return launch_gesv<T, 16>(g, maxn, grid, kind == 2, s);
     if (nb == 32) return launch_gesv<T, 32>(g, maxn, grid, kind == 2, s);
@@ -1064,7 +1260,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_batched_mfma_kernel(GemmBatchArg
     __syncthreads();
     if (tid == 0) s_item = atomicAdd(g.counter, 1);
     __syncthreads();
-    const int it = s_item;
+    const int it = __builtin_amdgcn_readfirstlane(s_item);   /* scalar: addresses too */
     if (it >= total) return;
     int lo = 0, hi = g.count - 1;
     while (lo < hi) {

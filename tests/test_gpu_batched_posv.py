@@ -1,0 +1,77 @@
+"""The batched Cholesky factor + solve at the edges of its 32-column panels
+and 32-row tiles, for every right-hand-side count, failing minors in every
+part of a panel, and the largest order (where LDS holds no split diagonal
+sum).  Bounds: |A - L L^T| <= c (n + 1) u |L| |L|^T elementwise (Higham,
+Accuracy and Stability, Theorem 10.3; c = 8 for the products with the
+diagonal blocks' inverses, whose condition is below 8 for these matrices),
+||b - A x|| <= c n u ||A|| ||x|| in the infinity norm."""
+import numpy as np
+import pytest
+
+import atlas_amd as X
+
+pytestmark = pytest.mark.gpu
+
+
+def _spd(rng, n):
+    B = rng.standard_normal((n, n))
+    return B @ B.T / n + np.eye(n)
+
+
+def _check(torch, sizes, dt, nrhs, fails=()):
+    rng = np.random.default_rng(sum(sizes) + nrhs)
+    u = np.finfo(dt).eps / 2
+    A0 = [_spd(rng, n).astype(dt) for n in sizes]
+    for i, col in fails:
+        A0[i][col - 1, col - 1] = -1.0
+    up = [np.triu(rng.standard_normal(a.shape), 1).astype(dt) for a in A0]   # never read
+    B0 = [rng.uniform(-1, 1, (n, nrhs)).astype(dt) for n in sizes]
+    dev = lambda m: torch.tensor(np.ascontiguousarray(m.T), device="cuda")   # noqa: E731
+    As, Bs = [dev(np.tril(a) + w) for a, w in zip(A0, up)], [dev(b) for b in B0]
+    info = torch.full((len(sizes),), -7, dtype=torch.int32, device="cuda")
+    with X.posv_batch(As, Bs if nrhs else [], info) as plan:
+        plan.run()
+        torch.cuda.synchronize()
+    inf = info.cpu().numpy()
+    bad = dict(fails)
+    for i, n in enumerate(sizes):
+        F = As[i].cpu().numpy().T
+        assert np.array_equal(np.triu(F, 1), up[i]), n
+        if i in bad:
+            assert inf[i] == bad[i], (n, inf[i])
+            assert np.array_equal(Bs[i].cpu().numpy().T, B0[i]) if nrhs else True
+            continue
+        assert inf[i] == 0, (n, inf[i])
+        L, A = np.tril(F).astype(np.float64), A0[i].astype(np.float64)
+        A = np.tril(A) + np.tril(A, -1).T
+        assert np.all(np.abs(A - L @ L.T) <= 8 * (n + 1) * u * (np.abs(L) @ np.abs(L).T)), n
+        if nrhs:
+            x, b = Bs[i].cpu().numpy().T.astype(np.float64), B0[i].astype(np.float64)
+            bound = 8 * n * u * np.abs(A).sum(1).max() * np.abs(x).max(0) + 1e-300
+            assert np.all(np.abs(b - A @ x).max(0) <= bound), n
+
+
+EDGES = [1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 95, 96, 97, 127, 129, 191, 193, 257]
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("nrhs", [0, 1, 3, 5, 8])
+def test_posv_panel_and_tile_edges(dt, nrhs):
+    import torch
+    X.use_torch_stream()
+    _check(torch, EDGES, dt, nrhs)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_posv_first_failing_minor(dt):
+    import torch
+    X.use_torch_stream()
+    cols = [1, 16, 17, 32, 33, 48, 64, 65, 100]
+    _check(torch, [100] * len(cols) + [40, 33], dt, 2, list(enumerate(cols)) + [(9, 40), (10, 33)])
+
+
+def test_posv_largest_order():
+    import torch
+    X.use_torch_stream()
+    n = X.lib().atlmx_batch_max_order(0, 1)
+    _check(torch, [n, 70], np.float64, 8)
