@@ -11,7 +11,7 @@ than keeping it, then
   LU:       B-bar = A^{-T} X-bar (getrs with the transpose),
             A-bar = -B-bar X^T   (batched GEMM);
   Cholesky: B-bar = A^{-1} X-bar (potrs), then the Cholesky adjoint kernel:
-            L-bar = -(B-bar X^T + X B-bar^T) L, P = Phi(L^T L-bar),
+            L-bar = -tril((B-bar X^T + X B-bar^T) L), P = Phi(L^T L-bar),
             A-bar = L^{-T} P L^{-1} symmetrised, returned for the lower
             triangle only (the entries potrf reads; each off-diagonal entry
             carries both of its positions, the upper triangle gets zero).
@@ -24,8 +24,15 @@ from . import NoTrans, Trans, use_torch_stream
 
 
 def _cm(t):
-    """column-major copy: storage of t^T, returned as (..., cols, rows)"""
+    """storage of t^T (column-major), returned as (..., cols, rows)"""
     return t.transpose(-1, -2).contiguous()
+
+
+def _cm_copy(t):
+    """the same in memory of its own (contiguous() returns t's when t already
+    is a transpose), for the plans that work in place"""
+    c = _cm(t)
+    return c.clone() if c.data_ptr() == t.data_ptr() else c
 
 
 def _check(A, B):
@@ -59,7 +66,7 @@ class CholeskySolve(torch.autograd.Function):
     def forward(ctx, A, B):
         _check(A, B)
         use_torch_stream()
-        Aw, Xw = _cm(A).clone(), _cm(B).clone()          # (batch, n, n), (batch, nrhs, n)
+        Aw, Xw = _cm_copy(A), _cm_copy(B)          # (batch, n, n), (batch, nrhs, n)
         info = _posv(Aw, Xw)
         if int(info.abs().sum().item()):
             raise RuntimeError("CholeskySolve: a matrix is not positive definite")
@@ -71,7 +78,7 @@ class CholeskySolve(torch.autograd.Function):
     def backward(ctx, Xb):
         A, X = ctx.saved_tensors
         use_torch_stream()
-        Lw, Bb = _cm(A).clone(), _cm(Xb).clone()
+        Lw, Bb = _cm_copy(A), _cm_copy(Xb)
         _posv(Lw, Bb)                                   # L recomputed, Bb = A^{-1} Xb
         Xc = _cm(X)
         G = torch.empty_like(Lw)
@@ -86,7 +93,7 @@ class LUSolve(torch.autograd.Function):
     def forward(ctx, A, B):
         _check(A, B)
         use_torch_stream()
-        Aw, Xw = _cm(A).clone(), _cm(B).clone()
+        Aw, Xw = _cm_copy(A), _cm_copy(B)
         info = _gesv(Aw, Xw)
         if int(info.abs().sum().item()):
             raise RuntimeError("LUSolve: a matrix is singular")
@@ -98,7 +105,7 @@ class LUSolve(torch.autograd.Function):
     def backward(ctx, Xb):
         A, X = ctx.saved_tensors
         use_torch_stream()
-        Lw, Bb = _cm(A).clone(), _cm(Xb).clone()
+        Lw, Bb = _cm_copy(A), _cm_copy(Xb)
         _gesv(Lw, Bb, trans=True)                       # LU recomputed, Bb = A^{-T} Xb
         Ga = torch.empty_like(Lw)                       # column-major n x n per instance
         Xc = _cm(X)

@@ -44,7 +44,7 @@ struct atlmx_batch {
   int *d_meta;                    /* order | n | lda | ldb  (| m | k | ldc | tile_start) */
   int *d_counter;
   void *const *A, *const *B, *const *C;
-  void *const *D, *const *E;      /* Cholesky adjoint: gradient G, scratch W */
+  void *const *D;                 /* Cholesky adjoint: gradient G */
   int *const *ipiv;
   int *info;
   int ta, tb;
@@ -203,12 +203,10 @@ static hipError_t launch(const atlmx_batch *p, int count, const int *meta, void 
     if (p->dbl)
       return atlmx_k_dbatch_chol_adjoint(count, order, n, (double *const *)A, lda, p->nrhs,
                                          (double *const *)B, (double *const *)C, ldb,
-                                         (double *const *)p->D, ldg, (double *const *)p->E,
-                                         p->d_counter, grid, s);
+                                         (double *const *)p->D, ldg, p->d_counter, grid, s);
     return atlmx_k_sbatch_chol_adjoint(count, order, n, (float *const *)A, lda, p->nrhs,
                                        (float *const *)B, (float *const *)C, ldb,
-                                       (float *const *)p->D, ldg, (float *const *)p->E,
-                                       p->d_counter, grid, s);
+                                       (float *const *)p->D, ldg, p->d_counter, grid, s);
   }
   if (p->dbl)
     return atlmx_k_dbatch_factor(p->kind == BK_GESVT ? 2 : p->kind, nb, count, order, n,
@@ -258,11 +256,9 @@ static void autotune(atlmx_batch *p, const int *h_order, const int *h_n, const i
   unsigned long long seed = 0x5DEECE66DULL;
   if (!sn || !offA || !hA) { fprintf(stderr, "%s: out of host memory\n", rout); exit(-1); }
   if (p->kind == BK_CHOLADJ) {
-    /* one configuration: two workgroups per CU (184 registers and 16 KB of
-     * LDS each), so one's barrier-bound triangular solves overlap the
-     * other's */
+    /* one configuration: memory-bound, eight small workgroups per CU */
     p->nb = 0;
-    p->grid = 2 * cus;
+    p->grid = p->count < 8 * cus ? (p->count > 0 ? p->count : 1) : 8 * cus;
     free(sn); free(offA); free(hA);
     return;
   }
@@ -433,7 +429,7 @@ static atlmx_batch *plan_create2(int kind, int dbl, int count, int ta, int tb, c
                                  const int *h_n, const int *h_k, double alpha, void *const *A,
                                  const int *h_lda, void *const *B, const int *h_ldb, double beta,
                                  void *const *C, const int *h_ldc, int *const *ipiv, int nrhs,
-                                 int *info, void *const *D, void *const *E, const char *rout);
+                                 int *info, void *const *D, const char *rout);
 
 static int cmp_cost_desc(const void *a, const void *b)
 {
@@ -448,14 +444,14 @@ static atlmx_batch *plan_create(int kind, int dbl, int count, int ta, int tb, co
                                 int *info, const char *rout)
 {
   return plan_create2(kind, dbl, count, ta, tb, h_m, h_n, h_k, alpha, A, h_lda, B, h_ldb, beta,
-                      C, h_ldc, ipiv, nrhs, info, NULL, NULL, rout);
+                      C, h_ldc, ipiv, nrhs, info, NULL, rout);
 }
 
 static atlmx_batch *plan_create2(int kind, int dbl, int count, int ta, int tb, const int *h_m,
                                  const int *h_n, const int *h_k, double alpha, void *const *A,
                                  const int *h_lda, void *const *B, const int *h_ldb, double beta,
                                  void *const *C, const int *h_ldc, int *const *ipiv, int nrhs,
-                                 int *info, void *const *D, void *const *E, const char *rout)
+                                 int *info, void *const *D, const char *rout)
 {
   atlmx_batch *p;
   double *cost;
@@ -481,7 +477,7 @@ static atlmx_batch *plan_create2(int kind, int dbl, int count, int ta, int tb, c
   p = (atlmx_batch *)calloc(1, sizeof(*p));
   if (!p) { fprintf(stderr, "%s: out of host memory\n", rout); exit(-1); }
   p->kind = kind; p->dbl = dbl; p->count = count; p->nrhs = nrhs;
-  p->A = A; p->B = B; p->C = C; p->ipiv = ipiv; p->info = info; p->D = D; p->E = E;
+  p->A = A; p->B = B; p->C = C; p->ipiv = ipiv; p->info = info; p->D = D;
   p->ta = ta; p->tb = tb; p->alpha = alpha; p->beta = beta;
   cost = (double *)malloc(sizeof(double) * 2 * count);
   h = (int *)malloc(sizeof(int) * nmeta);
@@ -670,9 +666,10 @@ atlmx_batch *atlmx_dposv_adjoint_batch_plan(int count, const int *h_n, double *c
 {
   static const char *rout = "atlmx_dposv_adjoint_batch_plan";
   if (count < 0 || nrhs < 0) cblas_xerbla(5, rout, "");
+  (void)d_W;
   return plan_create2(BK_CHOLADJ, 1, count, 0, 0, NULL, h_n, NULL, 0.0, (void *const *)d_L,
                       h_lda, (void *const *)d_X, h_ldx, 0.0, (void *const *)d_Bb, h_ldg, NULL,
-                      nrhs, NULL, (void *const *)d_G, (void *const *)d_W, rout);
+                      nrhs, NULL, (void *const *)d_G, rout);
 }
 
 atlmx_batch *atlmx_sposv_adjoint_batch_plan(int count, const int *h_n, float *const *d_L,
@@ -683,9 +680,10 @@ atlmx_batch *atlmx_sposv_adjoint_batch_plan(int count, const int *h_n, float *co
 {
   static const char *rout = "atlmx_sposv_adjoint_batch_plan";
   if (count < 0 || nrhs < 0) cblas_xerbla(5, rout, "");
+  (void)d_W;
   return plan_create2(BK_CHOLADJ, 0, count, 0, 0, NULL, h_n, NULL, 0.0, (void *const *)d_L,
                       h_lda, (void *const *)d_X, h_ldx, 0.0, (void *const *)d_Bb, h_ldg, NULL,
-                      nrhs, NULL, (void *const *)d_G, (void *const *)d_W, rout);
+                      nrhs, NULL, (void *const *)d_G, rout);
 }
 
 int atlmx_batch_max_order(int kind, int dbl)

@@ -793,208 +793,57 @@ __device__ void wg_gesv(int n, T *A, long lda, int *ipiv, int nrhs, T *B, long l
 /* ---------------------------------------------------------------------- */
 /* Cholesky adjoint of one instance by one workgroup                       */
 /* ---------------------------------------------------------------------- */
-/* C(tile r0.., c0..) = sum_k Aop(r, k) Bop(k, c) over k in [k0, k1), where
- * Aop(r, k) = A[r*ar + k*ak] and Bop(k, c) = B[k*bk + c*bc] (strides give
- * the transposes); only r >= c is written when lower_only. */
-template <typename T>
-__device__ void tile_gemm(T *C, long ldc, const T *A, long ar, long ak, const T *B, long bk,
-                          long bc, int k0, int k1, int mr, int mc, bool lower_only, int r0,
-                          int c0, T *s_a, T *s_b) {
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  T acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = T(0);
-  for (int kb = k0; kb < k1; kb += 16) {
-    const int kc = min(16, k1 - kb);
-    __syncthreads();
-    for (int e = tid; e < 16 * TS; e += NT) {
-      const int kk = e / TS, rr = e % TS;
-      s_a[kk * TS + rr] = (kk < kc && rr < mr) ? A[(size_t)rr * ar + (size_t)(kb + kk) * ak] : T(0);
-      s_b[kk * TS + rr] = (kk < kc && rr < mc) ? B[(size_t)(kb + kk) * bk + (size_t)rr * bc] : T(0);
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int kk = 0; kk < 16; ++kk) {
-      T a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = s_a[kk * TS + ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = s_b[kk * TS + tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = ty * 4 + i, c = tx * 4 + j;
-      if (r < mr && c < mc && (!lower_only || r0 + r >= c0 + c)) C[(size_t)c * ldc + r] = acc[i][j];
-    }
-}
-
-/* The adjoint's two triangular solves for n <= NT, in registers: the
- * right-hand sides are independent, so a block of ADJ_CB of them is solved
- * at a time with one unknown per thread.  Step i (from the last) has the
- * owner of unknown i divide by L(i,i) and publish its ADJ_CB values through
- * LDS (two buffers by the parity of i), then every thread t < i subtracts
- * L(i, t) times them: one barrier per step.  L(i, t) is loaded ADJ_PF
- * steps ahead into a ring of registers (the steps run in unrolled groups of
- * ADJ_PF, so every ring index is fixed).
- *   lt = 1: Y = L^{-T} W (W's columns are the right-hand sides; thread t
- *           holds row t of a block of columns);
- *   lt = 0: S = W L^{-1} (W's rows are; thread t holds column t of a block
- *           of rows).
- * Both read L(i, t) = L[t*lda + i] at step i. */
-constexpr int ADJ_CB = 16;
-constexpr int ADJ_PF = 8;
-
-template <typename T>
-__device__ void wg_adj_solve(int n, const T *L, long lda, T *W, int lt,
-                             T (*s_y)[ADJ_CB]) {
-  const int t = threadIdx.x;
-  for (int b0 = 0; b0 < n; b0 += ADJ_CB) {
-    const int bb = min(ADJ_CB, n - b0);
-    T y[ADJ_CB];
-#pragma unroll
-    for (int q = 0; q < ADJ_CB; ++q)
-      y[q] = (t < n && q < bb) ? (lt ? W[(size_t)(b0 + q) * n + t] : W[(size_t)t * n + b0 + q])
-                               : T(0);
-    T ring[ADJ_PF];
-#pragma unroll
-    for (int q = 0; q < ADJ_PF; ++q) {
-      const int i = n - 1 - q;
-      ring[q] = (i >= 0 && t < i) ? L[(size_t)t * lda + i] : T(0);
-    }
-    for (int i0 = n - 1; i0 >= 0; i0 -= ADJ_PF) {
-#pragma unroll
-      for (int q = 0; q < ADJ_PF; ++q) {
-        const int i = i0 - q;
-        if (i >= 0) {
-          const T li = ring[q];
-          const int ip = i - ADJ_PF;               /* the step this slot serves next */
-          ring[q] = (ip >= 0 && t < ip) ? L[(size_t)t * lda + ip] : T(0);
-          T *buf = s_y[i & 1];
-          if (t == i) {
-            const T rd = T(1) / L[(size_t)i * lda + i];
-#pragma unroll
-            for (int r = 0; r < ADJ_CB; ++r) {
-              y[r] *= rd;
-              buf[r] = y[r];
-            }
-          }
-          __syncthreads();
-          if (t < i) {
-#pragma unroll
-            for (int r = 0; r < ADJ_CB; ++r) y[r] -= li * buf[r];
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < ADJ_CB; ++q)
-      if (t < n && q < bb) {
-        if (lt) W[(size_t)(b0 + q) * n + t] = y[q];
-        else W[(size_t)t * n + b0 + q] = y[q];
-      }
-    __syncthreads();
-  }
-}
-
 /* Given L (lower triangle of A after potrf; its strict upper triangle is
  * overwritten with zeros here), X = A^{-1} B and Bb = A^{-1} Xb (the solve's
  * adjoint), write to G the gradient of <Xb, X> with respect to the lower
- * triangle of A (the entries potrf reads; strict upper part zero):
- *   Lb = tril(-(Bb X^T + X Bb^T) L)            (potrs adjoint: L's gradient)
- *   P  = Phi(L^T Lb)   (lower triangle, diagonal halved)
- *   S  = L^{-T} P L^{-1}                        (two triangular solves)
- *   G  = tril(S + S^T) - diag(S)  (the symmetric gradient (S + S^T)/2, each
- *        off-diagonal entry counted for both of its positions)
- * (Murray, "Differentiation of the Cholesky decomposition", 2016).  W: an
- * n x n scratch (leading dimension n). */
+ * triangle of A (the entries potrf reads; strict upper part zero).  The
+ * Cholesky adjoint (Murray, "Differentiation of the Cholesky decomposition",
+ * 2016) of the solve's L-bar is
+ *   Lb = -tril(M L),  M = Bb X^T + X Bb^T
+ *   P  = Phi(L^T Lb)             (lower triangle, diagonal halved)
+ *   S  = L^{-T} P L^{-1}         (two triangular solves)
+ *   G  = tril(S + S^T) - diag(S) (off-diagonal entries count twice).
+ * With U = L^T X and V = L^T Bb, M L = Bb U^T + X V^T.  An entry i >= j of
+ * L^T Lb sums over k >= i >= j, where the tril of Lb masks nothing, so it is
+ * -(V U^T + U V^T)(i, j): symmetric of rank 2 nrhs, and P + P^T is all of it.
+ * The two solves applied to those factors give back L^{-T} V = Bb and
+ * L^{-T} U = X, so
+ *   S + S^T = -(Bb X^T + X Bb^T)
+ * without forming the n x n intermediates: n^2 nrhs products and one write
+ * of G instead of ~2 n^3 flops (FP64, 512 of order 256, 8 right-hand sides:
+ * 6.7 -> 0.30 ms, bound by writing G and zeroing L's triangle), and
+ * without the solves' rounding. */
+constexpr int ADJ_CB = 4;                        /* columns of G at a time */
 template <typename T>
 __device__ void wg_chol_adjoint(int n, T *L, long lda, int nrhs, const T *Xs, const T *Bb,
-                                long ldx, T *G, long ldg, T *W, T *s_a, T *s_b,
-                                T (*s_y)[ADJ_CB]) {
-  const int tid = threadIdx.x;
-  const int nt = (n + TS - 1) / TS;
-  /* W = -(Bb X^T + X Bb^T); G = 0; strict upper of L = 0 */
-  for (int e = tid; e < n * n; e += NT) {
-    const int i = e % n, j = e / n;
-    T v = T(0);
-    for (int r = 0; r < nrhs; ++r)
-      v += Bb[(size_t)r * ldx + i] * Xs[(size_t)r * ldx + j] +
-           Xs[(size_t)r * ldx + i] * Bb[(size_t)r * ldx + j];
-    W[(size_t)j * n + i] = -v;
-    G[(size_t)j * ldg + i] = T(0);
-    if (i < j) L[(size_t)j * lda + i] = T(0);
-  }
-  __syncthreads();
-  /* G = tril(W L): G(i, j) = sum_{k >= j} W(i, k) L(k, j) */
-  for (int tj = 0; tj < nt; ++tj)
-    for (int ti = tj; ti < nt; ++ti) {
-      const int r0 = ti * TS, c0 = tj * TS;
-      tile_gemm(G + (size_t)c0 * ldg + r0, ldg, W + r0, 1, n, L + (size_t)c0 * lda, 1, lda, c0,
-                n, min(TS, n - r0), min(TS, n - c0), ti == tj, r0, c0, s_a, s_b);
+                                long ldx, T *G, long ldg) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int j0 = ADJ_CB * wave; j0 < n; j0 += ADJ_CB * (NT / 64)) {
+    for (int i = lane; i < n; i += 64) {
+      T acc[ADJ_CB];
+#pragma unroll
+      for (int c = 0; c < ADJ_CB; ++c) acc[c] = T(0);
+      if (i >= j0)
+        for (int r = 0; r < nrhs; ++r) {
+          const T bi = Bb[(size_t)r * ldx + i], xi = Xs[(size_t)r * ldx + i];
+#pragma unroll
+          for (int c = 0; c < ADJ_CB; ++c) {
+            const int j = min(j0 + c, n - 1);
+            const T bj = Bb[(size_t)r * ldx + j], xj = Xs[(size_t)r * ldx + j];
+            acc[c] += i == j ? bi * xj : bi * xj + xi * bj;
+          }
+        }
+#pragma unroll
+      for (int c = 0; c < ADJ_CB; ++c) {
+        const int j = j0 + c;
+        if (j < n) {
+          G[(size_t)j * ldg + i] = i >= j ? -acc[c] : T(0);
+          if (i < j) L[(size_t)j * lda + i] = T(0);
+        }
+      }
     }
-  __syncthreads();
-  /* W = L^T G on the lower triangle: P(i, j) = sum_{k >= i} L(k, i) G(k, j) */
-  for (int tj = 0; tj < nt; ++tj)
-    for (int ti = tj; ti < nt; ++ti) {
-      const int r0 = ti * TS, c0 = tj * TS;
-      tile_gemm(W + (size_t)c0 * n + r0, n, L + (size_t)r0 * lda, lda, 1, G + (size_t)c0 * ldg,
-                1, ldg, r0, n, min(TS, n - r0), min(TS, n - c0), ti == tj, r0, c0, s_a, s_b);
-    }
-  __syncthreads();
-  /* Phi: halve the diagonal, zero the strict upper triangle */
-  for (int e = tid; e < n * n; e += NT) {
-    const int i = e % n, j = e / n;
-    if (i < j) W[(size_t)j * n + i] = T(0);
-    else if (i == j) W[(size_t)j * n + i] *= T(0.5);
   }
-  __syncthreads();
-  if (n <= NT) {
-    wg_adj_solve<T>(n, L, lda, W, 1, s_y);   /* Y = L^{-T} P */
-    wg_adj_solve<T>(n, L, lda, W, 0, s_y);   /* S = Y L^{-1} */
-  } else {
-  /* Y = L^{-T} P in place: rows from the last; Y(i,:) /= L(i,i), then rows
-   * k < i lose L(i, k) Y(i,:) */
-  for (int i = n - 1; i >= 0; --i) {
-    const T d = L[(size_t)i * lda + i];
-    for (int c = tid; c < n; c += NT) W[(size_t)c * n + i] /= d;
-    __syncthreads();
-    for (int e = tid; e < i * n; e += NT) {
-      const int k = e % i, c = e / i;
-      W[(size_t)c * n + k] -= L[(size_t)k * lda + i] * W[(size_t)c * n + i];
-    }
-    __syncthreads();
-  }
-  /* S = Y L^{-1} in place: columns from the last; S(:,j) /= L(j,j), then
-   * columns j' < j lose S(:, j) L(j, j') */
-  for (int j = n - 1; j >= 0; --j) {
-    const T d = L[(size_t)j * lda + j];
-    for (int r = tid; r < n; r += NT) W[(size_t)j * n + r] /= d;
-    __syncthreads();
-    for (int e = tid; e < n * j; e += NT) {
-      const int r = e % n, jp = e / n;
-      W[(size_t)jp * n + r] -= W[(size_t)j * n + r] * L[(size_t)jp * lda + j];
-    }
-    __syncthreads();
-  }
-  }
-  /* G = tril(S + S^T) - diag(S) */
-  for (int e = tid; e < n * n; e += NT) {
-    const int i = e % n, j = e / n;
-    T v = T(0);
-    if (i > j) v = W[(size_t)j * n + i] + W[(size_t)i * n + j];
-    else if (i == j) v = W[(size_t)j * n + i];
-    G[(size_t)j * ldg + i] = v;
-  }
-  __syncthreads();
 }
 
 template <typename T>
@@ -1147,25 +996,23 @@ template <typename T>
 struct AdjArgs {
   int count, nrhs;
   const int *order, *n, *lda, *ldx, *ldg;
-  T *const *L; T *const *X; T *const *Bb; T *const *G; T *const *W;
+  T *const *L; T *const *X; T *const *Bb; T *const *G;
   /* L's strict upper triangle is zeroed */
   int *counter;
 };
 
 template <typename T>
 __global__ __launch_bounds__(NT) void chol_adjoint_kernel(AdjArgs<T> g) {
-  __shared__ T s_a[16 * TS], s_b[16 * TS];
-  __shared__ T s_y[2][ADJ_CB];
   __shared__ int s_item;
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) s_item = atomicAdd(g.counter, 1);
     __syncthreads();
-    const int it = s_item;
+    const int it = __builtin_amdgcn_readfirstlane(s_item);
     if (it >= g.count) return;
     const int i = g.order[it];
     wg_chol_adjoint<T>(g.n[i], g.L[i], g.lda[i], g.nrhs, g.X[i], g.Bb[i], g.ldx[i], g.G[i],
-                       g.ldg[i], g.W[i], s_a, s_b, s_y);
+                       g.ldg[i]);
   }
 }
 
@@ -1384,12 +1231,12 @@ hipError_t batch_gemm(int count, int ta, int tb, const int *order, const int *m,
 template <typename T>
 hipError_t chol_adjoint(int count, const int *order, const int *n, T *const *L, const int *lda,
                         int nrhs, T *const *Xs, T *const *Bb, const int *ldx, T *const *G,
-                        const int *ldg, T *const *W, int *counter, int grid, hipStream_t s) {
+                        const int *ldg, int *counter, int grid, hipStream_t s) {
   if (count <= 0) return hipSuccess;
   if (nrhs < 0 || grid <= 0) return hipErrorInvalidValue;
   AdjArgs<T> g;
   g.count = count; g.nrhs = nrhs; g.order = order; g.n = n; g.lda = lda; g.ldx = ldx;
-  g.ldg = ldg; g.L = L; g.X = Xs; g.Bb = Bb; g.G = G; g.W = W; g.counter = counter;
+  g.ldg = ldg; g.L = L; g.X = Xs; g.Bb = Bb; g.G = G; g.counter = counter;
   hipLaunchKernelGGL(chol_adjoint_kernel<T>, dim3(grid), dim3(NT), 0, s, g);
   return hipGetLastError();
 }
@@ -1400,19 +1247,18 @@ extern "C" hipError_t atlmx_k_dbatch_chol_adjoint(int count, const int *order, c
                                                   double *const *L, const int *lda, int nrhs,
                                                   double *const *X, double *const *Bb,
                                                   const int *ldx, double *const *G,
-                                                  const int *ldg, double *const *W, int *counter,
-                                                  int grid, hipStream_t s) {
-  return chol_adjoint<double>(count, order, n, L, lda, nrhs, X, Bb, ldx, G, ldg, W, counter,
-                              grid, s);
+                                                  const int *ldg, int *counter, int grid,
+                                                  hipStream_t s) {
+  return chol_adjoint<double>(count, order, n, L, lda, nrhs, X, Bb, ldx, G, ldg, counter, grid,
+                              s);
 }
 extern "C" hipError_t atlmx_k_sbatch_chol_adjoint(int count, const int *order, const int *n,
                                                   float *const *L, const int *lda, int nrhs,
                                                   float *const *X, float *const *Bb,
                                                   const int *ldx, float *const *G,
-                                                  const int *ldg, float *const *W, int *counter,
-                                                  int grid, hipStream_t s) {
-  return chol_adjoint<float>(count, order, n, L, lda, nrhs, X, Bb, ldx, G, ldg, W, counter,
-                             grid, s);
+                                                  const int *ldg, int *counter, int grid,
+                                                  hipStream_t s) {
+  return chol_adjoint<float>(count, order, n, L, lda, nrhs, X, Bb, ldx, G, ldg, counter, grid, s);
 }
 
 extern "C" hipError_t atlmx_k_dbatch_factor(int kind, int nb, int count, const int *order,

@@ -122,8 +122,8 @@ atlmx_batch *atlmx_sgemm_batch_plan(int TA, int TB, int count, const int *h_m, c
  * A^{-T} x-bar); posv_adjoint takes L[i] (potrf's lower triangle, its strict
  * upper triangle is zeroed), X[i] = A^{-1} B and Bb[i] = A^{-1} Xb and
  * writes G[i] = the gradient of <Xb, X> with respect to the lower triangle
- * of A[i], through Phi(L^T L-bar) and two triangular solves; W[i]: n x n
- * scratch (leading dimension n). */
+ * of A[i]: Phi(L^T L-bar) and its two triangular solves, carried out on the
+ * factors of rank 2 nrhs; W is not used (any pointer, or NULL). */
 atlmx_batch *atlmx_dgesv_t_batch_plan(int count, const int *h_n, double *const *d_A,
                                       const int *h_lda, int *const *d_ipiv, int nrhs,
                                       double *const *d_B, const int *h_ldb, int *d_info);
