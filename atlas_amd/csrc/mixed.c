@@ -418,6 +418,13 @@ static double ddot_dev(atlmx_ctx *c, int n, const double *u, const double *v, do
 }
 
 #define GM_RESTART 100
+/* An inner solve ends when its (preconditioned, recurrence) residual has
+ * fallen by this factor.  M^{-1} is applied in FP32, so the recurrence
+ * follows the true residual only to a few digits: at n = 16384, kappa 1e6
+ * a cycle gains three, whether it runs to 1e-4 in 9 steps or to 1e-12 in 27
+ * (four cycles and the same error either way: 35 steps, 170 ms, against
+ * 107, 320 ms).  At 1e-2 some systems need a further cycle. */
+#define GM_INNER_TOL 1e-4
 
 /* GMRES-based refinement (Carson and Higham, "Accelerating the solution of
  * linear systems by iterative refinement in three precisions", SIAM J. Sci.
@@ -506,7 +513,7 @@ static int gmres_refine(atlmx_ctx *c, const lp_fact *f, int N, int NRHS, const d
         g[k] = cs[k] * g[k];
         kk = k + 1;
         if (hn > 0.0) RT_CHECK(rout, atlmx_k_dscal2d(N, 1, 1.0 / hn, w, N, c->stream));
-        if (!(fabs(g[k + 1]) > 1e-12 * beta) || !(hn > 0.0)) break;
+        if (!(fabs(g[k + 1]) > GM_INNER_TOL * beta) || !(hn > 0.0)) break;
       }
       /* d = V y with H y = g (upper triangular, kk x kk); x += d */
       for (i = kk - 1; i >= 0; --i) {
