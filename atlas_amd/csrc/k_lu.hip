@@ -1,7 +1,7 @@
 /*
  * k_lu.hip -- the LU panel: partial-pivoting factorization of an m x w
- * column panel (w <= 64) in ONE cooperative launch, and the row-interchange
- * kernels around it.
+ * column panel (w <= 64) in ONE launch, and the row-interchange kernels
+ * around it.
  *
  * Replaces ATLAS's panel leaves -- getf2/LU1 (src/lapack/ATL_getf2.c:10-95),
  * LU2 (src/lapack/ATL_getrfC.c:46-136) and the threaded tgetf2 with its
@@ -11,25 +11,25 @@
  * the lower index, NaN never wins), swap the whole panel row, scale by the
  * reciprocal of the pivot when |p| >= SAFMIN (else divide), rank-1 update.
  *
- * Layout: the panel rows are spread over G workgroups of 256 threads; each
- * thread keeps RPT whole panel rows (w values each) in registers for the
- * whole factorization, so HBM is touched once to load and once to store.
+ * Layout: the panel rows are spread over G workgroups, one row per thread
+ * in registers for the whole factorization, so HBM is touched once to load
+ * and once to store.  No row moves during it: each thread keeps its row's
+ * current position, an interchange exchanges two positions, and the rows are
+ * stored to their final positions at the end.
  *
- * Cross-workgroup exchange, per column: every workgroup reduces its rows to
- * one candidate (wavefront shuffles, then LDS across the 4 wavefronts) and
- * publishes it in its record for the column's parity: the row index, |value|
- * and the candidate row, every 32 bits of payload in a 64-bit word whose
- * upper half is a tag unique to (launch, column).  A word is valid when its
- * tag is the current one, so no store has to wait for an earlier one to
- * land and no slot is ever reset.  Readers poll the G records' headers at
- * once (one lane per workgroup), reduce them in one wavefront, and then
- * fetch the one row they need: the winning candidate row, or, in the
- * winner's own workgroup, the row it swaps with.  Two record sets
- * (column parity) suffice: a workgroup can publish column c + 2 only after
- * reading every record of column c + 1, which each writer publishes only
- * after reading all of column c.  All exchanged words move with
- * device-coherent (sc1) accesses, so no L2 writeback/invalidate fence is
- * needed.
+ * Cross-workgroup exchange, per column (G > 1): every workgroup reduces its
+ * rows to one candidate (DPP within a wavefront, then LDS) and publishes it
+ * in its record for the column's parity: the position, |value| and the
+ * candidate row, every 32 bits of payload in a 64-bit word whose upper half
+ * is a tag unique to (launch, column).  A word is valid when its tag is the
+ * current one, so no store has to wait for an earlier one to land and no
+ * slot is ever reset.  Readers poll the G records' headers at once (one lane
+ * per workgroup), reduce them in one wavefront, and then fetch the winning
+ * row.  Two record sets (column parity) suffice: a workgroup can publish
+ * column c + 2 only after reading every record of column c + 1, which each
+ * writer publishes only after reading all of column c.  All exchanged words
+ * move with device-coherent (sc1) accesses, so no L2 writeback/invalidate
+ * fence is needed.
  */
 #include <hip/hip_runtime.h>
 #include <float.h>
@@ -40,6 +40,7 @@
 namespace {
 
 constexpr int NT = 256;
+constexpr int NTW = 512;    /* threads of the wide panel workgroup */
 constexpr int MAXG = 256;   /* cooperative workgroups at most (1 per CU) */
 constexpr int MAXW = ATLMX_PANEL_MAXW;
 constexpr int TALL_PARTS = 1024;   /* partial arg-maxes of the tall path */
@@ -48,35 +49,29 @@ template <typename T> struct Lim;
 template <> struct Lim<double> { __device__ static double safmin() { return DBL_MIN; } };
 template <> struct Lim<float> { __device__ static float safmin() { return FLT_MIN; } };
 
-template <typename T>
-__device__ inline void amax_combine(T &v, int &i, T v2, int i2) {
-  if (v2 > v || (v2 == v && i2 < i)) { v = v2; i = i2; }
-}
-
 /* Record of one workgroup for one column parity: 64-bit words tag << 32 |
- * payload, [0] the candidate's row index, [1], [2] the low and high halves
- * of its |value| as a double (-1 for NaN, -2 when the workgroup has no row
- * left), [RH + 2j], [RH + 2j + 1] the halves of entry j of the candidate
- * row.  One more record per parity holds the current row c (published by
- * workgroup 0, which holds rows 0..R-1 of the panel). */
+ * payload, [0] the candidate's position (INT_MAX: none), [1], [2] the low and
+ * high halves of its |value| as a double's bits (0: none, or no nonzero
+ * number), [RH + 2j], [RH + 2j + 1] the halves of entry j of the candidate
+ * row, j >= the column. */
 constexpr int RH = 4;
 constexpr int RECW = RH + 2 * MAXW;
 typedef unsigned long long u64;
 
 struct PanelSlots {
-  u64 *rec;          /* [2 parity][MAXG + 1][RECW]; record MAXG: the current row */
+  u64 *rec;          /* [2 parity][MAXG][RECW] */
   double *part_v;    /* tall path: per-workgroup arg-max partials */
   int *part_i;
 };
 
 __host__ __device__ inline size_t slots_bytes() {
-  return (size_t)2 * (MAXG + 1) * RECW * 8 + (size_t)TALL_PARTS * (8 + 4);
+  return (size_t)2 * MAXG * RECW * 8 + (size_t)TALL_PARTS * (8 + 4);
 }
 
 __device__ inline PanelSlots slots_view(void *base) {
   PanelSlots s;
   char *p = (char *)base;
-  s.rec = (u64 *)p;        p += (size_t)2 * (MAXG + 1) * RECW * 8;
+  s.rec = (u64 *)p;        p += (size_t)2 * MAXG * RECW * 8;
   s.part_v = (double *)p;  p += (size_t)TALL_PARTS * 8;
   s.part_i = (int *)p;
   return s;
@@ -102,148 +97,244 @@ __device__ inline double take_f64(u64 *p, unsigned tag) {
   return __longlong_as_double((long long)(((u64)hi << 32) | lo));
 }
 
-/* The panel rows of one workgroup live in LDS, row-major with a padded row
- * stride (W+1): a thread's own row is contiguous (its rank-1 update streams
- * through it), and column c of all rows is a stride-(W+1) gather. */
-template <typename T, int W, int R>
-__global__ __launch_bounds__(NT) void getf2_panel_lds_kernel(int m, int w, T *P, long ld,
-                                                         int row0, int *ipiv, int *info,
-                                                         void *scratch, int seq) {
-  constexpr int RPT = R / NT;
-  constexpr int LDW = W + 1;   /* odd stride: lanes hit distinct LDS banks */
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  T *rows = (T *)smem;                         /* [R][LDW] */
-  __shared__ double s_wv[NT / 64];
-  __shared__ int s_wi[NT / 64];
-  __shared__ T s_prow[W];
-  __shared__ int s_piv;
-  const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int rbase = g * R;                     /* first panel row of this workgroup */
-  PanelSlots S = slots_view(scratch);
-
-  for (int k = 0; k < w; ++k)
-#pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-      const int r = rbase + q * NT + tid;
-      rows[(q * NT + tid) * LDW + k] = (r < m) ? P[(size_t)k * ld + r] : T(0);
+/* arg-max over the wavefront of (key, then the lowest position): the key's
+ * halves one after the other with 32-bit DPP maxima; the low half and the
+ * positions are looked at only where the higher part ties.  key and pos
+ * become the winner's, in every lane. */
+template <int CTRL, int RM>
+__device__ __forceinline__ unsigned dpp_umax(unsigned v) {
+  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RM, 0xf, false);
+  return v > o ? v : o;
+}
+__device__ __forceinline__ unsigned wave_umax(unsigned v) {
+  v = dpp_umax<0x111, 0xf>(v);
+  v = dpp_umax<0x112, 0xf>(v);
+  v = dpp_umax<0x114, 0xf>(v);
+  v = dpp_umax<0x118, 0xf>(v);
+  v = dpp_umax<0x142, 0xa>(v);
+  v = dpp_umax<0x143, 0xc>(v);
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ void wave_argmax_key(u64 &key, int &pos) {
+  const unsigned hi = (unsigned)(key >> 32), lo = (unsigned)key;
+  const unsigned mh = wave_umax(hi);
+  u64 tie = __ballot(hi == mh);
+  if (tie & (tie - 1)) {
+    const unsigned ml = wave_umax(hi == mh ? lo : 0u);
+    tie = __ballot(hi == mh && lo == ml);
+    if (tie & (tie - 1)) {                         /* equal values: the lowest position */
+      const bool in = hi == mh && lo == ml;
+      const unsigned mp = wave_umax(in ? ~(unsigned)pos : 0u);
+      tie = __ballot(in && ~(unsigned)pos == mp);
     }
-  __syncthreads();
-
-  for (int c = 0; c < w; ++c) {
-    const int par = c & 1;
-    /* ---- local arg-max over my rows >= c ---- */
-    double bv = -2.0;
-    int bi = 0x7fffffff, bz = 0;
-#pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-      const int r = rbase + q * NT + tid;
-      if (r < m && r >= c) {
-        double v = (double)rows[(q * NT + tid) * LDW + c];
-        v = v < 0.0 ? -v : v;
-        if (!(v == v)) v = -1.0;
-        atlmx::argmax_combine(bv, bi, bz, v, r, 0);
-      }
-    }
-    atlmx::wave_argmax(bv, bi, bz);
-    if (lane == 0) { s_wv[wave] = bv; s_wi[wave] = bi; }
-    __syncthreads();
-
-    if (wave == 0) {
-      double wv = s_wv[0];
-      int wi = s_wi[0];
-#pragma unroll
-      for (int k = 1; k < NT / 64; ++k) atlmx::argmax_combine(wv, wi, bz, s_wv[k], s_wi[k], 0);
-      if (wv < 0.0) wi = 0x7fffffff;    /* only NaN or no rows: nothing to offer */
-      /* ---- publish this workgroup's record (and workgroup 0 the current
-       * row c), each word tagged; no store waits for another ---- */
-      const unsigned tag = (unsigned)seq * MAXW + (unsigned)c + 1u;
-      u64 *recs = S.rec + (size_t)par * (MAXG + 1) * RECW;
-      u64 *mine = recs + (size_t)g * RECW, *cur = recs + (size_t)MAXG * RECW;
-      if (lane < w) {
-        if (wi != 0x7fffffff) put_f64(mine + RH + 2 * lane, tag, (double)rows[(wi - rbase) * LDW + lane]);
-        if (g == 0) put_f64(cur + RH + 2 * lane, tag, (double)rows[c * LDW + lane]);
-      }
-      if (lane == 0) {
-        put_u32(mine, tag, (unsigned)wi);
-        put_f64(mine + 1, tag, wv);
-      }
-      /* ---- read the G headers (one lane per workgroup), reduce ---- */
-      double v = -2.0;
-      int i = 0x7fffffff, gi = 0;
-      for (int k0 = 0; k0 < G; k0 += 64) {
-        const int k = k0 + lane;
-        if (k < G) {
-          u64 *rk = recs + (size_t)k * RECW;
-          const int ik = (int)take_u32(rk, tag);
-          atlmx::argmax_combine(v, i, gi, take_f64(rk + 1, tag), ik, k);
-        }
-      }
-      atlmx::wave_argmax(v, i, gi);
-      /* all |a| zero or NaN: iamax answers the first row, i.e. c */
-      const int p = (v > 0.0) ? i : c;
-      if (lane < w) {
-        /* the pivot row: the winner's candidate (its own workgroup has it in
-         * LDS); the current row c: needed only where row p lives, i.e. in
-         * the winner's workgroup, which also has it in LDS when g == 0 */
-        const bool own = (p != c) && gi == g;
-        const T pr = (p == c) ? T(0)
-                              : (own ? rows[(p - rbase) * LDW + lane]
-                                     : (T)take_f64(recs + (size_t)gi * RECW + RH + 2 * lane, tag));
-        if (p != c) {
-          s_prow[lane] = pr;
-          /* swap the whole panel rows c and p where this workgroup holds
-           * them, one lane per column (p != c implies a nonzero pivot) */
-          if (p >= rbase && p < rbase + R) {
-            const T dr = (c >= rbase && c < rbase + R)
-                             ? rows[(c - rbase) * LDW + lane]
-                             : (T)take_f64(cur + RH + 2 * lane, tag);
-            rows[(p - rbase) * LDW + lane] = dr;
-          }
-          if (c >= rbase && c < rbase + R) rows[(c - rbase) * LDW + lane] = pr;
-        } else {
-          /* no interchange: the pivot row is row c itself, held by
-           * workgroup 0, published as the current row */
-          s_prow[lane] = (c >= rbase && c < rbase + R) ? rows[(c - rbase) * LDW + lane]
-                                                       : (T)take_f64(cur + RH + 2 * lane, tag);
-        }
-      }
-      if (lane == 0) {
-        s_piv = p;
-        if (g == 0) ipiv[c] = row0 + p;
-      }
-    }
-    __syncthreads();
-
-    const int p = s_piv;
-    const T pv = s_prow[c];
-    if (pv != T(0)) {
-      const bool recip = (pv < T(0) ? -pv : pv) >= Lim<T>::safmin();
-      const T rcp = T(1) / pv;
-#pragma unroll
-      for (int q = 0; q < RPT; ++q) {
-        const int r = rbase + q * NT + tid;
-        T *row = rows + (q * NT + tid) * LDW;
-        if (r < m && r > c) {
-          const T l = recip ? row[c] * rcp : row[c] / pv;
-          row[c] = l;
-#pragma unroll 8
-          for (int k = c + 1; k < w; ++k) row[k] -= l * s_prow[k];
-        }
-      }
-    } else if (g == 0 && tid == 0) {
-      atomicCAS(info, 0, row0 + c + 1);
-    }
-    /* LDS rows are rewritten next column: wait until all have read */
-    __syncthreads();
   }
+  const int w = __ffsll((long long)tie) - 1;
+  key = ((u64)mh << 32) | (unsigned)__builtin_amdgcn_readlane((int)lo, w);
+  pos = __builtin_amdgcn_readlane(pos, w);
+}
 
-  for (int k = 0; k < w; ++k)
+/* |v| as an integer that orders like it; NaN never better than zero */
+__device__ __forceinline__ u64 abs_key(double v) {
+  const u64 b = (u64)__double_as_longlong(v) & 0x7fffffffffffffffull;
+  return v == v ? b : 0ull;
+}
+
+/* entry n of a row of 16 lanes, to every lane of that row */
+template <int N> __device__ __forceinline__ double row_bcast(double v) {
+  return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + N, 0xf, 0xf, true);
+}
+template <int N> __device__ __forceinline__ float row_bcast(float v) {
+  return __builtin_amdgcn_update_dpp(0.0f, v, 0x150 + N, 0xf, 0xf, true);
+}
+
+/* b[n] = entry n of the 16 that every row of 16 lanes holds in p, to all
+ * lanes (all must be enabled: a DPP move from a disabled lane gives 0) */
+template <typename T, int N>
+__device__ __forceinline__ void row_spread(T (&b)[16], T p) {
+  if constexpr (N < 16) {
+    b[N] = row_bcast<N>(p);
+    row_spread<T, N + 1>(b, p);
+  }
+}
+
+template <typename T>
+struct PanelState {
+  int w, G, g, row0, seq;
+  int *ipiv, *info;
+  PanelSlots S;
+  T *s_prow;                     /* [64] the pivot row, from its column on, then zeros */
+  T *s_cand;                     /* [64] this workgroup's candidate row */
+  u64 *s_key; int *s_pos;        /* per wavefront */
+  int *s_piv;
+};
+
+/* Columns 64 - WA .. 64 - WA + 15 of the panel: a = this thread's row, pos =
+ * its position (-1: no row).  The loop is rolled, so that its code stays in
+ * the instruction cache (unrolled over the columns it was fetched anew for
+ * each, 1.6 us a column at one workgroup): an elimination step writes
+ * column k + 1 into register k, so the current column is always a[0], and
+ * the finished entry -- the multiplier, or the value a pivot row keeps --
+ * goes into the register freed at the end, a[WA - 1].  Step i finds columns
+ * C.. in [0, WA - i) and this segment's finished ones in [WA - i, WA), where
+ * the pivot row's entries are zero.
+ *
+ * The pivot row reaches the other lanes by DPP: each lane loads one entry of
+ * every 16 from LDS (four loads) and row_newbcast moves hand it on.
+ * Broadcast LDS reads return 64 lanes' worth of data for every two entries.
+ *
+ * Two barriers a column; with several workgroups the wavefront that holds
+ * the candidate does the exchange. */
+template <typename T, int NTH, int WA>
+__device__ __forceinline__ void panel_segment(const PanelState<T> &st, T (&a)[MAXW], int &pos) {
+  constexpr int NW = NTH / 64;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int i = 0; i < 16; ++i) {
+    const int C = MAXW - WA + i;
+    const T a0 = a[0];
+    if (C >= st.w) {                               /* beyond the panel: only move on */
 #pragma unroll
-    for (int q = 0; q < RPT; ++q) {
-      const int r = rbase + q * NT + tid;
-      if (r < m) P[(size_t)k * ld + r] = rows[(q * NT + tid) * LDW + k];
+      for (int k = 1; k < WA; ++k) a[k - 1] = a[k];
+      a[WA - 1] = a0;
+      continue;
     }
+    u64 key = pos >= C ? abs_key((double)a0) : 0ull;
+    int kp = pos >= C && (key != 0ull || pos == C) ? pos : 0x7fffffff;
+    wave_argmax_key(key, kp);
+    if (lane == 0) { st.s_key[wave] = key; st.s_pos[wave] = kp; }
+    __syncthreads();
+    int wsel = 0;
+    key = st.s_key[0];
+    kp = st.s_pos[0];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) {
+      const u64 k2 = st.s_key[q];
+      const int p2 = st.s_pos[q];
+      if (k2 > key || (k2 == key && p2 < kp)) { key = k2; kp = p2; wsel = q; }
+    }
+    kp = __builtin_amdgcn_readfirstlane(kp);
+    wsel = __builtin_amdgcn_readfirstlane(wsel);
+    if (wave == wsel) {
+      /* the candidate's holder lays its row out */
+      T *dst = st.G > 1 ? st.s_cand : st.s_prow;
+      if (pos == kp) {
+#pragma unroll
+        for (int k = 0; k < WA; ++k)
+          dst[k] = (k < WA - 16 || k < WA - i) ? a[k] : T(0);
+      }
+      if (st.G > 1) {
+        const unsigned tag = (unsigned)st.seq * MAXW + (unsigned)C + 1u;
+        u64 *recs = st.S.rec + (size_t)(C & 1) * MAXG * RECW;
+        u64 *mine = recs + (size_t)st.g * RECW;
+        const bool has = lane < MAXW - C;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (kp != 0x7fffffff && has) put_f64(mine + RH + 2 * lane, tag, (double)dst[lane]);
+        if (lane == 0) {
+          put_u32(mine, tag, (unsigned)kp);
+          put_u32(mine + 1, tag, (unsigned)key);
+          put_u32(mine + 2, tag, (unsigned)(key >> 32));
+        }
+        /* the G headers, one lane per workgroup */
+        u64 bk = 0ull;
+        int bp = 0x7fffffff, bg = 0;
+        for (int k = lane; k < st.G; k += 64) {
+          u64 *rk = recs + (size_t)k * RECW;
+          const int p2 = (int)take_u32(rk, tag);
+          const u64 k2 = (u64)take_u32(rk + 1, tag) | ((u64)take_u32(rk + 2, tag) << 32);
+          if (k2 > bk || (k2 == bk && p2 < bp)) { bk = k2; bp = p2; bg = k; }
+        }
+        const int mypos = bp;
+        wave_argmax_key(bk, bp);
+        kp = bp;                                   /* at least position C's holder offers it */
+        const int own = __ffsll((long long)__ballot(mypos == bp)) - 1;
+        const int gi = __builtin_amdgcn_readlane(bg, own);
+        if (lane < WA) {
+          T v = T(0);
+          if (has)
+            v = gi == st.g ? dst[lane]
+                           : (T)take_f64(recs + (size_t)gi * RECW + RH + 2 * lane, tag);
+          st.s_prow[lane] = v;
+        }
+      }
+      if (lane == 0) {
+        *st.s_piv = kp;
+        if (st.g == 0) st.ipiv[C] = st.row0 + kp;
+      }
+    }
+    __syncthreads();
+    const int p = *st.s_piv;
+    if (pos == p) pos = C;
+    else if (pos == C) pos = p;
+    T pr[WA / 16];
+#pragma unroll
+    for (int q = 0; q < WA / 16; ++q) pr[q] = st.s_prow[16 * q + (lane & 15)];
+    const T pv = st.s_prow[0];
+    const bool act = pos > C && pv != T(0);
+    const bool recip = (pv < T(0) ? -pv : pv) >= Lim<T>::safmin();   /* uniform */
+    const T l = act ? (recip ? a0 * (T(1) / pv) : a0 / pv) : T(0);
+    if (pv == T(0) && st.g == 0 && tid == 0) atomicCAS(st.info, 0, st.row0 + C + 1);
+    bool fin = __builtin_isfinite(l);
+#pragma unroll
+    for (int q = 0; q < WA / 16; ++q) fin = fin && __builtin_isfinite(pr[q]);
+    const bool plain = __ballot(!fin) == 0ull;
+#pragma unroll
+    for (int q = 0; q < WA / 16; ++q) {
+      T b[16];
+      row_spread<T, 0>(b, pr[q]);
+      if (plain) {                                 /* l = 0 or b = 0 changes nothing */
+#pragma unroll
+        for (int n = 0; n < 16; ++n)
+          if (16 * q + n > 0) a[16 * q + n - 1] = fma(-l, b[n], a[16 * q + n]);
+      } else {                                     /* nor may 0 * inf */
+#pragma unroll
+        for (int n = 0; n < 16; ++n)
+          if (16 * q + n > 0) {
+            const T v = a[16 * q + n];
+            a[16 * q + n - 1] = act && 16 * q + n < WA - i ? fma(-l, b[n], v) : v;
+          }
+      }
+    }
+    a[WA - 1] = act ? l : a0;
+  }
+}
+
+/* One row per thread.  What bounds it: the chain of one column -- key and
+ * arg-max, two barriers and LDS round trips, the winner's row laid out by
+ * its one lane, with G > 1 two device-coherent round trips (headers, then
+ * the winning row), the division and the update.  Measured per column, FP64:
+ * one workgroup (m = 256) 3.8 -> 1.5 us, 32 workgroups (m = 8192, average of
+ * its panels) 4.8 -> 3.7 us, against rows in LDS updated in place through
+ * read-modify-writes; getrf n = 500 2.95 -> 1.76 ms, n = 8192 57.6 -> 46.4. */
+template <typename T, int NTH>
+__global__ __launch_bounds__(NTH) void getf2_panel_kernel(int m, int w, T *P, long ld, int row0,
+                                                          int *ipiv, int *info, void *scratch,
+                                                          int seq) {
+  static_assert(MAXW == 64, "four segments of 16 columns");
+  __shared__ __attribute__((aligned(16))) T s_prow[MAXW], s_cand[MAXW];
+  __shared__ u64 s_key[NTH / 64];
+  __shared__ int s_pos[NTH / 64];
+  __shared__ int s_piv;
+  const int r = blockIdx.x * NTH + threadIdx.x;
+  PanelState<T> st;
+  st.w = w; st.G = gridDim.x; st.g = blockIdx.x; st.row0 = row0; st.seq = seq;
+  st.ipiv = ipiv; st.info = info; st.S = slots_view(scratch);
+  st.s_prow = s_prow; st.s_cand = s_cand; st.s_key = s_key; st.s_pos = s_pos; st.s_piv = &s_piv;
+  T a[MAXW];
+  int pos = r < m ? r : -1;
+#pragma unroll
+  for (int k = 0; k < MAXW; ++k) a[k] = (k < w && r < m) ? P[(size_t)k * ld + r] : T(0);
+  panel_segment<T, NTH, 64>(st, a, pos);
+  panel_segment<T, NTH, 48>(st, a, pos);
+  panel_segment<T, NTH, 32>(st, a, pos);
+  panel_segment<T, NTH, 16>(st, a, pos);
+  if (pos >= 0) {
+    /* segment s left its 16 columns in a[48 - 16 s ..] */
+#pragma unroll
+    for (int k = 0; k < MAXW; ++k)
+      if (k < w) P[(size_t)k * ld + pos] = a[48 - 16 * (k / 16) + k % 16];
+  }
 }
 
 __global__ void slots_init_kernel(u64 *h, size_t n) {
@@ -331,7 +422,7 @@ __global__ __launch_bounds__(NT) void tall_update_kernel(int m, int w, int c, T 
 template <typename T>
 hipError_t launch_tall(int m, int w, T *P, long ld, int row0, int *ipiv, int *info,
                        void *scratch, hipStream_t s) {
-  char *b = (char *)scratch + (size_t)2 * (MAXG + 1) * RECW * 8;   /* past the records */
+  char *b = (char *)scratch + (size_t)2 * MAXG * RECW * 8;   /* past the records */
   double *pv = (double *)b;                  /* TALL_G doubles, then TALL_G ints */
   int *pi = (int *)(pv + TALL_G);
   for (int c = 0; c < w; ++c) {
@@ -347,20 +438,16 @@ hipError_t launch_tall(int m, int w, T *P, long ld, int row0, int *ipiv, int *in
   return hipGetLastError();
 }
 
-template <typename T, int W, int R>
-hipError_t launch_wr(int G, void **args, hipStream_t s) {
-  static int attr_set = 0;
-  const int lds = R * (W + 1) * (int)sizeof(T);
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute((const void *)getf2_panel_lds_kernel<T, W, R>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) return e;
-    attr_set = 1;
-  }
-  return hipLaunchCooperativeKernel((const void *)getf2_panel_lds_kernel<T, W, R>, dim3(G),
-                                    dim3(NT), args, (unsigned)lds, s);
+template <typename T, int NTH>
+hipError_t launch_rows(int G, void **args, hipStream_t s) {
+  const void *f = (const void *)getf2_panel_kernel<T, NTH>;
+  if (G == 1) return hipLaunchKernel(f, dim3(1), dim3(NTH), args, 0, s);
+  return hipLaunchCooperativeKernel(f, dim3(G), dim3(NTH), args, 0, s);
 }
 
+/* Up to 512 rows are one workgroup's (no exchange); then 256 rows each, so
+ * that a workgroup's four wavefronts sit one per SIMD, up to 256 workgroups,
+ * then 512 rows each; beyond that the panel stays in HBM. */
 template <typename T>
 hipError_t launch_panel(int m, int w, T *P, long ld, int row0, int *ipiv, int *info,
                         void *scratch, int seq, hipStream_t s) {
@@ -368,17 +455,10 @@ hipError_t launch_panel(int m, int w, T *P, long ld, int row0, int *ipiv, int *i
   if (w > MAXW || ld < m || !P || !ipiv || !info || !scratch) return hipErrorInvalidValue;
   if (w > m || seq < 0 || seq >= ATLMX_PANEL_SEQ_MAX) return hipErrorInvalidValue;
   void *args[] = {&m, &w, &P, &ld, &row0, &ipiv, &info, &scratch, &seq};
-  /* rows per workgroup: 256, or 512 for taller panels (then w <= 32 in FP64
-   * so the LDS tile stays within 160 KB) */
-  if ((long)m <= (long)NT * MAXG) {
-    const int G = (m + NT - 1) / NT;
-    return launch_wr<T, MAXW, NT>(G, args, s);
-  }
-  if ((long)m > (long)2 * NT * MAXG) return launch_tall<T>(m, w, P, ld, row0, ipiv, info,
-                                                          scratch, s);
-  if (w > MAXW / 2) return hipErrorInvalidValue;
-  const int G = (m + 2 * NT - 1) / (2 * NT);
-  return launch_wr<T, MAXW / 2, 2 * NT>(G, args, s);
+  if (m > NT && m <= NTW) return launch_rows<T, NTW>(1, args, s);
+  if ((long)m <= (long)NT * MAXG) return launch_rows<T, NT>((m + NT - 1) / NT, args, s);
+  if ((long)m <= (long)NTW * MAXG) return launch_rows<T, NTW>((m + NTW - 1) / NTW, args, s);
+  return launch_tall<T>(m, w, P, ld, row0, ipiv, info, scratch, s);
 }
 
 /* ------------------------------------------------------------------------
@@ -654,7 +734,7 @@ extern "C" size_t atlmx_k_panel_scratch_bytes(int m, int w) {
 }
 
 extern "C" hipError_t atlmx_k_panel_scratch_init(void *scratch, hipStream_t s) {
-  const size_t n = (size_t)2 * (MAXG + 1) * RECW;  /* the records of both parities */
+  const size_t n = (size_t)2 * MAXG * RECW;  /* the records of both parities */
   hipLaunchKernelGGL(slots_init_kernel, dim3(256), dim3(256), 0, s, (u64 *)scratch, n);
   return hipGetLastError();
 }

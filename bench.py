@@ -284,7 +284,7 @@ def bench_lapack(n, seed, torch, X, log, reps=3):
     fl = 2.0 * n ** 3 / 3 - n ** 2 / 2.0 - n / 6.0
     out["getrf"] = {"ms": round(t * 1e3, 2), "gflops": round(fl / t / 1e9, 1)}
     # one more factorization with HIP events around the panel launches
-    # (getf2_panel_lds_kernel: bytes = the panel loaded and stored once) and
+    # (getf2_panel_kernel: bytes = the panel loaded and stored once) and
     # the GEMM launches (trailing updates and the panel recursion's, flops)
     Aw.copy_(A0)
     torch.cuda.synchronize()
@@ -296,7 +296,7 @@ def bench_lapack(n, seed, torch, X, log, reps=3):
     if pcnt:
         bw = pwork / pcnt / (pms / pcnt * 1e-3)
         out["roofline_panel"] = {
-            "bound": "hbm", "kernel": "getf2_panel_lds_kernel (FP64 LU panel)",
+            "bound": "hbm", "kernel": "getf2_panel_kernel (FP64 LU panel)",
             "achieved": round(bw / 1e9, 2), "peak": PEAK_HBM / 1e9, "unit": "GB/s",
             "frac": round(bw / PEAK_HBM, 5), "launches": pcnt,
             "avg_launch_ms": round(pms / pcnt, 4), "ms_total": round(pms, 2),
