@@ -12,8 +12,8 @@
  * kernel into a hipGraph.  Running the plan replays that graph on the
  * calling thread's stream.
  *
- * The autotuner times every candidate configuration of the LU and the GEMM
- * -- panel width 16 or 32, one to three persistent workgroups per CU; for GEMM the kernel
+ * The autotuner times every candidate configuration of the LU above order
+ * 256 and the GEMM -- panel width 16 or 32, one to three persistent workgroups per CU; for GEMM the kernel
  * (vector FMAs, or MFMA with one or four wavefronts per 64 x 64 tile) and
  * the workgroups per CU -- on a replica of up to AT_SAMPLE instances drawn evenly from the
  * ordered batch (well-conditioned synthetic data of the same sizes, so
@@ -271,6 +271,15 @@ static void autotune(atlmx_batch *p, const int *h_order, const int *h_n, const i
      * No more than instances, so that a few spread over all units (256 of
      * order 512: 0.74 ms with 256 workgroups, 0.99 with 512). */
     const int grid = (p->dbl ? 2 : 3) * cus;
+    p->nb = 32;
+    p->grid = p->count < grid ? (p->count > 0 ? p->count : 1) : grid;
+    free(sn); free(offA); free(hA);
+    return;
+  }
+  if ((p->kind == BK_GESV || p->kind == BK_GESVT) && p->maxn <= ATLMX_BATCH_ROWS) {
+    /* the LU with one panel row per thread: one panel width, and again as
+     * many workgroups as fit */
+    const int grid = 2 * cus;
     p->nb = 32;
     p->grid = p->count < grid ? (p->count > 0 ? p->count : 1) : grid;
     free(sn); free(offA); free(hA);

@@ -14,11 +14,13 @@
  *     32-row tiles, the right-hand sides among them, are accumulated from
  *     the finished columns on the matrix cores and multiplied by the diagonal
  *     block's inverse.
- *   gesv (LU, partial pivoting): the (n-k) x NB panel lives in LDS while it
- *     is factored with partial pivoting (workgroup arg-max per column, ties
- *     to the lower row, NaN never wins, like cblas_idamax), its interchanges
- *     are applied to the other columns, U12 is solved column by column and
- *     the trailing matrix is updated in 64 x 64 tiles.
+ *   gesv (LU, partial pivoting), orders up to 256: 32-column panels one row
+ *     per thread in registers, the columns right of them and the right-hand
+ *     sides in 16-column strips, each one wavefront's.  Larger orders: the
+ *     (n-k) x NB panel lives in LDS while it is factored (workgroup arg-max
+ *     per column, ties to the lower row, NaN never wins, like cblas_idamax),
+ *     its interchanges are applied to the other columns, U12 is solved column
+ *     by column and the trailing matrix is updated in 64 x 64 tiles.
  *
  * The GEMM work item is one 64 x 64 tile of one instance.
  */
@@ -26,10 +28,11 @@
 #include <float.h>
 #include <math.h>
 #include "kernels.h"
+#include "lu_panel.h"
 
 namespace {
 
-constexpr int NT = 256;
+constexpr int NT = ATLMX_BATCH_ROWS;
 constexpr int TS = 64;                 /* trailing-update / GEMM tile */
 constexpr int MAXR = ATLMX_BATCH_MAXRHS;
 
@@ -793,6 +796,318 @@ __device__ void wg_gesv(int n, T *A, long lda, int *ipiv, int nrhs, T *B, long l
 /* ---------------------------------------------------------------------- */
 /* Cholesky adjoint of one instance by one workgroup                       */
 /* ---------------------------------------------------------------------- */
+/* ---------------------------------------------------------------------- */
+/* LU factor + solve of one instance of order <= NT: one panel row a thread */
+/* ---------------------------------------------------------------------- */
+/* Right-looking, panels of PB = 32 columns held in registers, one row per
+ * thread (lu_panel.h).  The columns right of the panel are taken in strips
+ * of 16, each wholly one wavefront's, so a strip's steps need no barrier:
+ * gather the 32 rows that come to the top, put the displaced top rows where
+ * those came from, U12 = inv(L11) times the gathered rows, and the trailing
+ * rows -= L21 U12, products on the matrix cores formed transposed
+ * (D[column][row]: a lane's 16 neighbours run down a column of A; the U12
+ * accumulators are the operand of the update as they stand).  The
+ * right-hand sides are one more strip, in LDS, so the forward substitution
+ * costs no pass of its own.  The columns left of a panel get their
+ * interchanges once at the end, as one map per panel composed from the
+ * later panels' maps.
+ *
+ * Bound by the panel's chain (about 1 us a column, two workgroups to a
+ * compute unit hiding each other's); the form it replaces at these orders kept
+ * the panel in LDS, swapped rows one dependent load at a time in every
+ * column, and updated through uncoalesced tiles.  FP64, 4000 of order
+ * 8..256, one right-hand side: 8.9 -> 2.8 ms; FP32 8.0 -> 2.2. */
+constexpr int MAXPAN = NT / PB;
+
+template <typename T>
+struct RowsPanel {
+  int w, row0;
+  int *ipiv;
+  T *s_prow, *s_cand;
+  atlmx::u64 *s_key;
+  int *s_pos, *s_piv, *s_zero;
+  __device__ bool first() const { return true; }
+  __device__ void zero_pivot(int C) const { if (*s_zero == 0) *s_zero = row0 + C + 1; }
+};
+
+/* inv(L11), unit lower, L11 at s_l[c PLD + r]: every lane one column of the
+ * inverse, the multipliers by readlane from the lanes that hold the rows;
+ * to s_inv[l PLD + c] = inv(c, l) */
+template <typename T>
+__device__ __forceinline__ void unit_lower_inverse(const T *s_l, T *s_inv) {
+  const int ln = fresh_lane() & (PB - 1);
+  T v[PB], z[PB];
+#pragma unroll
+  for (int c = 0; c < PB; ++c) {
+    v[c] = c < ln ? s_l[c * PLD + ln] : T(0);
+    z[c] = c == ln ? T(1) : T(0);
+  }
+#pragma unroll
+  for (int j = 0; j < PB; ++j) {
+    /* ties step j's readlanes to z[j]: they depend on no step, and all 992
+     * scalars were read ahead and spilled */
+    asm volatile("" : "+v"(v[j]), "+v"(z[j]));
+#pragma unroll
+    for (int c = j + 1; c < PB; ++c) z[c] = fma(-z[j], bcast(v[j], c), z[c]);
+  }
+#pragma unroll
+  for (int c = 0; c < PB; ++c) s_inv[ln * PLD + c] = z[c];
+}
+
+template <typename T>
+struct GesvLds {
+  T *l11, *inv;            /* PB x PLD each */
+  T *part;                 /* 4 x MAXR x PB */
+  T *x;                    /* n x nrhs */
+  int *src, *dst;          /* PB each: row now at top j; where top row j went (-1: stays) */
+  unsigned char *map;      /* MAXPAN x NT: row -> position, relative to the panel */
+  unsigned char *fin;      /* NT */
+};
+
+template <typename T>
+__device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, T *B, long ldb,
+                             int *info, const GesvLds<T> &S, RowsPanel<T> st, bool trans) {
+  typedef TMfma<T> MF;
+  typedef typename MF::acc_t acc_t;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15;
+  const int nr_fwd = trans ? 0 : nrhs;             /* right-hand sides carried along */
+  if (tid == 0) *st.s_zero = 0;
+  for (int e = tid; e < n * nrhs; e += NT) S.x[e] = B[(size_t)(e / n) * ldb + e % n];
+  __syncthreads();
+
+  for (int k = 0; k < n; k += PB) {
+    const int kb = min(PB, n - k), mp = n - k;
+    const long lda = fresh(lda0);
+    /* ---- the panel ---- */
+    T a[PB];
+    int pos = tid < mp ? tid : -1;
+#pragma unroll
+    for (int c = 0; c < PB; ++c)
+      a[c] = (c < kb && tid < mp) ? A[(size_t)(k + c) * lda + k + tid] : T(0);
+    st.w = kb; st.row0 = k; st.ipiv = ipiv + k;
+    atlmx::panel_segment<T, NT, PB, 32, false>(st, a, pos);
+    atlmx::panel_segment<T, NT, PB, 16, false>(st, a, pos);
+    if (tid < PB) S.dst[tid] = -1;
+    __syncthreads();
+    if (pos >= 0) {
+      const long ldp = fresh(lda0);
+#pragma unroll
+      for (int c = 0; c < PB; ++c) {
+        const T v = a[16 - 16 * (c / 16) + c % 16];
+        if (c < kb) A[(size_t)(k + c) * ldp + k + pos] = v;
+        if (pos < PB) S.l11[c * PLD + pos] = (c < kb && c < pos) ? v : T(0);
+      }
+      S.map[(k / PB) * NT + tid] = (unsigned char)pos;
+      if (pos < kb) S.src[pos] = tid;
+      else if (tid < kb) S.dst[tid] = pos;
+    } else if (tid < PB) {                         /* beyond the matrix: nothing below the diagonal */
+#pragma unroll
+      for (int c = 0; c < PB; ++c) S.l11[c * PLD + tid] = T(0);
+    }
+    if (tid >= kb && tid < PB) S.src[tid] = 0;
+    __syncthreads();
+    const int ns = (n - k - kb + 15) / 16;         /* strips of A's columns */
+    if (ns == 0 && nr_fwd == 0) break;
+    if (wave == 0) unit_lower_inverse(S.l11, S.inv);
+    __syncthreads();
+
+    /* ---- strips: columns j0.. of A, then the right-hand sides.  cp(c) is
+     * column c's base; clamped columns are read but not written. ---- */
+    auto strip = [&](auto cp, int nc) {
+      acc_t xv[2], tv[2], u[2];
+#pragma unroll
+      for (int l = 0; l < 2; ++l)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = 16 * l + MF::drow(lane, e);
+          auto col = cp(min(li, nc - 1));
+          xv[l][e] = j < kb ? col[k + S.src[j]] : T(0);
+          tv[l][e] = j < kb ? col[k + j] : T(0);
+        }
+      /* U12 = inv(L11) X: u[c][col] as D[row][col], rows in the elements */
+#pragma unroll
+      for (int c = 0; c < 2; ++c) u[c] = acc_t{0, 0, 0, 0};
+#pragma unroll
+      for (int l = 0; l < 2; ++l)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = 16 * l + MF::drow(lane, e);
+#pragma unroll
+          for (int c = l; c < 2; ++c)
+            u[c] = MF::mma(S.inv[row * PLD + 16 * c + li], xv[l][e], u[c]);
+        }
+      __threadfence_block();                       /* every read above is done */
+      if (li < nc) {
+        auto col = cp(li);
+#pragma unroll
+        for (int l = 0; l < 2; ++l)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int j = 16 * l + MF::drow(lane, e);
+            if (j < kb) {
+              const int d = S.dst[j];
+              if (d >= 0) col[k + d] = tv[l][e];
+              col[k + j] = u[l][e];
+            }
+          }
+      }
+      __threadfence_block();                       /* the displaced rows are read below */
+      /* the rows below: D'[col][row] = sum over j of U(j, col) L21(row, j) */
+      for (int r0 = k + PB; r0 < n; r0 += 32) {    /* then kb == PB */
+        const int ra = min(r0 + li, n - 1), rb = min(r0 + 16 + li, n - 1);
+        acc_t d0 = acc_t{0, 0, 0, 0}, d1 = acc_t{0, 0, 0, 0}, c0, c1;
+        T b0[2][4], b1[2][4];
+#pragma unroll
+        for (int l = 0; l < 2; ++l)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const T *Lc = A + (size_t)(k + 16 * l + MF::drow(lane, e)) * lda;
+            b0[l][e] = Lc[ra];
+            b1[l][e] = Lc[rb];
+          }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          auto col = cp(min(MF::drow(lane, e), nc - 1));
+          c0[e] = col[ra];
+          c1[e] = col[rb];
+        }
+#pragma unroll
+        for (int l = 0; l < 2; ++l)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            d0 = MF::mma(u[l][e], b0[l][e], d0);
+            d1 = MF::mma(u[l][e], b1[l][e], d1);
+          }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = MF::drow(lane, e);
+          if (c < nc) {
+            auto col = cp(c);
+            if (r0 + li < n) col[ra] = c0[e] - d0[e];
+            if (r0 + 16 + li < n) col[rb] = c1[e] - d1[e];
+          }
+        }
+      }
+    };
+    for (int q = wave; q < ns; q += NT / 64) {
+      const int j0 = k + kb + 16 * q;
+      T *base = A + (size_t)j0 * lda;
+      strip([=](int c) { return base + (size_t)c * lda; }, min(16, n - j0));
+    }
+    if (nr_fwd > 0 && wave == (ns & 3)) {
+      T *xs = S.x;
+      strip([=](int c) { return xs + c * n; }, nr_fwd);
+    }
+    __syncthreads();
+  }
+
+  /* ---- the interchanges of the columns left of each panel: fin[i] = where
+   * the row at absolute index i ends, composed from the last panel back ---- */
+  {
+    const int np = (n + PB - 1) / PB;
+    if (tid < n) S.fin[tid] = (unsigned char)tid;
+    for (int q = np - 2; q >= 0; --q) {
+      const int k1 = (q + 1) * PB;                 /* the panel whose map enters now */
+      __syncthreads();
+      int f = 0;
+      if (tid >= k1 && tid < n) f = S.fin[k1 + S.map[(q + 1) * NT + tid - k1]];
+      __syncthreads();
+      if (tid >= k1 && tid < n) S.fin[tid] = (unsigned char)f;
+      const bool moved = tid >= k1 && tid < n && f != tid;
+      const long lda = fresh(lda0);
+      T v[PB];
+      if (moved) {
+#pragma unroll
+        for (int c = 0; c < PB; ++c) v[c] = A[(size_t)(q * PB + c) * lda + tid];
+      }
+      __syncthreads();
+      if (moved) {
+#pragma unroll
+        for (int c = 0; c < PB; ++c) A[(size_t)(q * PB + c) * lda + f] = v[c];
+      }
+    }
+  }
+  __syncthreads();
+  const int first0 = *st.s_zero;
+  if (tid == 0) *info = first0;
+  if (nrhs <= 0 || first0) return;
+
+  if (trans) {
+    /* A^T = U^T L^T P: U^T z = b, L^T w = z (unit), x = P^T w */
+    wg_trsv(n, nrhs, A, lda0, false, true, false, S.x, S.l11, S.part);
+    wg_trsv(n, nrhs, A, lda0, true, true, true, S.x, S.l11, S.part);
+    if (tid < nrhs)
+      for (int j = n - 1; j >= 0; --j) {
+        const int p = ipiv[j];
+        if (p != j) { const T t = S.x[tid * n + j]; S.x[tid * n + j] = S.x[tid * n + p]; S.x[tid * n + p] = t; }
+      }
+    __syncthreads();
+  } else {
+    /* ---- U x = y, blocks from the last: the columns right of block k
+     * contribute U(r, j) x(j), split over the wavefronts by 16 columns, then
+     * the 32 x 32 triangle, one unknown per lane, wavefront w solving
+     * right-hand side w in lanes 0..31 and w + 4 in lanes 32..63 ---- */
+    for (int k = (n - 1) / PB * PB; k >= 0; k -= PB) {
+      const long lda = fresh(lda0);
+      const int kb = min(PB, n - k), lane = fresh_lane(), li = lane & 15, lk = lane >> 4;
+      const int ln = lane & (PB - 1), rhs = wave + 4 * (lane / PB);
+      T uc[PB], rd = T(0);
+      if (wave < nrhs) {
+#pragma unroll
+        for (int j = 0; j < PB; ++j)
+          uc[j] = (ln < j && j < kb) ? A[(size_t)(k + j) * lda + k + ln] : T(0);
+        if (ln < kb) rd = T(1) / A[(size_t)(k + ln) * lda + k + ln];
+      }
+      acc_t acc[2] = {acc_t{0, 0, 0, 0}, acc_t{0, 0, 0, 0}};
+      const T *xr = S.x + (size_t)min(li, nrhs - 1) * n;
+      for (int j0 = k + PB + 16 * wave; j0 < n; j0 += 16 * (NT / 64)) {
+        T ua[2][4], b[4];
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4) {
+          const int j = j0 + 4 * s4 + lk;
+          const T *col = A + (size_t)min(j, n - 1) * lda + k;
+          ua[0][s4] = col[li];
+          ua[1][s4] = col[16 + li];
+          b[s4] = j < n ? xr[j] : T(0);
+        }
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4) {
+          acc[0] = MF::mma(ua[0][s4], b[s4], acc[0]);
+          acc[1] = MF::mma(ua[1][s4], b[s4], acc[1]);
+        }
+      }
+      if (li < nrhs) {
+        T *sp = S.part + wave * MAXR * PB;
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sp[li * PB + 16 * c + MF::drow(lane, e)] = acc[c][e];
+      }
+      __syncthreads();
+      if (wave < nrhs) {
+        T g = T(0);
+        if (rhs < nrhs && ln < kb) {
+          const T *sp = S.part + rhs * PB + ln;
+          g = S.x[(size_t)rhs * n + k + ln] -
+              ((sp[0] + sp[MAXR * PB]) + (sp[2 * MAXR * PB] + sp[3 * MAXR * PB]));
+        }
+#pragma unroll
+        for (int j = PB - 1; j >= 0; --j) {        /* steps past kb change nothing */
+          const T x = g * rd;                      /* lane j's is x_j */
+          T xj = bcast(x, j);
+          if (nrhs > 4) xj = lane < PB ? xj : bcast(x, PB + j);
+          g = ln == j ? x : fma(-uc[j], xj, g);
+        }
+        if (rhs < nrhs && ln < kb) S.x[(size_t)rhs * n + k + ln] = g;
+      }
+      __syncthreads();
+    }
+  }
+  for (int e = tid; e < n * nrhs; e += NT) B[(size_t)(e / n) * ldb + e % n] = S.x[e];
+}
+
 /* Given L (lower triangle of A after potrf; its strict upper triangle is
  * overwritten with zeros here), X = A^{-1} B and Bb = A^{-1} Xb (the solve's
  * adjoint), write to G the gradient of <Xb, X> with respect to the lower
@@ -897,6 +1212,34 @@ __global__ __launch_bounds__(NT) void gesv_batched_kernel(BatchArgs<T> g, int ma
     const int i = g.order[it];
     wg_gesv<T, NB>(g.n[i], g.A[i], g.lda[i], g.ipiv[i], g.nrhs, g.B ? g.B[i] : nullptr,
                    g.ldb ? g.ldb[i] : 1, &g.info[i], s_p, s_a, s_b, s_x, s_v, s_i, trans != 0);
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(NT, 2) void gesv_rows_batched_kernel(BatchArgs<T> g, int trans) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ __attribute__((aligned(16))) T s_prow[PB];
+  __shared__ atlmx::u64 s_key[NT / 64];
+  __shared__ int s_pos[NT / 64], s_src[PB], s_dst[PB], s_piv, s_zero, s_item;
+  __shared__ unsigned char s_map[MAXPAN * NT], s_fin[NT];
+  GesvLds<T> S;
+  S.l11 = (T *)smem;
+  S.inv = S.l11 + PB * PLD;
+  S.part = S.inv + PB * PLD;
+  S.x = S.part + 4 * MAXR * PB;                        /* maxn x nrhs */
+  S.src = s_src; S.dst = s_dst; S.map = s_map; S.fin = s_fin;
+  RowsPanel<T> st;
+  st.s_prow = st.s_cand = s_prow; st.s_key = s_key; st.s_pos = s_pos; st.s_piv = &s_piv;
+  st.s_zero = &s_zero; st.w = st.row0 = 0; st.ipiv = nullptr;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) s_item = atomicAdd(g.counter, 1);
+    __syncthreads();
+    const int it = __builtin_amdgcn_readfirstlane(s_item);
+    if (it >= g.count) return;
+    const int i = g.order[it];
+    wg_gesv_rows<T>(g.n[i], g.A[i], g.lda[i], g.ipiv[i], g.nrhs, g.B ? g.B[i] : nullptr,
+                    g.ldb ? g.ldb[i] : 1, &g.info[i], S, st, trans != 0);
   }
 }
 
@@ -1042,6 +1385,15 @@ hipError_t launch_gesv(const BatchArgs<T> &g, int maxn, int grid, int trans, hip
 }
 
 template <typename T>
+hipError_t launch_gesv_rows(const BatchArgs<T> &g, int maxn, int grid, int trans,
+                            hipStream_t s) {
+  const size_t lds = sizeof(T) * (2 * (size_t)PB * PLD + 4 * MAXR * PB + (size_t)maxn * g.nrhs);
+  if (maxn > NT || lds > 64 * 1024) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((gesv_rows_batched_kernel<T>), dim3(grid), dim3(NT), lds, s, g, trans);
+  return hipGetLastError();
+}
+
+template <typename T>
 hipError_t batch_factor(int kind, int nb, int count, const int *order, const int *n, T *const *A,
                         const int *lda, int *const *ipiv, int nrhs, T *const *B, const int *ldb,
                         int *info, int *counter, int maxn, int grid, hipStream_t s) {
@@ -1053,6 +1405,7 @@ hipError_t batch_factor(int kind, int nb, int count, const int *order, const int
   if (kind == 0) {
     if (nb == 16 || nb == 32) return launch_posv<T>(g, maxn, grid, s);   /* one panel width */
   } else if (kind == 1 || kind == 2) {      /* 2: solve with A^T */
+    if (maxn <= NT) return launch_gesv_rows<T>(g, maxn, grid, kind == 2, s);
     if (nb == 16) return launch_gesv<T, 16>(g, maxn, grid, kind == 2, s);
     if (nb == 32) return launch_gesv<T, 32>(g, maxn, grid, kind == 2, s);
   }

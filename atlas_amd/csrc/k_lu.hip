@@ -36,6 +36,7 @@
 #include <stdint.h>
 #include "kernels.h"
 #include "wave_argmax.h"
+#include "lu_panel.h"
 
 namespace {
 
@@ -45,10 +46,6 @@ constexpr int MAXG = 256;   /* cooperative workgroups at most (1 per CU) */
 constexpr int MAXW = ATLMX_PANEL_MAXW;
 constexpr int TALL_PARTS = 1024;   /* partial arg-maxes of the tall path */
 
-template <typename T> struct Lim;
-template <> struct Lim<double> { __device__ static double safmin() { return DBL_MIN; } };
-template <> struct Lim<float> { __device__ static float safmin() { return FLT_MIN; } };
-
 /* Record of one workgroup for one column parity: 64-bit words tag << 32 |
  * payload, [0] the candidate's position (INT_MAX: none), [1], [2] the low and
  * high halves of its |value| as a double's bits (0: none, or no nonzero
@@ -56,7 +53,9 @@ template <> struct Lim<float> { __device__ static float safmin() { return FLT_MI
  * row, j >= the column. */
 constexpr int RH = 4;
 constexpr int RECW = RH + 2 * MAXW;
-typedef unsigned long long u64;
+using atlmx::u64;
+using atlmx::Lim;
+using atlmx::wave_argmax_key;
 
 struct PanelSlots {
   u64 *rec;          /* [2 parity][MAXG][RECW] */
@@ -97,66 +96,6 @@ __device__ inline double take_f64(u64 *p, unsigned tag) {
   return __longlong_as_double((long long)(((u64)hi << 32) | lo));
 }
 
-/* arg-max over the wavefront of (key, then the lowest position): the key's
- * halves one after the other with 32-bit DPP maxima; the low half and the
- * positions are looked at only where the higher part ties.  key and pos
- * become the winner's, in every lane. */
-template <int CTRL, int RM>
-__device__ __forceinline__ unsigned dpp_umax(unsigned v) {
-  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RM, 0xf, false);
-  return v > o ? v : o;
-}
-__device__ __forceinline__ unsigned wave_umax(unsigned v) {
-  v = dpp_umax<0x111, 0xf>(v);
-  v = dpp_umax<0x112, 0xf>(v);
-  v = dpp_umax<0x114, 0xf>(v);
-  v = dpp_umax<0x118, 0xf>(v);
-  v = dpp_umax<0x142, 0xa>(v);
-  v = dpp_umax<0x143, 0xc>(v);
-  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
-__device__ __forceinline__ void wave_argmax_key(u64 &key, int &pos) {
-  const unsigned hi = (unsigned)(key >> 32), lo = (unsigned)key;
-  const unsigned mh = wave_umax(hi);
-  u64 tie = __ballot(hi == mh);
-  if (tie & (tie - 1)) {
-    const unsigned ml = wave_umax(hi == mh ? lo : 0u);
-    tie = __ballot(hi == mh && lo == ml);
-    if (tie & (tie - 1)) {                         /* equal values: the lowest position */
-      const bool in = hi == mh && lo == ml;
-      const unsigned mp = wave_umax(in ? ~(unsigned)pos : 0u);
-      tie = __ballot(in && ~(unsigned)pos == mp);
-    }
-  }
-  const int w = __ffsll((long long)tie) - 1;
-  key = ((u64)mh << 32) | (unsigned)__builtin_amdgcn_readlane((int)lo, w);
-  pos = __builtin_amdgcn_readlane(pos, w);
-}
-
-/* |v| as an integer that orders like it; NaN never better than zero */
-__device__ __forceinline__ u64 abs_key(double v) {
-  const u64 b = (u64)__double_as_longlong(v) & 0x7fffffffffffffffull;
-  return v == v ? b : 0ull;
-}
-
-/* entry n of a row of 16 lanes, to every lane of that row */
-template <int N> __device__ __forceinline__ double row_bcast(double v) {
-  return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + N, 0xf, 0xf, true);
-}
-template <int N> __device__ __forceinline__ float row_bcast(float v) {
-  return __builtin_amdgcn_update_dpp(0.0f, v, 0x150 + N, 0xf, 0xf, true);
-}
-
-/* b[n] = entry n of the 16 that every row of 16 lanes holds in p, to all
- * lanes (all must be enabled: a DPP move from a disabled lane gives 0) */
-template <typename T, int N>
-__device__ __forceinline__ void row_spread(T (&b)[16], T p) {
-  if constexpr (N < 16) {
-    b[N] = row_bcast<N>(p);
-    row_spread<T, N + 1>(b, p);
-  }
-}
-
 template <typename T>
 struct PanelState {
   int w, G, g, row0, seq;
@@ -166,139 +105,53 @@ struct PanelState {
   T *s_cand;                     /* [64] this workgroup's candidate row */
   u64 *s_key; int *s_pos;        /* per wavefront */
   int *s_piv;
-};
 
-/* Columns 64 - WA .. 64 - WA + 15 of the panel: a = this thread's row, pos =
- * its position (-1: no row).  The loop is rolled, so that its code stays in
- * the instruction cache (unrolled over the columns it was fetched anew for
- * each, 1.6 us a column at one workgroup): an elimination step writes
- * column k + 1 into register k, so the current column is always a[0], and
- * the finished entry -- the multiplier, or the value a pivot row keeps --
- * goes into the register freed at the end, a[WA - 1].  Step i finds columns
- * C.. in [0, WA - i) and this segment's finished ones in [WA - i, WA), where
- * the pivot row's entries are zero.
- *
- * The pivot row reaches the other lanes by DPP: each lane loads one entry of
- * every 16 from LDS (four loads) and row_newbcast moves hand it on.
- * Broadcast LDS reads return 64 lanes' worth of data for every two entries.
- *
- * Two barriers a column; with several workgroups the wavefront that holds
- * the candidate does the exchange. */
-template <typename T, int NTH, int WA>
-__device__ __forceinline__ void panel_segment(const PanelState<T> &st, T (&a)[MAXW], int &pos) {
-  constexpr int NW = NTH / 64;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  for (int i = 0; i < 16; ++i) {
-    const int C = MAXW - WA + i;
-    const T a0 = a[0];
-    if (C >= st.w) {                               /* beyond the panel: only move on */
-#pragma unroll
-      for (int k = 1; k < WA; ++k) a[k - 1] = a[k];
-      a[WA - 1] = a0;
-      continue;
+  __device__ bool first() const { return g == 0; }
+  __device__ void zero_pivot(int C) const { atomicCAS(info, 0, row0 + C + 1); }
+
+  /* Called by the wavefront whose lane laid the candidate (key, kp) out in
+   * s_cand: publish it, find the winner over the workgroups and put its row
+   * into s_prow (zeros in [64 - C, WA)); returns the winner's position. */
+  __device__ __forceinline__ int exchange(int C, u64 key, int kp, int WA) const {
+    const int lane = threadIdx.x & 63;
+    const T *dst = s_cand;
+    const unsigned tag = (unsigned)seq * MAXW + (unsigned)C + 1u;
+    u64 *recs = S.rec + (size_t)(C & 1) * MAXG * RECW;
+    u64 *mine = recs + (size_t)g * RECW;
+    const bool has = lane < MAXW - C;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (kp != 0x7fffffff && has) put_f64(mine + RH + 2 * lane, tag, (double)dst[lane]);
+    if (lane == 0) {
+      put_u32(mine, tag, (unsigned)kp);
+      put_u32(mine + 1, tag, (unsigned)key);
+      put_u32(mine + 2, tag, (unsigned)(key >> 32));
     }
-    u64 key = pos >= C ? abs_key((double)a0) : 0ull;
-    int kp = pos >= C && (key != 0ull || pos == C) ? pos : 0x7fffffff;
-    wave_argmax_key(key, kp);
-    if (lane == 0) { st.s_key[wave] = key; st.s_pos[wave] = kp; }
-    __syncthreads();
-    int wsel = 0;
-    key = st.s_key[0];
-    kp = st.s_pos[0];
-#pragma unroll
-    for (int q = 1; q < NW; ++q) {
-      const u64 k2 = st.s_key[q];
-      const int p2 = st.s_pos[q];
-      if (k2 > key || (k2 == key && p2 < kp)) { key = k2; kp = p2; wsel = q; }
+    /* the G headers, one lane per workgroup */
+    u64 bk = 0ull;
+    int bp = 0x7fffffff, bg = 0;
+    for (int k = lane; k < G; k += 64) {
+      u64 *rk = recs + (size_t)k * RECW;
+      const int p2 = (int)take_u32(rk, tag);
+      const u64 k2 = (u64)take_u32(rk + 1, tag) | ((u64)take_u32(rk + 2, tag) << 32);
+      if (k2 > bk || (k2 == bk && p2 < bp)) { bk = k2; bp = p2; bg = k; }
     }
-    kp = __builtin_amdgcn_readfirstlane(kp);
-    wsel = __builtin_amdgcn_readfirstlane(wsel);
-    if (wave == wsel) {
-      /* the candidate's holder lays its row out */
-      T *dst = st.G > 1 ? st.s_cand : st.s_prow;
-      if (pos == kp) {
-#pragma unroll
-        for (int k = 0; k < WA; ++k)
-          dst[k] = (k < WA - 16 || k < WA - i) ? a[k] : T(0);
-      }
-      if (st.G > 1) {
-        const unsigned tag = (unsigned)st.seq * MAXW + (unsigned)C + 1u;
-        u64 *recs = st.S.rec + (size_t)(C & 1) * MAXG * RECW;
-        u64 *mine = recs + (size_t)st.g * RECW;
-        const bool has = lane < MAXW - C;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (kp != 0x7fffffff && has) put_f64(mine + RH + 2 * lane, tag, (double)dst[lane]);
-        if (lane == 0) {
-          put_u32(mine, tag, (unsigned)kp);
-          put_u32(mine + 1, tag, (unsigned)key);
-          put_u32(mine + 2, tag, (unsigned)(key >> 32));
-        }
-        /* the G headers, one lane per workgroup */
-        u64 bk = 0ull;
-        int bp = 0x7fffffff, bg = 0;
-        for (int k = lane; k < st.G; k += 64) {
-          u64 *rk = recs + (size_t)k * RECW;
-          const int p2 = (int)take_u32(rk, tag);
-          const u64 k2 = (u64)take_u32(rk + 1, tag) | ((u64)take_u32(rk + 2, tag) << 32);
-          if (k2 > bk || (k2 == bk && p2 < bp)) { bk = k2; bp = p2; bg = k; }
-        }
-        const int mypos = bp;
-        wave_argmax_key(bk, bp);
-        kp = bp;                                   /* at least position C's holder offers it */
-        const int own = __ffsll((long long)__ballot(mypos == bp)) - 1;
-        const int gi = __builtin_amdgcn_readlane(bg, own);
-        if (lane < WA) {
-          T v = T(0);
-          if (has)
-            v = gi == st.g ? dst[lane]
-                           : (T)take_f64(recs + (size_t)gi * RECW + RH + 2 * lane, tag);
-          st.s_prow[lane] = v;
-        }
-      }
-      if (lane == 0) {
-        *st.s_piv = kp;
-        if (st.g == 0) st.ipiv[C] = st.row0 + kp;
-      }
+    const int mypos = bp;
+    wave_argmax_key(bk, bp);
+    kp = bp;                                   /* at least position C's holder offers it */
+    const int own = __ffsll((long long)__ballot(mypos == bp)) - 1;
+    const int gi = __builtin_amdgcn_readlane(bg, own);
+    if (lane < WA) {
+      T v = T(0);
+      if (has)
+        v = gi == g ? dst[lane]
+                       : (T)take_f64(recs + (size_t)gi * RECW + RH + 2 * lane, tag);
+      s_prow[lane] = v;
     }
-    __syncthreads();
-    const int p = *st.s_piv;
-    if (pos == p) pos = C;
-    else if (pos == C) pos = p;
-    T pr[WA / 16];
-#pragma unroll
-    for (int q = 0; q < WA / 16; ++q) pr[q] = st.s_prow[16 * q + (lane & 15)];
-    const T pv = st.s_prow[0];
-    const bool act = pos > C && pv != T(0);
-    const bool recip = (pv < T(0) ? -pv : pv) >= Lim<T>::safmin();   /* uniform */
-    const T l = act ? (recip ? a0 * (T(1) / pv) : a0 / pv) : T(0);
-    if (pv == T(0) && st.g == 0 && tid == 0) atomicCAS(st.info, 0, st.row0 + C + 1);
-    bool fin = __builtin_isfinite(l);
-#pragma unroll
-    for (int q = 0; q < WA / 16; ++q) fin = fin && __builtin_isfinite(pr[q]);
-    const bool plain = __ballot(!fin) == 0ull;
-#pragma unroll
-    for (int q = 0; q < WA / 16; ++q) {
-      T b[16];
-      row_spread<T, 0>(b, pr[q]);
-      if (plain) {                                 /* l = 0 or b = 0 changes nothing */
-#pragma unroll
-        for (int n = 0; n < 16; ++n)
-          if (16 * q + n > 0) a[16 * q + n - 1] = fma(-l, b[n], a[16 * q + n]);
-      } else {                                     /* nor may 0 * inf */
-#pragma unroll
-        for (int n = 0; n < 16; ++n)
-          if (16 * q + n > 0) {
-            const T v = a[16 * q + n];
-            a[16 * q + n - 1] = act && 16 * q + n < WA - i ? fma(-l, b[n], v) : v;
-          }
-      }
-    }
-    a[WA - 1] = act ? l : a0;
+    return kp;
   }
-}
+};
 
 /* One row per thread.  What bounds it: the chain of one column -- key and
  * arg-max, two barriers and LDS round trips, the winner's row laid out by
@@ -307,7 +160,7 @@ __device__ __forceinline__ void panel_segment(const PanelState<T> &st, T (&a)[MA
  * one workgroup (m = 256) 3.8 -> 1.5 us, 32 workgroups (m = 8192, average of
  * its panels) 4.8 -> 3.7 us, against rows in LDS updated in place through
  * read-modify-writes; getrf n = 500 2.95 -> 1.76 ms, n = 8192 57.6 -> 46.4. */
-template <typename T, int NTH>
+template <typename T, int NTH, bool MULTI>
 __global__ __launch_bounds__(NTH) void getf2_panel_kernel(int m, int w, T *P, long ld, int row0,
                                                           int *ipiv, int *info, void *scratch,
                                                           int seq) {
@@ -325,10 +178,10 @@ __global__ __launch_bounds__(NTH) void getf2_panel_kernel(int m, int w, T *P, lo
   int pos = r < m ? r : -1;
 #pragma unroll
   for (int k = 0; k < MAXW; ++k) a[k] = (k < w && r < m) ? P[(size_t)k * ld + r] : T(0);
-  panel_segment<T, NTH, 64>(st, a, pos);
-  panel_segment<T, NTH, 48>(st, a, pos);
-  panel_segment<T, NTH, 32>(st, a, pos);
-  panel_segment<T, NTH, 16>(st, a, pos);
+  atlmx::panel_segment<T, NTH, MAXW, 64, MULTI>(st, a, pos);
+  atlmx::panel_segment<T, NTH, MAXW, 48, MULTI>(st, a, pos);
+  atlmx::panel_segment<T, NTH, MAXW, 32, MULTI>(st, a, pos);
+  atlmx::panel_segment<T, NTH, MAXW, 16, MULTI>(st, a, pos);
   if (pos >= 0) {
     /* segment s left its 16 columns in a[48 - 16 s ..] */
 #pragma unroll
@@ -440,9 +293,11 @@ hipError_t launch_tall(int m, int w, T *P, long ld, int row0, int *ipiv, int *in
 
 template <typename T, int NTH>
 hipError_t launch_rows(int G, void **args, hipStream_t s) {
-  const void *f = (const void *)getf2_panel_kernel<T, NTH>;
-  if (G == 1) return hipLaunchKernel(f, dim3(1), dim3(NTH), args, 0, s);
-  return hipLaunchCooperativeKernel(f, dim3(G), dim3(NTH), args, 0, s);
+  if (G == 1)
+    return hipLaunchKernel((const void *)getf2_panel_kernel<T, NTH, false>, dim3(1), dim3(NTH),
+                           args, 0, s);
+  return hipLaunchCooperativeKernel((const void *)getf2_panel_kernel<T, NTH, true>, dim3(G),
+                                    dim3(NTH), args, 0, s);
 }
 
 /* Up to 512 rows are one workgroup's (no exchange); then 256 rows each, so

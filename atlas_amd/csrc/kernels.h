@@ -204,6 +204,7 @@ hipError_t atlmx_k_sbatch_chol_adjoint(int count, const int *order, const int *n
  * tile_start[p] = first tile of instance order[p] (count + 1 entries).
  * variant: 0 vector FMAs (256 threads per tile), 1 MFMA with one
  * wavefront per tile, 2 MFMA with four wavefronts per tile. */
+#define ATLMX_BATCH_ROWS 256  /* largest order of the LU with one panel row per thread */
 #define ATLMX_BATCH_TILE 64
 hipError_t atlmx_k_dbatch_gemm(int count, int ta, int tb, const int *order, const int *m,
                                const int *n,

@@ -1,0 +1,87 @@
+"""The batched LU factor + solve with one panel row per thread (orders up to
+256): edges of its 32-column panels, 16-column strips and 32-row tiles, every
+right-hand-side count, zero pivots in every part of a panel, the transposed
+solve, and a batch one order above, which takes the other kernel.  Pivots
+equal the oracle's; |P A - L U| <= gamma_n |L| |U| (Higham, Accuracy and
+Stability, Theorem 9.3, doubled for the product with inv(L11)); the solve by
+its normwise backward error, c n u with c the growth observed (<= 64)."""
+import numpy as np
+import pytest
+
+import atlas_amd as X
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(torch, sizes, dt, nrhs, zeros=(), trans=False):
+    rng = np.random.default_rng(sum(sizes) * 3 + nrhs)
+    u = np.finfo(dt).eps / 2
+    A0 = [rng.uniform(-1, 1, (n, n)).astype(dt) for n in sizes]
+    for i, col in zeros:
+        A0[i][:, col] = 0
+    B0 = [rng.uniform(-1, 1, (n, nrhs)).astype(dt) for n in sizes]
+    dev = lambda m: torch.tensor(np.ascontiguousarray(m.T), device="cuda")   # noqa: E731
+    As, Bs = [dev(a) for a in A0], [dev(b) for b in B0]
+    piv = [torch.full((n,), -1, dtype=torch.int32, device="cuda") for n in sizes]
+    info = torch.full((len(sizes),), -7, dtype=torch.int32, device="cuda")
+    mk = X.gesv_t_batch if trans else X.gesv_batch
+    with mk(As, piv, Bs if nrhs else [], info) as plan:
+        plan.run()
+        torch.cuda.synchronize()
+    inf, zero = info.cpu().numpy(), dict(zeros)
+    for i, n in enumerate(sizes):
+        F, p = As[i].cpu().numpy().T.astype(np.float64), piv[i].cpu().numpy()
+        A = A0[i].astype(np.float64)
+        if dt == np.float64:
+            assert np.array_equal(p, O.getrf(A.copy(order="F"))[1]), n
+        P = A.copy()
+        for k, q in enumerate(p):
+            assert k <= q < n
+            P[[k, q]] = P[[q, k]]
+        L, U = np.tril(F, -1) + np.eye(n), np.triu(F)
+        assert np.all(np.abs(P - L @ U) <= 4 * (n + 1) * u * (np.abs(L) @ np.abs(U)) + 1e-300), n
+        assert np.abs(np.tril(F, -1)).max(initial=0) <= 1.0
+        if i in zero:
+            assert inf[i] == zero[i] + 1
+            continue
+        assert inf[i] == 0
+        if nrhs:
+            x, b = Bs[i].cpu().numpy().T.astype(np.float64), B0[i].astype(np.float64)
+            M = A.T if trans else A
+            r = np.abs(b - M @ x).max(0) / (np.abs(M).sum(1).max() * np.abs(x).max(0))
+            assert np.all(r <= 64 * max(n, 8) * u), (n, r.max() / (n * u))
+
+
+EDGES = [1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 79, 81, 95, 97, 127, 129, 160, 191,
+         193, 224, 255, 256]
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("nrhs", [0, 1, 3, 5, 8])
+def test_gesv_panel_strip_and_tile_edges(dt, nrhs):
+    import torch
+    X.use_torch_stream()
+    _run(torch, EDGES, dt, nrhs)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("nrhs", [1, 8])
+def test_gesv_transposed(dt, nrhs):
+    import torch
+    X.use_torch_stream()
+    _run(torch, EDGES, dt, nrhs, trans=True)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_gesv_zero_pivots(dt):
+    import torch
+    X.use_torch_stream()
+    cols = [0, 15, 16, 31, 32, 47, 63, 99]
+    _run(torch, [100] * len(cols) + [64], dt, 2, list(enumerate(cols)))
+
+
+def test_gesv_above_the_one_row_orders():
+    import torch
+    X.use_torch_stream()
+    _run(torch, [257, 40, 300], np.float64, 2)
