@@ -23,12 +23,73 @@ constexpr int TNB = ATLMX_TRI_NB;
  * diagonal sub-blocks are inverted by substitution (lane = column), then
  * two doubling levels fill in the off-diagonal parts,
  *     inv([A 0; C B]) = [inv(A) 0; -inv(B) C inv(A) inv(B)],
- * as two small products each, spread over all threads.  LDS holds the
- * factor's strict lower triangle, the inverse's strict lower triangle
- * transposed into the strict upper half of the same array, the inverse's
- * diagonal, and the product's intermediate; every product loop runs over
- * the nonzero (triangular) range only.
+ * as two products each on the matrix cores, the first one's accumulators
+ * (element e of lane group g is row drow(e)) being the operand of the second
+ * as they stand.  The products run over the triangles' zeros too, so a block
+ * with an infinity or a NaN takes loops over the nonzero range instead.
+ * One or two blocks (a panel's): 23 -> 15 us; the loops, of one dependent LDS
+ * read pair per term, had bound it.
  * ---------------------------------------------------------------------- */
+typedef double iv_d4 __attribute__((ext_vector_type(4)));
+typedef float iv_f4 __attribute__((ext_vector_type(4)));
+template <typename T> struct IvMfma;
+template <> struct IvMfma<double> {
+  typedef iv_d4 acc_t;
+  __device__ static acc_t mma(double a, double b, acc_t c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  __device__ static int drow(int lane, int r) { return (lane >> 4) + 4 * r; }
+};
+template <> struct IvMfma<float> {
+  typedef iv_f4 acc_t;
+  __device__ static acc_t mma(float a, float b, acc_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  __device__ static int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+
+/* The doubling levels on the matrix cores.  Ls: the factor, lower, [i][j];
+ * Xs: the inverse, zero but for its four 16x16 diagonal blocks on entry. */
+template <typename T>
+__device__ __forceinline__ void tri_doubling_mfma(const T (*Ls)[TNB + 1], T (*Xs)[TNB + 1]) {
+  typedef IvMfma<T> MF;
+  typedef typename MF::acc_t acc_t;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  if (wave < 2) {                                  /* 16: pair at 32 wave */
+    const int c0 = 32 * wave, r0 = c0 + 16;
+    acc_t t = acc_t{0, 0, 0, 0}, x = acc_t{0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      t = MF::mma(Ls[r0 + li][c0 + 4 * s + lk], Xs[c0 + 4 * s + lk][c0 + li], t);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x = MF::mma(Xs[r0 + li][r0 + MF::drow(lane, e)], t[e], x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) Xs[r0 + MF::drow(lane, e)][c0 + li] = -x[e];
+  }
+  __syncthreads();
+  /* 32: wavefront w forms columns 16 (w & 1) of T and, from them, its 16x16
+   * tile of X21 */
+  const int jb = 16 * (wave & 1), ib = 16 * (wave >> 1);
+  acc_t t[2], x = acc_t{0, 0, 0, 0};
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    t[r] = acc_t{0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      t[r] = MF::mma(Ls[32 + 16 * r + li][4 * s + lk], Xs[4 * s + lk][jb + li], t[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      x = MF::mma(Xs[32 + ib + li][32 + 16 * r + MF::drow(lane, e)], t[r][e], x);
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < 4; ++e) Xs[32 + ib + MF::drow(lane, e)][jb + li] = -x[e];
+  __syncthreads();
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void tri_inv_kernel(int lower, int unit, int n,
                                                       const T *__restrict__ A, long lda,
@@ -36,7 +97,8 @@ __global__ __launch_bounds__(256) void tri_inv_kernel(int lower, int unit, int n
                                                       const int *abort_flag) {
   static_assert(TNB == 64, "tri_inv_kernel is written for 64x64 blocks");
   if (abort_flag && *abort_flag) return;
-  __shared__ T Ls[TNB][TNB + 1];   /* (i > j): L(i,j) at [i][j], X(i,j) at [j][i] */
+  __shared__ T Ls[TNB][TNB + 1];   /* (i > j): L(i,j) at [i][j]; loops: X(i,j) at [j][i] */
+  __shared__ T Xs[TNB][TNB + 1];   /* matrix cores: the inverse */
   __shared__ T dL[TNB], dX[TNB];
   __shared__ T Tb[32][33];
   const int tid = threadIdx.x;
@@ -45,7 +107,9 @@ __global__ __launch_bounds__(256) void tri_inv_kernel(int lower, int unit, int n
   const int nb = min(TNB, n - b0);
   /* load: the block as the lower triangle L (L = U^T for an upper block);
    * outside the n x n matrix the block is the identity */
+  int odd = 0;
   for (int e = tid; e < TNB * TNB; e += 256) {
+    Xs[e >> 6][e & (TNB - 1)] = T(0);
     const int r = e & (TNB - 1), c = e >> 6;           /* element (r, c) of the block */
     const int i = lower ? r : c, j = lower ? c : r;    /* its place in L */
     if (i < j) continue;
@@ -53,9 +117,11 @@ __global__ __launch_bounds__(256) void tri_inv_kernel(int lower, int unit, int n
     if (r < nb && c < nb) v = A[(size_t)(b0 + c) * lda + (b0 + r)];
     else v = (i == j) ? T(1) : T(0);
     if (i == j) dL[i] = (unit && i < nb) ? T(1) : v;
-    else Ls[i][j] = v;
+    else { Ls[i][j] = v; odd |= !__builtin_isfinite(v); }
   }
-  __syncthreads();
+  /* (an upper half of Ls not yet written is read by no product below: every
+   * L block there lies wholly below the diagonal) */
+  odd = __syncthreads_or(odd);
   /* the 16x16 diagonal sub-blocks, by substitution: lane (q, c) builds
    * column c of inv(L_qq) */
   if (tid < 64) {
@@ -72,11 +138,14 @@ __global__ __launch_bounds__(256) void tri_inv_kernel(int lower, int unit, int n
     for (int i = 0; i < 16; ++i) {
       if (i == c) dX[o + c] = x[i];
       else if (i > c) Ls[o + c][o + i] = x[i];
+      if (i >= c) Xs[o + i][o + c] = x[i];
+      odd |= !__builtin_isfinite(x[i]);
     }
   }
-  __syncthreads();
-  /* doubling: blocks of 2h from two blocks of h */
-#pragma unroll
+  odd = __syncthreads_or(odd);
+  if (!odd) tri_doubling_mfma<T>(Ls, Xs);
+  /* doubling by loops: blocks of 2h from two blocks of h */
+  if (odd)
   for (int h = 16; h < TNB; h *= 2) {
     const int nout = (TNB / (2 * h)) * h * h;   /* 512, then 1024 */
     /* T = L21 * X11, L21 = L(r0.., c0..), X11 = X(c0.., c0..) lower */
@@ -105,7 +174,8 @@ __global__ __launch_bounds__(256) void tri_inv_kernel(int lower, int unit, int n
     const int r = e & (TNB - 1), c = e >> 6;
     const int i = lower ? r : c, j = lower ? c : r;    /* inv(U) = inv(L)^T */
     T v = T(0);
-    if (i == j) v = dX[i];
+    if (!odd) v = i >= j ? Xs[i][j] : T(0);
+    else if (i == j) v = dX[i];
     else if (i > j) v = Ls[j][i];
     out[(size_t)c * TNB + r] = v;
   }

@@ -816,7 +816,7 @@ __device__ void wg_gesv(int n, T *A, long lda, int *ipiv, int nrhs, T *B, long l
  * compute unit hiding each other's); the form it replaces at these orders kept
  * the panel in LDS, swapped rows one dependent load at a time in every
  * column, and updated through uncoalesced tiles.  FP64, 4000 of order
- * 8..256, one right-hand side: 8.9 -> 2.8 ms; FP32 8.0 -> 2.2. */
+ * 8..256, one right-hand side: 8.9 -> 2.8 ms. */
 constexpr int MAXPAN = NT / PB;
 
 template <typename T>

@@ -864,10 +864,14 @@ hipError_t launch_gemm(int ta, int tb, int M, int N, int K, T alpha, const T *A,
   const long ntiles = (long)g.tiles_m * g.tiles_n;
   if (ntiles > (1L << 30)) return hipErrorInvalidValue;
   g.per_xcd = (int)((ntiles + 7) / 8);
-  /* an in-place product (C is an operand, within one tile row or column of
-   * 128) and the K bands keep the 128-tile */
-  if (C != A && C != B && !(tri >= KX_KBAND_AL && tri <= KX_KBAND_RBU)) {
-    const int ts = gemm_tile(M, N, K);
+  /* The K bands keep the 128-tile.  So does an in-place product (C is an
+   * operand, within one tile row or column: a workgroup reads all of its
+   * operand before it writes), unless it fits one of 64 (FP64 64 x 64 x 64:
+   * 19 us in the 128-tile, 8 in the 64-tile). */
+  const bool in_place = C == A || C == B;
+  if ((!in_place || ((C != B || M <= 64) && (C != A || N <= 64))) &&
+      !(tri >= KX_KBAND_AL && tri <= KX_KBAND_RBU)) {
+    const int ts = in_place ? 64 : gemm_tile(M, N, K);
     if (ts == 64) {
       const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
       if (K <= 128) return launch_small_t<T, 64, 1>(ta, tb, g, s);
