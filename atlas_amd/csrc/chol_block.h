@@ -1,0 +1,207 @@
+/*
+ * chol_block.h -- the 32 x 32 pieces of a Cholesky factorization: sums of
+ * row tiles on the matrix cores, a diagonal block's factor and inverse by
+ * one wavefront.  Shared by the diagonal block of one large matrix
+ * (k_chol.hip) and the batched kernels (k_batched.hip).
+ */
+#ifndef ATLMX_CHOL_BLOCK_H
+#define ATLMX_CHOL_BLOCK_H
+
+#include <hip/hip_runtime.h>
+#include <math.h>
+
+namespace atlmx {
+
+/* v from lane `src` (a constant) to every lane of the wavefront */
+__device__ inline double bcast(double v, int src) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), src);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ inline float bcast(float v, int src) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+}
+template <typename T> __device__ inline T dsqrt(T x);
+template <> __device__ inline double dsqrt<double>(double x) { return sqrt(x); }
+template <> __device__ inline float dsqrt<float>(float x) { return sqrtf(x); }
+
+typedef double td4 __attribute__((ext_vector_type(4)));
+typedef float tf4 __attribute__((ext_vector_type(4)));
+template <typename T> struct TMfma;
+template <> struct TMfma<double> {
+  typedef td4 acc_t;
+  __device__ static acc_t mma(double a, double b, acc_t c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  /* v_mfma_f64_16x16x4f64: lane l, element r holds D[(l>>4) + 4r][l&15] */
+  __device__ static int drow(int lane, int r) { return (lane >> 4) + 4 * r; }
+};
+template <> struct TMfma<float> {
+  typedef tf4 acc_t;
+  __device__ static acc_t mma(float a, float b, acc_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  /* v_mfma_f32_16x16x4f32: lane l, element r holds D[4(l>>4) + r][l&15] */
+  __device__ static int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+
+constexpr int PB = 32;
+constexpr int PLD = PB + 1;
+
+template <typename T> struct Rng;
+template <> struct Rng<double> {
+  __device__ static double rsq(double d) { return __builtin_amdgcn_rsq(d); }
+  __device__ static bool plain(double d) { return d >= 1e-280 && d <= 1e280; }
+};
+template <> struct Rng<float> {
+  __device__ static float rsq(float d) { return __builtin_amdgcn_rsqf(d); }
+  __device__ static bool plain(float d) { return d >= 1e-30f && d <= 1e30f; }
+};
+
+/* sd = sqrt(d) and ri = 1 / sd (d > 0), each within an ulp: the hardware
+ * reciprocal square root and two coupled Newton steps (one in FP32), a
+ * shorter chain than the library's square root and division; outside the
+ * range where no step can over- or underflow, those. */
+template <typename T>
+__device__ inline void sqrt_inv(T d, T &sd, T &ri) {
+  if (Rng<T>::plain(d)) {
+    T y = Rng<T>::rsq(d), g = d * y, h = T(0.5) * y;
+#pragma unroll
+    for (int it = 0; it < (sizeof(T) == 8 ? 2 : 1); ++it) {
+      const T r = fma(-h, g, T(0.5));
+      g = fma(g, r, g);
+      h = fma(h, r, h);
+    }
+    sd = fma(fma(-g, g, d), h, g);
+    ri = T(2) * h;
+    ri = fma(fma(-ri, sd, T(1)), ri, ri);
+  } else {
+    sd = dsqrt(d);
+    ri = T(1) / sd;
+  }
+}
+
+/* acc[ci][rj] += sum over j in [j0, j1) of Y(16 ci + c, j) X(16 rj + r, j):
+ * lane (li, lk) reads Y(16 ci + li, j + lk) at y[ci][(j + lk) ys] and X
+ * likewise.  j1 - j0 is a multiple of 4 U; the next U steps' operands are
+ * loaded before the current steps' MFMAs. */
+template <typename T, int NC, int RJ, int U>
+__device__ __forceinline__ void panel_acc(typename TMfma<T>::acc_t (&acc)[NC][RJ],
+                                          const T *const (&y)[NC], long ys,
+                                          const T *const (&x)[RJ], long xs, int j0, int j1) {
+  const int lk = (threadIdx.x & 63) >> 4;
+  T yc[U][NC], xc[U][RJ];
+  auto load = [&](int j) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) yc[u][c] = y[c][(size_t)(j + 4 * u + lk) * ys];
+#pragma unroll
+      for (int r = 0; r < RJ; ++r) xc[u][r] = x[r][(size_t)(j + 4 * u + lk) * xs];
+    }
+  };
+  if (j0 >= j1) return;
+  load(j0);
+  for (int j = j0; j < j1; j += 4 * U) {
+    T ya[U][NC], xa[U][RJ];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) ya[u][c] = yc[u][c];
+#pragma unroll
+      for (int r = 0; r < RJ; ++r) xa[u][r] = xc[u][r];
+    }
+    if (j + 4 * U < j1) load(j + 4 * U);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int r = 0; r < RJ; ++r) acc[c][r] = TMfma<T>::mma(ya[u][c], xa[u][r], acc[c][r]);
+  }
+}
+
+template <typename acc_t, int NC, int RJ>
+__device__ __forceinline__ void zero_tile(acc_t (&t)[NC][RJ]) {
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int r = 0; r < RJ; ++r) t[c][r] = acc_t{0, 0, 0, 0};
+}
+
+/* w <- w inv^T for a tile held as accumulators: out[c][r] = the sum over l of
+ * inv(c, l) w(l, r), the inverse (lower) at s_inv[l PLD + c] in LDS */
+template <typename T, int RJ>
+__device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][RJ],
+                                               const T *s_inv) {
+  typename TMfma<T>::acc_t out[2][RJ];
+  const int lane = threadIdx.x & 63, li = lane & 15;
+  zero_tile(out);
+#pragma unroll
+  for (int l = 0; l < 2; ++l)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 16 * l + TMfma<T>::drow(lane, e);
+#pragma unroll
+      for (int c = l; c < 2; ++c) {                /* inv(c, l) = 0 above the diagonal */
+        const T a = s_inv[row * PLD + 16 * c + li];
+#pragma unroll
+        for (int r = 0; r < RJ; ++r) out[c][r] = TMfma<T>::mma(a, w[l][r][e], out[c][r]);
+      }
+    }
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int r = 0; r < RJ; ++r) w[c][r] = out[c][r];
+}
+
+/* A scalar, or this lane's number, that the compiler takes for a new value
+ * here: without it the products of lda with dozens of column numbers, and
+ * one 64-bit mask for every lane compare, are computed ahead of the panel
+ * loop and spilled across it (the Cholesky: 252 scalar spills). */
+__device__ __forceinline__ long fresh(long v) {
+  int lo = __builtin_amdgcn_readfirstlane((int)v);   /* a leading dimension: 31 bits */
+  asm volatile("" : "+s"(lo));
+  return lo;
+}
+__device__ __forceinline__ int fresh_lane() {
+  int l = threadIdx.x & 63;
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
+/* Wavefront 0: the Cholesky factor of the 32 x 32 block at s_d[c PLD + r]
+ * (identity beyond the matrix), lanes 0..31 one row each, and its inverse,
+ * lanes 32..63 one column each: both are the same elimination step,
+ * v[c] -= v[j] L(c, j), the inverse's columns starting from the identity's.
+ * Column j's entries reach all lanes by readlane.  Returns 0 or 1 + the
+ * failing column; v holds the row of L or the column of the inverse. */
+template <typename T>
+__device__ __forceinline__ int block_factor(T (&v)[PB], const T *s_d) {
+  const int lane = fresh_lane();
+  int fail = 0;
+#pragma unroll
+  for (int c = 0; c < PB; ++c)
+    v[c] = lane < PB ? s_d[c * PLD + lane] : (c == lane - PB ? T(1) : T(0));
+#pragma unroll
+  for (int j = 0; j < PB; ++j) {
+    if (!fail) {
+      const T d = bcast(v[j], j);
+      if (!(d > T(0))) {
+        fail = j + 1;                              /* uniform: every lane saw the same d */
+      } else {
+        T sd, ri;
+        sqrt_inv(d, sd, ri);
+        v[j] = lane == j ? sd : v[j] * ri;
+#pragma unroll
+        for (int c = j + 1; c < PB; ++c) v[c] = fma(-v[j], bcast(v[j], c), v[c]);
+      }
+    }
+  }
+  return fail;
+}
+
+}  // namespace atlmx
+
+#endif

@@ -1,133 +1,171 @@
 /*
- * k_chol.hip -- Cholesky of one diagonal block (n <= 128) in registers, and
- * the solve of the panel below (right of) it.
+ * k_chol.hip -- Cholesky of one diagonal block (n <= 128) with the inverses
+ * of its 64x64 diagonal blocks, and the solve of the panel below (right of)
+ * it.
  *
  * Replaces the leaves of ATLAS's recursive Cholesky: the closed-form 4x4,
  * 3x3, 2x2 kernels (src/lapack/ATL_potrfL.c:104-202, ATL_potrfU.c:98-197)
- * and the small-N recursion above them.  The whole block is held in the
- * registers of one 256-thread workgroup and factored right-looking, one
- * column at a time: rank-1 update of the trailing triangle with the
- * unscaled column over the pivot; the square roots and the column scaling
- * are applied once, when the block is written back.  A non-positive (or NaN) pivot stops the
- * factorization and records the 1-based global column in *info, as
- * ATL_potrfL.c:238-240 does; later kernels of the same Cholesky see the
+ * and the small-N recursion above them.  A non-positive (or NaN) pivot
+ * stops the factorization and records the 1-based global column in *info,
+ * as ATL_potrfL.c:238-240 does; later kernels of the same Cholesky see the
  * nonzero info and do nothing.  Only the referenced triangle is read or
  * written.
  */
 #include <hip/hip_runtime.h>
 #include "kernels.h"
+#include "chol_block.h"
 
 namespace {
 
 constexpr int CNB = ATLMX_CHOL_NB;
 constexpr int NT = 256;
 
-template <typename T>
-__device__ inline T dsqrt(T x);
-template <>
-__device__ inline double dsqrt<double>(double x) { return sqrt(x); }
-template <>
-__device__ inline float dsqrt<float>(float x) { return sqrtf(x); }
+using namespace atlmx;
 
-/* 1/x for the rank-1 multipliers: the hardware reciprocal refined by
- * Newton steps (two for double, one for float), within an ulp or so of
- * the rounded quotient and a short dependent chain on every column step. */
-__device__ inline double rcp_nr(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-  return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-}
-__device__ inline float rcp_nr(float x) {
-  const float r = __builtin_amdgcn_rcpf(x);
-  return __builtin_fmaf(r, __builtin_fmaf(-x, r, 1.0f), r);
-}
-
-/* The block lives in registers: thread (ti, tj) of a 16 x 16 grid holds the
- * 8 x 8 tile of rows ti*8.., columns tj*8.. (tiles above the diagonal stay
- * idle).  Step k: the owners of column k publish it as it stands (below the
- * pivot, zeros above) and the pivot d_k through LDS, and every tile right
- * of column k subtracts a(i,k) * a(j,k) / d_k in registers.  Column k stays
- * unscaled: L(i,k) = a(i,k) / sqrt(d_k) and L(k,k) = sqrt(d_k) are formed
- * for the whole block at write-back, so no square root or division by it
- * sits on the step-to-step chain.  One barrier per step: the column buffers
- * alternate with the parity of k, so a step's writes never meet the
- * previous step's reads, and every thread reads the same d_k, so a failed
- * pivot stops all of them at once.  The eight steps of a tile column are
- * unrolled, so every register index is fixed at compile time. */
+/* One workgroup, left-looking in 32-column panels with the pieces of the
+ * batched Cholesky (chol_block.h): the diagonal tile's sum split over the
+ * four wavefronts, its factor and inverse by wavefront 0, the row tiles
+ * below (at most three, one per other wavefront) accumulated meanwhile and
+ * then multiplied by the inverse.  Every second panel completes a 64x64
+ * diagonal block, whose inverse the panel solve needs, [i11 0; -i22 L21 i11,
+ * i22]: formed here from the two 32x32 inverses instead of by a launch of
+ * its own.  L(i, k) is A[i rs + k cs], so that Upper (A = U^T U, L = U^T) is
+ * the same code.  What bounds it: four times the one-wavefront factor of 32
+ * columns (5 us).  128 columns, FP64: 87 us for one barrier-separated step
+ * per column, and 15 for the inverses' launch, -> 71 us for both. */
 template <typename T>
-__global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long lda,
+__global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long lda, T *inv,
                                                    int info_base, int *info) {
+  typedef TMfma<T> MF;
+  typedef typename MF::acc_t acc_t;
+  constexpr int BLK = PB * PLD, IB = 64;
   if (*info != 0) return;
-  __shared__ T col[2][CNB];
-  __shared__ T piv[CNB];
-  const int tid = threadIdx.x;
-  const int ti = tid >> 4, tj = tid & 15;
-  const bool own = ti >= tj;
-  T a[8][8];
+  __shared__ T s_blk[4 * BLK], s_i[2][BLK];
+  __shared__ int s_ready, s_fail;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  const long rs = lower ? 1 : lda, cs = lower ? lda : 1;
+  if (tid == 0) s_ready = s_fail = 0;
+  __syncthreads();
+  for (int k = 0; k < n; k += PB) {
+    const int kb = min(PB, n - k), p = k / PB;
+    const T *yp[2] = {A + (long)min(k + li, n - 1) * rs, A + (long)min(k + 16 + li, n - 1) * rs};
+    {
+      acc_t acc[2][2];
+      zero_tile(acc);
+      const int w = k / 4;                         /* a multiple of 8 */
+      panel_acc<T, 2, 2, 2>(acc, yp, cs, yp, cs, wave * w, wave * w + w);
+      T *sp = s_blk + wave * BLK;
 #pragma unroll
-  for (int r = 0; r < 8; ++r)
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int i = ti * 8 + r, j = tj * 8 + c;
-      a[r][c] = (own && i < n && j < n && i >= j)
-                    ? (lower ? A[(size_t)j * lda + i] : A[(size_t)i * lda + j])
-                    : T(0);
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sp[(16 * c + MF::drow(lane, e)) * PLD + 16 * r + li] = acc[c][r][e];
     }
-  int done = n;
-  const int nkt = (n + 7) / 8;
-  for (int kt = 0; kt < nkt && done == n; ++kt) {
+    __syncthreads();
+    for (int e = tid; e < PB * PB; e += NT) {
+      const int c = e / PB, r = e % PB;
+      T *o = s_blk + c * PLD + r;
+      T v = r == c ? T(1) : T(0);                  /* beyond the matrix: the identity */
+      if (r < kb && c < kb && r >= c)
+        v = A[(long)(k + r) * rs + (long)(k + c) * cs] -
+            ((o[0] + o[BLK]) + (o[2 * BLK] + o[3 * BLK]));
+      *o = v;
+    }
+    __syncthreads();
+    const int nt = (n - k + PB - 1) / PB;
+    if (wave == 0) {
+      T v[PB];
+      const int fail = block_factor(v, s_blk);
+      const int ln = fresh_lane();
+      if (ln < PB) {
+        /* on failure the columns before the failing one, as far as they are */
+        const int nc = fail ? fail - 1 : PB;
 #pragma unroll
-    for (int kc = 0; kc < 8; ++kc) {
-      const int k = kt * 8 + kc;
-      if (k >= n) break;
-      T *ck = col[k & 1];
-      if (tj == kt && own) {
+        for (int c = 0; c < PB; ++c)
+          if (c <= ln && c < nc && ln < kb) A[(long)(k + ln) * rs + (long)(k + c) * cs] = v[c];
+      } else {
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          const int i = ti * 8 + r;
-          ck[i] = (i > k && i < n) ? a[r][kc] : T(0);
-        }
-        if (ti == kt) piv[k] = a[kc][kc];
+        for (int c = 0; c < PB; ++c) s_i[p & 1][(ln - PB) * PLD + c] = v[c];
       }
-      __syncthreads();
-      const T d = piv[k];
-      if (!__builtin_amdgcn_readfirstlane((int)(d > T(0)))) {
-        if (tid == 0) atomicCAS(info, 0, info_base + k + 1);
-        done = k;
-        break;
+      if (ln == 0) {
+        if (fail) s_fail = k + fail;
+        __hip_atomic_store(&s_ready, p + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
-      if (own && tj >= kt) {
-        const T rd = rcp_nr(d);
-        T x[8], y[8];
+    } else if (wave < nt) {                        /* row tile `wave`; then kb == PB */
+      const int ra = k + wave * PB + li, rb = ra + 16;
+      const T *xp[2] = {A + (long)min(ra, n - 1) * rs, A + (long)min(rb, n - 1) * rs};
+      acc_t acc[2][2], w[2][2];
+      zero_tile(acc);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) x[r] = ck[ti * 8 + r];
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int c = 0; c < 8; ++c) y[c] = ck[tj * 8 + c] * rd;
+        for (int r = 0; r < 2; ++r)
 #pragma unroll
-        for (int r = 0; r < 8; ++r)
+          for (int e = 0; e < 4; ++e)
+            w[c][r][e] = xp[r][(long)(k + 16 * c + MF::drow(lane, e)) * cs];
+      panel_acc<T, 2, 2, 4>(acc, yp, cs, xp, cs, 0, k);
 #pragma unroll
-          for (int c = 0; c < 8; ++c) a[r][c] -= x[r] * y[c];
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < 2; ++r) w[c][r] -= acc[c][r];
+      while (__hip_atomic_load(&s_ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < p + 1)
+        __builtin_amdgcn_s_sleep(1);
+      if (!s_fail) {
+        tile_times_inv<T, 2>(w, s_i[p & 1]);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            T *col = A + (long)(k + 16 * c + MF::drow(lane, e)) * cs;
+            if (ra < n) col[(long)ra * rs] = w[c][0][e];
+            if (rb < n) col[(long)rb * rs] = w[c][1][e];
+          }
       }
     }
-  }
-  /* write back the factored columns (the whole block when it succeeded; on
-   * failure the columns before the failing one, as the reference leaves
-   * them factored), each scaled by its pivot's square root */
-  if (own) {
+    __syncthreads();
+    if (s_fail) {
+      if (tid == 0) atomicCAS(info, 0, info_base + s_fail);
+      return;
+    }
+    if (!(p & 1) && k + PB < n) continue;
+    /* ---- inverse of the 64x64 block b: wavefront w forms columns 16 (w & 1)
+     * of L21 i11 and from them its 16x16 tile of X21 ---- */
+    const int b = p / 2, r0 = IB * b + PB, two = p & 1;
+    T *out = inv + (size_t)b * IB * IB;            /* inv(L)(r, c), transposed for Upper */
+    auto put = [&](int r, int c, T v) { out[lower ? c * IB + r : r * IB + c] = v; };
+    for (int e = tid; e < PB * PB; e += NT) {
+      const int c = e / PB, r = e % PB;
+      put(r, c, s_i[0][c * PLD + r]);
+      put(PB + r, PB + c, two ? s_i[1][c * PLD + r] : (r == c ? T(1) : T(0)));
+      put(r, PB + c, T(0));
+      if (!two) put(PB + r, c, T(0));
+    }
+    if (two) {
+      const int jb = 16 * (wave & 1), ib = 16 * (wave >> 1);
+      acc_t t[2], x = acc_t{0, 0, 0, 0};
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int j = tj * 8 + c;
-      if (j >= done) continue;
-      const T sd = dsqrt(piv[j]), rs = T(1) / sd;
+      for (int r = 0; r < 2; ++r) {
+        const int row = r0 + 16 * r + li;
+        T l[8];
 #pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const int i = ti * 8 + r;
-        if (i < n && i >= j) {
-          const T v = (i == j) ? sd : a[r][c] * rs;
-          if (lower) A[(size_t)j * lda + i] = v;
-          else A[(size_t)i * lda + j] = v;
-        }
+        for (int s = 0; s < 8; ++s)
+          l[s] = row < n ? A[(long)row * rs + (long)(IB * b + 4 * s + lk) * cs] : T(0);
+        t[r] = acc_t{0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+          t[r] = MF::mma(l[s], s_i[0][(jb + li) * PLD + 4 * s + lk], t[r]);
       }
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          x = MF::mma(s_i[1][(16 * r + MF::drow(lane, e)) * PLD + ib + li], t[r][e], x);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) put(PB + ib + MF::drow(lane, e), jb + li, -x[e]);
     }
   }
 }
@@ -144,30 +182,12 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
  * (the MFMA's four k lane groups take k = 16 lk + t in step t); a product's
  * result is turned into the next one's operand layout through the
  * wavefront's own slice of LDS, so no workgroup barrier is needed. */
-template <typename T> struct CMfma;
-template <> struct CMfma<double> {
-  typedef double acc_t __attribute__((ext_vector_type(4)));
-  __device__ static acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  /* v_mfma_f64_16x16x4f64: lane l, element r holds D[(l>>4) + 4r][l&15] */
-  __device__ static int drow(int lane, int r) { return (lane >> 4) + 4 * r; }
-};
-template <> struct CMfma<float> {
-  typedef float acc_t __attribute__((ext_vector_type(4)));
-  __device__ static acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  /* v_mfma_f32_16x16x4f32: lane l, element r holds D[4(l>>4) + r][l&15] */
-  __device__ static int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
-
 template <typename T>
 __global__ __launch_bounds__(NT) void chol_panel_solve_kernel(int lower, int nr, int jb,
                                                               const T *__restrict__ D, long lda,
                                                               const T *__restrict__ inv, T *P,
                                                               const int *info) {
-  typedef CMfma<T> MF;
+  typedef TMfma<T> MF;
   typedef typename MF::acc_t acc_t;
   constexpr int B = 64;
   if (*info != 0) return;
@@ -294,24 +314,24 @@ hipError_t launch_chol_panel(int uplo, int nr, int jb, const T *D, long lda, con
 }
 
 template <typename T>
-hipError_t launch_potf2(int uplo, int n, T *A, long lda, int info_base, int *info,
+hipError_t launch_potf2(int uplo, int n, T *A, long lda, T *inv, int info_base, int *info,
                         hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  if (n > CNB || lda < n || !A || !info) return hipErrorInvalidValue;
+  if (n > CNB || lda < n || !A || !inv || !info) return hipErrorInvalidValue;
   hipLaunchKernelGGL(potf2_kernel<T>, dim3(1), dim3(NT), 0, s, uplo == KX_LOWER, n, A, lda,
-                     info_base, info);
+                     inv, info_base, info);
   return hipGetLastError();
 }
 
 }  // namespace
 
-extern "C" hipError_t atlmx_k_dpotf2(int uplo, int n, double *A, long lda, int info_base,
-                                     int *info, hipStream_t s) {
-  return launch_potf2<double>(uplo, n, A, lda, info_base, info, s);
+extern "C" hipError_t atlmx_k_dpotf2(int uplo, int n, double *A, long lda, double *inv,
+                                     int info_base, int *info, hipStream_t s) {
+  return launch_potf2<double>(uplo, n, A, lda, inv, info_base, info, s);
 }
-extern "C" hipError_t atlmx_k_spotf2(int uplo, int n, float *A, long lda, int info_base,
-                                     int *info, hipStream_t s) {
-  return launch_potf2<float>(uplo, n, A, lda, info_base, info, s);
+extern "C" hipError_t atlmx_k_spotf2(int uplo, int n, float *A, long lda, float *inv,
+                                     int info_base, int *info, hipStream_t s) {
+  return launch_potf2<float>(uplo, n, A, lda, inv, info_base, info, s);
 }
 extern "C" hipError_t atlmx_k_dchol_panel(int uplo, int nr, int jb, const double *D, long lda,
                                           const double *inv, double *P, const int *info,

@@ -310,12 +310,13 @@ hipError_t atlmx_k_slaswp_apply(float *A, long lda, int c0, int c1, int s0,
                                 int s1, const int *plan, hipStream_t s);
 
 /* Cholesky of one n x n diagonal block (n <= 128) in place (lower or
- * upper).  On a non-positive pivot sets *info = info_base + k + 1 (if still
+ * upper), and into inv the inverses of its 64 x 64 diagonal blocks, as
+ * atlmx_k_?tri_inv lays them out.  On a non-positive pivot sets *info = info_base + k + 1 (if still
  * 0) and stops; does nothing when *info is already nonzero. */
 #define ATLMX_CHOL_NB 128
-hipError_t atlmx_k_dpotf2(int uplo, int n, double *A, long lda, int info_base,
+hipError_t atlmx_k_dpotf2(int uplo, int n, double *A, long lda, double *inv, int info_base,
                           int *info, hipStream_t s);
-hipError_t atlmx_k_spotf2(int uplo, int n, float *A, long lda, int info_base,
+hipError_t atlmx_k_spotf2(int uplo, int n, float *A, long lda, float *inv, int info_base,
                           int *info, hipStream_t s);
 /* The panel's triangular solve after a jb x jb (jb <= 128) diagonal block D
  * is factored (uplo as for potf2): nr vectors of P (Lower: the rows of the

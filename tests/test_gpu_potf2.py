@@ -1,0 +1,48 @@
+"""The Cholesky of one 128-wide diagonal block (and through it potrf): orders
+at the edges of its 32-column panels and 64-wide inverses, both triangles,
+against |A - L L^T| <= 8 (n + 1) u |L| |L|^T (Higham, Accuracy and Stability,
+Theorem 10.3; 8 for the products with the blocks' inverses, whose condition
+is below 8 here), the other triangle untouched, and the first failing minor
+at every panel and block edge."""
+import numpy as np
+import pytest
+
+import atlas_amd as X
+
+pytestmark = pytest.mark.gpu
+
+
+def _spd(rng, n):
+    B = rng.standard_normal((n, n))
+    return B @ B.T / n + np.eye(n)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("uplo", [X.Lower, X.Upper])
+@pytest.mark.parametrize("n", [1, 16, 17, 31, 32, 33, 48, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160,
+                               193, 257, 300])
+def test_potrf_block_edges(dt, uplo, n):
+    rng = np.random.default_rng(n)
+    S = _spd(rng, n).astype(dt)
+    S = np.tril(S) + np.tril(S, -1).T
+    A = np.asfortranarray(S)
+    junk = rng.standard_normal((n, n)).astype(dt)
+    keep, other = (np.tril, lambda M: np.triu(M, 1)) if uplo == X.Lower else \
+        (np.triu, lambda M: np.tril(M, -1))
+    A = np.asfortranarray(keep(A) + other(junk))
+    assert X.potrf(A, uplo) == 0
+    assert np.array_equal(other(A), other(junk))
+    L = keep(A).astype(np.float64)
+    L = L if uplo == X.Lower else L.T
+    u = np.finfo(dt).eps / 2
+    assert np.all(np.abs(S.astype(np.float64) - L @ L.T) <= 8 * (n + 1) * u * (np.abs(L) @ np.abs(L).T))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("uplo", [X.Lower, X.Upper])
+@pytest.mark.parametrize("col", [1, 16, 32, 33, 64, 65, 96, 97, 128, 129, 200])
+def test_potrf_first_failing_minor(dt, uplo, col):
+    rng = np.random.default_rng(col)
+    A = np.asfortranarray(_spd(rng, 200).astype(dt))
+    A[col - 1, col - 1] = -1
+    assert X.potrf(A, uplo) == col
