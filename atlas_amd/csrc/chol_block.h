@@ -52,20 +52,20 @@ constexpr int PLD = PB + 1;
 template <typename T> struct Rng;
 template <> struct Rng<double> {
   __device__ static double rsq(double d) { return __builtin_amdgcn_rsq(d); }
-  __device__ static bool plain(double d) { return d >= 1e-280 && d <= 1e280; }
+  __device__ static bool plain(double d) { return (d >= 1e-280) & (d <= 1e280); }
 };
 template <> struct Rng<float> {
   __device__ static float rsq(float d) { return __builtin_amdgcn_rsqf(d); }
-  __device__ static bool plain(float d) { return d >= 1e-30f && d <= 1e30f; }
+  __device__ static bool plain(float d) { return (d >= 1e-30f) & (d <= 1e30f); }
 };
 
 /* sd = sqrt(d) and ri = 1 / sd (d > 0), each within an ulp: the hardware
  * reciprocal square root and two coupled Newton steps (one in FP32), a
- * shorter chain than the library's square root and division; outside the
- * range where no step can over- or underflow, those. */
-template <typename T>
+ * shorter chain than the library's square root and division; PLAIN: d is in
+ * the range where no step can over- or underflow.  Outside it, those. */
+template <typename T, bool PLAIN>
 __device__ inline void sqrt_inv(T d, T &sd, T &ri) {
-  if (Rng<T>::plain(d)) {
+  if (PLAIN || Rng<T>::plain(d)) {
     T y = Rng<T>::rsq(d), g = d * y, h = T(0.5) * y;
 #pragma unroll
     for (int it = 0; it < (sizeof(T) == 8 ? 2 : 1); ++it) {
@@ -176,30 +176,45 @@ __device__ __forceinline__ int fresh_lane() {
  * lanes 32..63 one column each: both are the same elimination step,
  * v[c] -= v[j] L(c, j), the inverse's columns starting from the identity's.
  * Column j's entries reach all lanes by readlane.  Returns 0 or 1 + the
- * failing column; v holds the row of L or the column of the inverse. */
-template <typename T>
-__device__ __forceinline__ int block_factor(T (&v)[PB], const T *s_d) {
+ * failing column; v holds the row of L or the column of the inverse.
+ *
+ * The 32 pivots are one serial chain, and a branch at each kept the columns'
+ * updates from filling its gaps (FP64: 8.9 us a block).  They are therefore
+ * first all taken as plain ones, with no branch between the columns, and only
+ * where one was not (too small or large for the short square root, negative,
+ * NaN) is the block done again with the tests: the same arithmetic on every
+ * column before it.  6.3 us. */
+template <typename T, bool PLAIN>
+__device__ __forceinline__ int block_columns(T (&v)[PB], const T *s_d) {
   const int lane = fresh_lane();
   int fail = 0;
+  bool plain = true;
 #pragma unroll
   for (int c = 0; c < PB; ++c)
     v[c] = lane < PB ? s_d[c * PLD + lane] : (c == lane - PB ? T(1) : T(0));
 #pragma unroll
   for (int j = 0; j < PB; ++j) {
-    if (!fail) {
+    if (PLAIN || !fail) {
       const T d = bcast(v[j], j);
-      if (!(d > T(0))) {
+      if (!PLAIN && !(d > T(0))) {
         fail = j + 1;                              /* uniform: every lane saw the same d */
       } else {
+        if (PLAIN) plain = plain & Rng<T>::plain(d);
         T sd, ri;
-        sqrt_inv(d, sd, ri);
+        sqrt_inv<T, PLAIN>(d, sd, ri);
         v[j] = lane == j ? sd : v[j] * ri;
 #pragma unroll
         for (int c = j + 1; c < PB; ++c) v[c] = fma(-v[j], bcast(v[j], c), v[c]);
       }
     }
   }
-  return fail;
+  return PLAIN ? !plain : fail;
+}
+
+template <typename T>
+__device__ __forceinline__ int block_factor(T (&v)[PB], const T *s_d) {
+  if (block_columns<T, true>(v, s_d) == 0) return 0;
+  return block_columns<T, false>(v, s_d);
 }
 
 }  // namespace atlmx

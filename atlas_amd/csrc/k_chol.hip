@@ -29,34 +29,65 @@ using namespace atlmx;
  * then multiplied by the inverse.  Every second panel completes a 64x64
  * diagonal block, whose inverse the panel solve needs, [i11 0; -i22 L21 i11,
  * i22]: formed here from the two 32x32 inverses instead of by a launch of
- * its own.  L(i, k) is A[i rs + k cs], so that Upper (A = U^T U, L = U^T) is
- * the same code.  What bounds it: four times the one-wavefront factor of 32
- * columns (5 us).  128 columns, FP64: 87 us for one barrier-separated step
- * per column, and 15 for the inverses' launch, -> 71 us for both. */
+ * its own.  The ten 32x32 tiles of the triangle stay in LDS from one load to
+ * one store, so that no step of the chain waits for memory.  L(i, k) is
+ * A[i rs + k cs], so that Upper (A = U^T U, L = U^T) is the same code.  What
+ * bounds it: four times the one-wavefront factor of 32 columns.  128
+ * columns, FP64: 87 us for one barrier-separated step per column, and 15 for
+ * the inverses' launch; 71 for both with the tiles in memory; 46 so: 3 for
+ * the load, 6.3 for each panel's factor, 2 to 4 for its products, 4 for the
+ * store. */
+constexpr int TBLK = PB * PLD;
+constexpr int NTILE = (CNB / PB) * (CNB / PB + 1) / 2;
+
 template <typename T>
 __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long lda, T *inv,
                                                    int info_base, int *info) {
   typedef TMfma<T> MF;
   typedef typename MF::acc_t acc_t;
-  constexpr int BLK = PB * PLD, IB = 64;
+  constexpr int IB = 64;
   if (*info != 0) return;
-  __shared__ T s_blk[4 * BLK], s_i[2][BLK];
+  __shared__ T s_l[NTILE * TBLK], s_blk[4 * TBLK], s_i[2][TBLK];
   __shared__ int s_ready, s_fail;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lk = lane >> 4;
   const long rs = lower ? 1 : lda, cs = lower ? lda : 1;
+  const int nt = (n + PB - 1) / PB;
+  auto tile = [&](int i, int j) { return s_l + (i * (i + 1) / 2 + j) * TBLK; };
   if (tid == 0) s_ready = s_fail = 0;
+  /* row and column within a tile: neighbouring threads at neighbouring addresses */
+  const int f = tid % PB, g = tid / PB;
+  T in[NTILE][PB * PB / NT];                       /* every load before the first use */
+#pragma unroll
+  for (int i = 0, q = 0; i < CNB / PB; ++i)
+#pragma unroll
+    for (int j = 0; j <= i; ++j, ++q)
+#pragma unroll
+      for (int h = 0; h < PB * PB / NT; ++h) {
+        const int r = lower ? f : g + h * (NT / PB), c = lower ? g + h * (NT / PB) : f;
+        const int ar = i * PB + r, ac = j * PB + c;
+        in[q][h] = ar == ac ? T(1) : T(0);         /* beyond the matrix: the identity */
+        if (ar < n && ac <= ar) in[q][h] = A[(long)ar * rs + (long)ac * cs];
+      }
+#pragma unroll
+  for (int q = 0; q < NTILE; ++q)
+#pragma unroll
+    for (int h = 0; h < PB * PB / NT; ++h) {
+      const int r = lower ? f : g + h * (NT / PB), c = lower ? g + h * (NT / PB) : f;
+      s_l[q * TBLK + c * PLD + r] = in[q][h];
+    }
   __syncthreads();
-  for (int k = 0; k < n; k += PB) {
-    const int kb = min(PB, n - k), p = k / PB;
-    const T *yp[2] = {A + (long)min(k + li, n - 1) * rs, A + (long)min(k + 16 + li, n - 1) * rs};
-    {
+  for (int p = 0; p < nt; ++p) {
+    if (p) {
       acc_t acc[2][2];
       zero_tile(acc);
-      const int w = k / 4;                         /* a multiple of 8 */
-      panel_acc<T, 2, 2, 2>(acc, yp, cs, yp, cs, wave * w, wave * w + w);
-      T *sp = s_blk + wave * BLK;
+      for (int t = 0; t < p; ++t) {                /* 8 of each tile's columns */
+        const T *y = tile(p, t) + li;
+        const T *yp[2] = {y, y + 16};
+        panel_acc<T, 2, 2, 2>(acc, yp, PLD, yp, PLD, 8 * wave, 8 * wave + 8);
+      }
+      T *sp = s_blk + wave * TBLK;
 #pragma unroll
       for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -64,54 +95,51 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
 #pragma unroll
           for (int e = 0; e < 4; ++e)
             sp[(16 * c + MF::drow(lane, e)) * PLD + 16 * r + li] = acc[c][r][e];
+      __syncthreads();
+#pragma unroll
+      for (int h = 0; h < PB; h += NT / PB) {
+        const int r = f, c = g + h;
+        T *o = tile(p, p) + c * PLD + r;
+        const T *q = s_blk + c * PLD + r;
+        if (r >= c && p * PB + r < n) *o -= (q[0] + q[TBLK]) + (q[2 * TBLK] + q[3 * TBLK]);
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    for (int e = tid; e < PB * PB; e += NT) {
-      const int c = e / PB, r = e % PB;
-      T *o = s_blk + c * PLD + r;
-      T v = r == c ? T(1) : T(0);                  /* beyond the matrix: the identity */
-      if (r < kb && c < kb && r >= c)
-        v = A[(long)(k + r) * rs + (long)(k + c) * cs] -
-            ((o[0] + o[BLK]) + (o[2 * BLK] + o[3 * BLK]));
-      *o = v;
-    }
-    __syncthreads();
-    const int nt = (n - k + PB - 1) / PB;
     if (wave == 0) {
       T v[PB];
-      const int fail = block_factor(v, s_blk);
+      T *d = tile(p, p);
+      const int fail = block_factor(v, d);
       const int ln = fresh_lane();
       if (ln < PB) {
         /* on failure the columns before the failing one, as far as they are */
         const int nc = fail ? fail - 1 : PB;
 #pragma unroll
         for (int c = 0; c < PB; ++c)
-          if (c <= ln && c < nc && ln < kb) A[(long)(k + ln) * rs + (long)(k + c) * cs] = v[c];
+          if (c <= ln && c < nc) d[c * PLD + ln] = v[c];
       } else {
 #pragma unroll
         for (int c = 0; c < PB; ++c) s_i[p & 1][(ln - PB) * PLD + c] = v[c];
       }
       if (ln == 0) {
-        if (fail) s_fail = k + fail;
+        if (fail) s_fail = p * PB + fail;
         __hip_atomic_store(&s_ready, p + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
-    } else if (wave < nt) {                        /* row tile `wave`; then kb == PB */
-      const int ra = k + wave * PB + li, rb = ra + 16;
-      const T *xp[2] = {A + (long)min(ra, n - 1) * rs, A + (long)min(rb, n - 1) * rs};
+    } else if (p + wave < nt) {                    /* row tile p + wave */
       acc_t acc[2][2], w[2][2];
+      T *x = tile(p + wave, p);
       zero_tile(acc);
+      for (int t = 0; t < p; ++t) {
+        const T *y = tile(p, t) + li, *z = tile(p + wave, t) + li;
+        const T *yp[2] = {y, y + 16}, *xp[2] = {z, z + 16};
+        panel_acc<T, 2, 2, 2>(acc, yp, PLD, xp, PLD, 0, PB);
+      }
 #pragma unroll
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int r = 0; r < 2; ++r)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            w[c][r][e] = xp[r][(long)(k + 16 * c + MF::drow(lane, e)) * cs];
-      panel_acc<T, 2, 2, 4>(acc, yp, cs, xp, cs, 0, k);
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int r = 0; r < 2; ++r) w[c][r] -= acc[c][r];
+            w[c][r][e] = x[(16 * c + MF::drow(lane, e)) * PLD + 16 * r + li] - acc[c][r][e];
       while (__hip_atomic_load(&s_ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < p + 1)
         __builtin_amdgcn_s_sleep(1);
       if (!s_fail) {
@@ -119,26 +147,23 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            T *col = A + (long)(k + 16 * c + MF::drow(lane, e)) * cs;
-            if (ra < n) col[(long)ra * rs] = w[c][0][e];
-            if (rb < n) col[(long)rb * rs] = w[c][1][e];
-          }
+          for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              x[(16 * c + MF::drow(lane, e)) * PLD + 16 * r + li] = w[c][r][e];
       }
     }
     __syncthreads();
-    if (s_fail) {
-      if (tid == 0) atomicCAS(info, 0, info_base + s_fail);
-      return;
-    }
-    if (!(p & 1) && k + PB < n) continue;
+    if (s_fail) break;
+    if (!(p & 1) && p + 1 < nt) continue;
     /* ---- inverse of the 64x64 block b: wavefront w forms columns 16 (w & 1)
      * of L21 i11 and from them its 16x16 tile of X21 ---- */
-    const int b = p / 2, r0 = IB * b + PB, two = p & 1;
+    const int b = p / 2, two = p & 1;
     T *out = inv + (size_t)b * IB * IB;            /* inv(L)(r, c), transposed for Upper */
     auto put = [&](int r, int c, T v) { out[lower ? c * IB + r : r * IB + c] = v; };
-    for (int e = tid; e < PB * PB; e += NT) {
-      const int c = e / PB, r = e % PB;
+#pragma unroll
+    for (int h = 0; h < PB; h += NT / PB) {
+      const int r = lower ? f : g + h, c = lower ? g + h : f;
       put(r, c, s_i[0][c * PLD + r]);
       put(PB + r, PB + c, two ? s_i[1][c * PLD + r] : (r == c ? T(1) : T(0)));
       put(r, PB + c, T(0));
@@ -146,18 +171,15 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
     }
     if (two) {
       const int jb = 16 * (wave & 1), ib = 16 * (wave >> 1);
+      const T *l21 = tile(2 * b + 1, 2 * b);
       acc_t t[2], x = acc_t{0, 0, 0, 0};
 #pragma unroll
       for (int r = 0; r < 2; ++r) {
-        const int row = r0 + 16 * r + li;
-        T l[8];
-#pragma unroll
-        for (int s = 0; s < 8; ++s)
-          l[s] = row < n ? A[(long)row * rs + (long)(IB * b + 4 * s + lk) * cs] : T(0);
         t[r] = acc_t{0, 0, 0, 0};
 #pragma unroll
         for (int s = 0; s < 8; ++s)
-          t[r] = MF::mma(l[s], s_i[0][(jb + li) * PLD + 4 * s + lk], t[r]);
+          t[r] = MF::mma(l21[(4 * s + lk) * PLD + 16 * r + li], s_i[0][(jb + li) * PLD + 4 * s + lk],
+                         t[r]);
       }
 #pragma unroll
       for (int r = 0; r < 2; ++r)
@@ -168,6 +190,15 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
       for (int e = 0; e < 4; ++e) put(PB + ib + MF::drow(lane, e), jb + li, -x[e]);
     }
   }
+  for (int i = 0; i < nt; ++i)
+    for (int j = 0; j <= i; ++j)
+#pragma unroll
+      for (int h = 0; h < PB; h += NT / PB) {
+        const int r = lower ? f : g + h, c = lower ? g + h : f;
+        const int ar = i * PB + r, ac = j * PB + c;
+        if (ar < n && ac <= ar) A[(long)ar * rs + (long)ac * cs] = tile(i, j)[c * PLD + r];
+      }
+  if (s_fail && tid == 0) atomicCAS(info, 0, info_base + s_fail);
 }
 
 /* The panel's triangular solve after the diagonal block (jb <= 128 rows)

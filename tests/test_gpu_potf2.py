@@ -46,3 +46,21 @@ def test_potrf_first_failing_minor(dt, uplo, col):
     A = np.asfortranarray(_spd(rng, 200).astype(dt))
     A[col - 1, col - 1] = -1
     assert X.potrf(A, uplo) == col
+
+
+@pytest.mark.parametrize("dt,scale", [(np.float64, 1e-290), (np.float64, 1e290),
+                                      (np.float32, 1e-33), (np.float32, 1e33)])
+@pytest.mark.parametrize("uplo", [X.Lower, X.Upper])
+def test_potrf_pivots_outside_the_short_square_root(dt, scale, uplo):
+    """Pivots where the reciprocal square root's steps would over- or
+    underflow: the block is done again with the library's square root."""
+    n = 150
+    S = (_spd(np.random.default_rng(5), n) * scale).astype(dt)
+    A = np.asfortranarray(np.tril(S) if uplo == X.Lower else np.triu(np.tril(S).T))
+    assert X.potrf(A, uplo) == 0
+    L = np.tril(A).astype(np.float64) if uplo == X.Lower else np.triu(A).T.astype(np.float64)
+    S = np.tril(S).astype(np.float64)
+    u = np.finfo(dt).eps / 2
+    E = np.abs(S / scale - np.tril((L / np.sqrt(scale)) @ (L / np.sqrt(scale)).T))
+    La = np.abs(L / np.sqrt(scale))
+    assert np.all(E <= 8 * (n + 1) * u * (La @ La.T))
