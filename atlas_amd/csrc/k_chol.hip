@@ -205,7 +205,7 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
  * is factored: every panel vector v (a row of A21 for Lower, a column of
  * A12 for Upper) becomes y with L y^T = v^T, L the block's lower factor
  * (Lower: L11; Upper: U11^T).  With L split into 64-row blocks, L = [L00 0;
- * L10 L11'] and the inverted diagonal blocks from atlmx_k_?tri_inv:
+ * L10 L11'] and the inverted diagonal blocks from potf2_kernel:
  *   y0 = v0 inv(L00)^T,   y1 = (v1 - y0 L10^T) inv(L11')^T
  * -- the two-block TRSM ATLAS's Cholesky makes (ATL_potrfL.c:236-246), as
  * three 64-wide products in one launch.  A workgroup takes 64 vectors,

@@ -311,8 +311,9 @@ hipError_t atlmx_k_slaswp_apply(float *A, long lda, int c0, int c1, int s0,
 
 /* Cholesky of one n x n diagonal block (n <= 128) in place (lower or
  * upper), and into inv the inverses of its 64 x 64 diagonal blocks, as
- * atlmx_k_?tri_inv lays them out.  On a non-positive pivot sets *info = info_base + k + 1 (if still
- * 0) and stops; does nothing when *info is already nonzero. */
+ * atlmx_k_?tri_inv lays them out.  On a non-positive pivot sets *info =
+ * info_base + k + 1 (if still 0) and stops; does nothing when *info is
+ * already nonzero. */
 #define ATLMX_CHOL_NB 128
 hipError_t atlmx_k_dpotf2(int uplo, int n, double *A, long lda, double *inv, int info_base,
                           int *info, hipStream_t s);
@@ -322,7 +323,7 @@ hipError_t atlmx_k_spotf2(int uplo, int n, float *A, long lda, float *inv, int i
  * is factored (uplo as for potf2): nr vectors of P (Lower: the rows of the
  * nr x jb block below D; Upper: the columns of the jb x nr block right of
  * it) are solved in place against D's factor, using inv = the inverted
- * 64 x 64 diagonal blocks of D from atlmx_k_?tri_inv.  Does nothing when
+ * 64 x 64 diagonal blocks of D from atlmx_k_?potf2.  Does nothing when
  * *info is nonzero. */
 hipError_t atlmx_k_dchol_panel(int uplo, int nr, int jb, const double *D, long lda,
                                const double *inv, double *P, const int *info, hipStream_t s);
