@@ -43,16 +43,14 @@ constexpr int MAXR = ATLMX_BATCH_MAXRHS;
 /* Trailing updates on the matrix cores, one 64 x 64 tile per wavefront    */
 /* ---------------------------------------------------------------------- */
 /* C(tile) -= X Y^T for a 64 x 64 tile by one wavefront, K <= KMAX: X(r, k)
- * = X[r + k ldx] (rows r0 of the tile), Y(c, k) = Y[c*ycs + k*yks] (NT:
+ * = X[r + k ldx], Y(c, k) = Y[c*ycs + k*yks] (NT:
  * ycs = 1, yks = ld; NN with Y = U^T: ycs = ld, yks = 1).  Operands go from
  * memory straight into the MFMA lanes (lane l: row or column l&15 of a
  * 16-block, k = 4s + (l>>4)), no LDS and no barrier, so the wavefronts of a
- * workgroup work on different tiles at once.  lower_only: only r0 + r >=
- * c0 + c is written. */
+ * workgroup work on different tiles at once. */
 template <typename T, int KMAX>
 __device__ void wave_tile_update(T *C, long ldc, const T *X, long ldx, const T *Y, long ycs,
-                                 long yks, int K, int mr, int mc, bool lower_only, int r0,
-                                 int c0) {
+                                 long yks, int K, int mr, int mc) {
   typedef TMfma<T> MF;
   typedef typename MF::acc_t acc_t;
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
@@ -88,8 +86,7 @@ __device__ void wave_tile_update(T *C, long ldc, const T *X, long ldx, const T *
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int rr = 16 * i + MF::drow(lane, r), cc = 16 * j + li;
-        if (rr < mr && cc < mc && (!lower_only || r0 + rr >= c0 + cc))
-          C[(size_t)cc * ldc + rr] -= acc[i][j][r];
+        if (rr < mr && cc < mc) C[(size_t)cc * ldc + rr] -= acc[i][j][r];
       }
 }
 
@@ -572,7 +569,7 @@ __device__ void wg_gesv(int n, T *A, long lda, int *ipiv, int nrhs, T *B, long l
       const int r0 = m0 + ti * TS, c0 = m0 + tj * TS;
       wave_tile_update<T, NB>(A + (size_t)c0 * lda + r0, lda, A + (size_t)k * lda + r0, lda,
                               A + (size_t)c0 * lda + k, lda, 1, kb, min(TS, n - r0),
-                              min(TS, n - c0), false, r0, c0);
+                              min(TS, n - c0));
     }
   }
   if (tid == 0) *info = first0;
