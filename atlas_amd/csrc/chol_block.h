@@ -131,7 +131,11 @@ __device__ __forceinline__ void zero_tile(acc_t (&t)[NC][RJ]) {
 }
 
 /* w <- w inv^T for a tile held as accumulators: out[c][r] = the sum over l of
- * inv(c, l) w(l, r), the inverse (lower) at s_inv[l PLD + c] in LDS */
+ * inv(c, l) w(l, r), the inverse (lower) at s_inv[l PLD + c] in LDS.  The
+ * products run over the inverse's zeros too, so where a sum is not finite
+ * all are formed again over l <= c alone: an infinity or a NaN in column l
+ * of the tile's row stays in that row, from column l on, as in a
+ * substitution. */
 template <typename T, int RJ>
 __device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][RJ],
                                                const T *s_inv) {
@@ -150,6 +154,37 @@ __device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][
         for (int r = 0; r < RJ; ++r) out[c][r] = TMfma<T>::mma(a, w[l][r][e], out[c][r]);
       }
     }
+  bool odd = false;
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int r = 0; r < RJ; ++r)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) odd |= !__builtin_isfinite(out[c][r][e]);
+  if (__ballot(odd)) {
+    zero_tile(out);
+#pragma unroll
+    for (int l = 0; l < 2; ++l)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll 1
+        for (int g = 0; g < 4; ++g) {              /* lane group g holds w(row, .) */
+          const int row = 16 * l + TMfma<T>::drow(16 * g, e);
+          T x[RJ];
+#pragma unroll
+          for (int r = 0; r < RJ; ++r) x[r] = __shfl(w[l][r][e], 16 * g + li);
+#pragma unroll
+          for (int c = l; c < 2; ++c)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+              const int col = 16 * c + TMfma<T>::drow(lane, f);
+              const T a = s_inv[row * PLD + col];
+#pragma unroll
+              for (int r = 0; r < RJ; ++r)
+                out[c][r][f] = col >= row ? fma(a, x[r], out[c][r][f]) : out[c][r][f];
+            }
+        }
+  }
 #pragma unroll
   for (int c = 0; c < 2; ++c)
 #pragma unroll

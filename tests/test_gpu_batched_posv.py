@@ -75,3 +75,37 @@ def test_posv_largest_order():
     X.use_torch_stream()
     n = X.lib().atlmx_batch_max_order(0, 1)
     _check(torch, [n, 70], np.float64, 8)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_posv_nonfinite_entry_stays_right_of_its_column(dt, bad):
+    """A(70, c) not finite: the factorization stops at row 70, and that row's
+    entries left of column c are what they are without it, as a substitution
+    leaves them; every other row above the failing panel too."""
+    import torch
+    X.use_torch_stream()
+    n, r = 100, 70
+    cols = [0, 1, 7, 14, 15, 16, 17, 30, 31, 33, 47, 50, 63]
+    rng = np.random.default_rng(11)
+    S = _spd(rng, n).astype(dt)
+    L = np.linalg.cholesky(np.tril(S).astype(np.float64) + np.tril(S, -1).T.astype(np.float64))
+    As = []
+    for c in cols:
+        A = np.tril(S)
+        A[r, c] = bad
+        As.append(torch.tensor(np.ascontiguousarray(A.T), device="cuda"))
+    info = torch.full((len(cols),), -7, dtype=torch.int32, device="cuda")
+    with X.posv_batch(As, [], info) as plan:
+        plan.run()
+        torch.cuda.synchronize()
+    assert info.cpu().tolist() == [r + 1] * len(cols)
+    # |L - fl(L)| <= c n u kappa(S) |L| in norm; kappa(S) < 8 here
+    tol = 64 * n * np.finfo(dt).eps
+    for c, A in zip(cols, As):
+        F = A.cpu().numpy().T.astype(np.float64)
+        assert np.abs(F[r, :c] - L[r, :c]).max(initial=0) <= tol, c
+        assert not np.isfinite(F[r, c]), c
+        others = [i for i in range(64, n) if i != r]
+        assert np.abs(np.tril(F - L)[:64, :64]).max() <= tol, c
+        assert np.abs((F - L)[others, :64]).max() <= tol, c

@@ -64,3 +64,25 @@ def test_potrf_pivots_outside_the_short_square_root(dt, scale, uplo):
     E = np.abs(S / scale - np.tril((L / np.sqrt(scale)) @ (L / np.sqrt(scale)).T))
     La = np.abs(L / np.sqrt(scale))
     assert np.all(E <= 8 * (n + 1) * u * (La @ La.T))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("uplo", [X.Lower, X.Upper])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("c", [0, 1, 14, 15, 16, 17, 31, 33, 50, 63])
+def test_potrf_nonfinite_entry_stays_right_of_its_column(dt, uplo, bad, c):
+    """A(70, c) not finite: info names row 70, and that row's entries left of
+    column c are what they are without it."""
+    n, r = 100, 70
+    S = _spd(np.random.default_rng(11), n).astype(dt)
+    S = np.tril(S) + np.tril(S, -1).T
+    L = np.linalg.cholesky(S.astype(np.float64))
+    A = np.asfortranarray(S)
+    A[(r, c) if uplo == X.Lower else (c, r)] = bad
+    assert X.potrf(A, uplo) == r + 1
+    F = (A if uplo == X.Lower else A.T).astype(np.float64)
+    tol = 64 * n * np.finfo(dt).eps          # c n u kappa(S) |L|, kappa(S) < 8
+    assert np.abs(F[r, :c] - L[r, :c]).max(initial=0) <= tol
+    others = [i for i in range(64, n) if i != r]
+    assert np.abs(np.tril(F - L)[:64, :64]).max() <= tol
+    assert np.abs((F - L)[others, :64]).max() <= tol
