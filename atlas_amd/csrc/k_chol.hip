@@ -111,7 +111,7 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
       const int fail = block_factor(v, d);
       const int ln = fresh_lane();
       if (ln < PB) {
-        /* on failure the columns before the failing one, as far as they are */
+        /* on failure the columns before the failing one; so below */
         const int nc = fail ? fail - 1 : PB;
 #pragma unroll
         for (int c = 0; c < PB; ++c)
@@ -142,16 +142,17 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
             w[c][r][e] = x[(16 * c + MF::drow(lane, e)) * PLD + 16 * r + li] - acc[c][r][e];
       while (__hip_atomic_load(&s_ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < p + 1)
         __builtin_amdgcn_s_sleep(1);
-      if (!s_fail) {
-        tile_times_inv<T, 2>(w, s_i[p & 1]);
+      tile_times_inv<T, 2>(w, s_i[p & 1]);
+      const int nc = s_fail ? s_fail - 1 - p * PB : PB;
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int r = 0; r < 2; ++r)
+        for (int e = 0; e < 4; ++e) {
+          const int col = 16 * c + MF::drow(lane, e);
+          if (col < nc)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              x[(16 * c + MF::drow(lane, e)) * PLD + 16 * r + li] = w[c][r][e];
-      }
+            for (int r = 0; r < 2; ++r) x[col * PLD + 16 * r + li] = w[c][r][e];
+        }
     }
     __syncthreads();
     if (s_fail) break;
@@ -190,13 +191,16 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
       for (int e = 0; e < 4; ++e) put(PB + ib + MF::drow(lane, e), jb + li, -x[e]);
     }
   }
+  /* on failure the columns before the failing one are stored, factored in
+   * every row of the block; the others stay as they came */
+  const int done = s_fail ? s_fail - 1 : n;
   for (int i = 0; i < nt; ++i)
     for (int j = 0; j <= i; ++j)
 #pragma unroll
       for (int h = 0; h < PB; h += NT / PB) {
         const int r = lower ? f : g + h, c = lower ? g + h : f;
         const int ar = i * PB + r, ac = j * PB + c;
-        if (ar < n && ac <= ar) A[(long)ar * rs + (long)ac * cs] = tile(i, j)[c * PLD + r];
+        if (ar < n && ac <= ar && ac < done) A[(long)ar * rs + (long)ac * cs] = tile(i, j)[c * PLD + r];
       }
   if (s_fail && tid == 0) atomicCAS(info, 0, info_base + s_fail);
 }

@@ -86,3 +86,22 @@ def test_potrf_nonfinite_entry_stays_right_of_its_column(dt, uplo, bad, c):
     others = [i for i in range(64, n) if i != r]
     assert np.abs(np.tril(F - L)[:64, :64]).max() <= tol
     assert np.abs((F - L)[others, :64]).max() <= tol
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("uplo", [X.Lower, X.Upper])
+@pytest.mark.parametrize("n,col", [(20, 9), (100, 1), (100, 17), (100, 33), (100, 75), (128, 128)])
+def test_potrf_failure_leaves_the_columns_before_it_factored(dt, uplo, n, col):
+    """Within a block of 128: the columns before the failing one hold the
+    factor in every row, the failing one and those after it are as given."""
+    S = _spd(np.random.default_rng(col), n).astype(dt)
+    S = np.tril(S) + np.tril(S, -1).T
+    L = np.linalg.cholesky(S.astype(np.float64))
+    S[col - 1, col - 1] = -1
+    A = np.asfortranarray(S)
+    assert X.potrf(A, uplo) == col
+    F = A if uplo == X.Lower else A.T
+    assert np.array_equal(F[:, col - 1:], S[:, col - 1:])
+    # c n u kappa(S) |L|, kappa(S) < 8
+    assert np.abs(np.tril(F.astype(np.float64) - L)[:, :col - 1]).max(initial=0) <= \
+        64 * n * np.finfo(dt).eps
