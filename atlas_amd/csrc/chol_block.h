@@ -130,6 +130,21 @@ __device__ __forceinline__ void zero_tile(acc_t (&t)[NC][RJ]) {
     for (int r = 0; r < RJ; ++r) t[c][r] = acc_t{0, 0, 0, 0};
 }
 
+/* A scalar, or this lane's number, that the compiler takes for a new value
+ * here: without it the products of lda with dozens of column numbers, and
+ * one 64-bit mask for every lane compare, are computed ahead of the panel
+ * loop and spilled across it (the Cholesky: 252 scalar spills). */
+__device__ __forceinline__ long fresh(long v) {
+  int lo = __builtin_amdgcn_readfirstlane((int)v);   /* a leading dimension: 31 bits */
+  asm volatile("" : "+s"(lo));
+  return lo;
+}
+__device__ __forceinline__ int fresh_lane() {
+  int l = threadIdx.x & 63;
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
 /* w <- w inv^T for a tile held as accumulators: out[c][r] = the sum over l of
  * inv(c, l) w(l, r), the inverse (lower) at s_inv[l PLD + c] in LDS.  The
  * products run over the inverse's zeros too, so where a sum is not finite
@@ -162,6 +177,7 @@ __device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][
 #pragma unroll
       for (int e = 0; e < 4; ++e) odd |= !__builtin_isfinite(out[c][r][e]);
   if (__ballot(odd)) {
+    const int ln = fresh_lane();
     zero_tile(out);
 #pragma unroll
     for (int l = 0; l < 2; ++l)
@@ -172,12 +188,12 @@ __device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][
           const int row = 16 * l + TMfma<T>::drow(16 * g, e);
           T x[RJ];
 #pragma unroll
-          for (int r = 0; r < RJ; ++r) x[r] = __shfl(w[l][r][e], 16 * g + li);
+          for (int r = 0; r < RJ; ++r) x[r] = __shfl(w[l][r][e], 16 * g + (ln & 15));
 #pragma unroll
           for (int c = l; c < 2; ++c)
 #pragma unroll
             for (int f = 0; f < 4; ++f) {
-              const int col = 16 * c + TMfma<T>::drow(lane, f);
+              const int col = 16 * c + TMfma<T>::drow(ln, f);
               const T a = s_inv[row * PLD + col];
 #pragma unroll
               for (int r = 0; r < RJ; ++r)
@@ -191,44 +207,40 @@ __device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][
     for (int r = 0; r < RJ; ++r) w[c][r] = out[c][r];
 }
 
-/* A scalar, or this lane's number, that the compiler takes for a new value
- * here: without it the products of lda with dozens of column numbers, and
- * one 64-bit mask for every lane compare, are computed ahead of the panel
- * loop and spilled across it (the Cholesky: 252 scalar spills). */
-__device__ __forceinline__ long fresh(long v) {
-  int lo = __builtin_amdgcn_readfirstlane((int)v);   /* a leading dimension: 31 bits */
-  asm volatile("" : "+s"(lo));
-  return lo;
-}
-__device__ __forceinline__ int fresh_lane() {
-  int l = threadIdx.x & 63;
-  asm volatile("" : "+v"(l));
-  return l;
-}
-
 /* Wavefront 0: the Cholesky factor of the 32 x 32 block at s_d[c PLD + r]
- * (identity beyond the matrix), lanes 0..31 one row each, and its inverse,
- * lanes 32..63 one column each: both are the same elimination step,
+ * (identity beyond the matrix: column nb), lanes 0..31 one row each, and its
+ * inverse, lanes 32..63 one column each: both are the same elimination step,
  * v[c] -= v[j] L(c, j), the inverse's columns starting from the identity's.
  * Column j's entries reach all lanes by readlane.  Returns 0 or 1 + the
  * failing column; v holds the row of L or the column of the inverse.
  *
+ * The columns are taken in groups (GRP0, then GRP wide).  A group's entries
+ * gather the earlier columns' products on their own and are added to the
+ * matrix's when the group begins: subtracted from them one by one, every
+ * product rounds at the entry's size, 1.4 times the factor's error (FP32,
+ * order 32: 1.03e-7; by groups 0.72e-7).  Groups beyond the matrix are left out.
+ *
  * The 32 pivots are one serial chain, and a branch at each kept the columns'
  * updates from filling its gaps (FP64: 8.9 us a block).  They are therefore
- * first all taken as plain ones, with no branch between the columns, and only
- * where one was not (too small or large for the short square root, negative,
- * NaN) is the block done again with the tests: the same arithmetic on every
- * column before it.  6.3 us. */
-template <typename T, bool PLAIN>
-__device__ __forceinline__ int block_columns(T (&v)[PB], const T *s_d) {
+ * first all taken as plain ones, with no branch between the columns of a
+ * group, and only where one was not (too small or large for the short square
+ * root, negative, NaN) is the block done again with the tests: the same
+ * arithmetic on every column before it.  6.3 us. */
+constexpr int GRP0 = 4, GRP = 8;
+template <typename T, bool PLAIN, int G0, int W>
+__device__ __forceinline__ void block_group(T (&v)[PB], const T *s_d, int nb, int &fail,
+                                            bool &plain) {
+  if (G0 >= nb || (!PLAIN && fail)) return;        /* uniform */
   const int lane = fresh_lane();
-  int fail = 0;
-  bool plain = true;
+  if (G0 > 0) {
 #pragma unroll
-  for (int c = 0; c < PB; ++c)
-    v[c] = lane < PB ? s_d[c * PLD + lane] : (c == lane - PB ? T(1) : T(0));
+    for (int c = G0; c < G0 + W; ++c) {
+      const T d = s_d[c * PLD + (lane & (PB - 1))];
+      v[c] += lane < PB ? d : T(0);
+    }
+  }
 #pragma unroll
-  for (int j = 0; j < PB; ++j) {
+  for (int j = G0; j < G0 + W; ++j) {
     if (PLAIN || !fail) {
       const T d = bcast(v[j], j);
       if (!PLAIN && !(d > T(0))) {
@@ -243,13 +255,30 @@ __device__ __forceinline__ int block_columns(T (&v)[PB], const T *s_d) {
       }
     }
   }
+}
+
+template <typename T, bool PLAIN>
+__device__ __forceinline__ int block_columns(T (&v)[PB], const T *s_d, int nb) {
+  const int lane = fresh_lane();
+  int fail = 0;
+  bool plain = true;
+#pragma unroll
+  for (int c = 0; c < PB; ++c) {
+    v[c] = c == lane - PB ? T(1) : T(0);
+    if (c < GRP0 && lane < PB) v[c] = s_d[c * PLD + lane];
+  }
+  block_group<T, PLAIN, 0, GRP0>(v, s_d, nb, fail, plain);
+  block_group<T, PLAIN, GRP0, GRP - GRP0>(v, s_d, nb, fail, plain);
+  block_group<T, PLAIN, GRP, GRP>(v, s_d, nb, fail, plain);
+  block_group<T, PLAIN, 2 * GRP, GRP>(v, s_d, nb, fail, plain);
+  block_group<T, PLAIN, 3 * GRP, GRP>(v, s_d, nb, fail, plain);
   return PLAIN ? !plain : fail;
 }
 
 template <typename T>
-__device__ __forceinline__ int block_factor(T (&v)[PB], const T *s_d) {
-  if (block_columns<T, true>(v, s_d) == 0) return 0;
-  return block_columns<T, false>(v, s_d);
+__device__ __forceinline__ int block_factor(T (&v)[PB], const T *s_d, int nb) {
+  if (block_columns<T, true>(v, s_d, nb) == 0) return 0;
+  return block_columns<T, false>(v, s_d, nb);
 }
 
 }  // namespace atlmx

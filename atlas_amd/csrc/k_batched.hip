@@ -311,7 +311,7 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
 
     if (wave == 0) {
       T v[PB];
-      const int fail = block_factor(v, s_d);
+      const int fail = block_factor(v, s_d, kb);
       const long lda = fresh(lda0);
       const int ln = fresh_lane();
       if (ln < PB) {

@@ -108,7 +108,7 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
     if (wave == 0) {
       T v[PB];
       T *d = tile(p, p);
-      const int fail = block_factor(v, d);
+      const int fail = block_factor(v, d, min(PB, n - p * PB));
       const int ln = fresh_lane();
       if (ln < PB) {
         /* on failure the columns before the failing one; so below */

@@ -109,3 +109,46 @@ def test_posv_nonfinite_entry_stays_right_of_its_column(dt, bad):
         others = [i for i in range(64, n) if i != r]
         assert np.abs(np.tril(F - L)[:64, :64]).max() <= tol, c
         assert np.abs((F - L)[others, :64]).max() <= tol, c
+
+
+def _cholesky_by_16(A):
+    """batch of FP32 matrices: right-looking, 16 columns at a time, divisions
+    and substitutions, every operation rounded (products fused)"""
+    f = np.float32
+    fma = lambda a, b, c: (a.astype(np.float64) * b + c).astype(f)     # noqa: E731
+    A = np.tril(A)
+    n = A.shape[1]
+    for k in range(0, n, 16):
+        e = min(n, k + 16)
+        for j in range(k, e):
+            A[:, j, j] = np.sqrt(A[:, j, j])
+            A[:, j + 1:, j] /= A[:, j, j, None]
+            A[:, j + 1:, j + 1:e] = fma(-A[:, j + 1:, j, None], A[:, None, j + 1:e, j],
+                                        A[:, j + 1:, j + 1:e])
+        S = np.zeros_like(A[:, e:, e:])
+        for j in range(k, e):
+            S = fma(A[:, e:, j, None], A[:, None, e:, j], S)
+        A[:, e:, e:] -= S
+    return np.tril(A)
+
+
+@pytest.mark.parametrize("n,count", [(8, 2000), (20, 1000), (32, 1000), (64, 300), (100, 200)])
+def test_posv_rounding_no_larger_than_by_substitution(n, count):
+    """The mean error of the FP32 factors over a batch against that of the
+    same batch by divisions and substitutions; 2% for the samples' spread."""
+    import torch
+    X.use_torch_stream()
+    rng = np.random.default_rng(n)
+    A = rng.uniform(-1, 1, (count, n, n))
+    A = (A @ A.transpose(0, 2, 1) / n + 0.05 * np.eye(n)).astype(np.float32)
+    A = np.tril(A) + np.tril(A, -1).transpose(0, 2, 1)
+    L = np.linalg.cholesky(A.astype(np.float64))
+    dev = torch.tensor(A, device="cuda")
+    info = torch.zeros(count, dtype=torch.int32, device="cuda")
+    with X.posv_batch(list(dev), [], info) as plan:
+        plan.run()
+        torch.cuda.synchronize()
+    assert not info.any()
+    err = lambda F: (np.linalg.norm(F - L, axis=(1, 2)) / np.linalg.norm(L, axis=(1, 2))).mean()  # noqa: E731
+    F = np.tril(dev.cpu().numpy().transpose(0, 2, 1)).astype(np.float64)
+    assert err(F) <= 1.02 * err(_cholesky_by_16(A).astype(np.float64))
