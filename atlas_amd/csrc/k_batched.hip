@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 #include <float.h>
 #include <math.h>
+#include <type_traits>
 #include "kernels.h"
 #include "lu_panel.h"
 #include "chol_block.h"
@@ -234,6 +235,15 @@ __device__ void wg_trsv(int n, int nrhs, const T *A, long lda, bool lower, bool 
   __syncthreads();
 }
 
+/* g / d from rd = 1 / d, d and rd both normal numbers: the product and one
+ * correction round like the division (the product alone: 3% on a small
+ * solve's error), in a chain half as long */
+template <typename T>
+__device__ __forceinline__ T quotient(T g, T d, T rd) {
+  const T q = g * rd, c = fma(fma(-q, d, g), rd, q);
+  return __builtin_isfinite(c) ? c : q;
+}
+
 /* ---------------------------------------------------------------------- */
 /* Cholesky factor + solve of one instance by one workgroup                */
 /* ---------------------------------------------------------------------- */
@@ -414,13 +424,14 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
     const long lda = fresh(lda0);
     const int kb = min(PB, n - k), lane = fresh_lane(), li = lane & 15, lk = lane >> 4;
     const int ln = lane & (PB - 1), rhs = wave + 4 * (lane / PB);
-    T lc[PB], rd = T(0);
+    T lc[PB], d = T(1);                            /* a square root: 1 / d is normal */
     if (wave < nrhs) {
 #pragma unroll
       for (int j = 0; j < PB; ++j)
         lc[j] = (ln < j && j < kb) ? A[(size_t)(k + ln) * lda + k + j] : T(0);
-      if (ln < kb) rd = T(1) / A[(size_t)(k + ln) * lda + k + ln];
+      if (ln < kb) d = A[(size_t)(k + ln) * lda + k + ln];
     }
+    const T rd = T(1) / d;
     acc_t acc[2] = {acc_t{0, 0, 0, 0}, acc_t{0, 0, 0, 0}};
     const T *xr = s_x + (size_t)min(li, nrhs - 1) * n;
     for (int r0 = k + PB + 16 * wave; r0 < n; r0 += 16 * (NT / 64)) {
@@ -455,7 +466,7 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
       }
 #pragma unroll
       for (int j = PB - 1; j >= 0; --j) {          /* steps past kb change nothing */
-        const T x = g * rd;                        /* lane j's is x_j */
+        const T x = quotient(g, d, rd);            /* lane j's is x_j */
         T xj = bcast(x, j);
         if (nrhs > 4) xj = lane < PB ? xj : bcast(x, PB + j);
         g = ln == j ? x : fma(-lc[j], xj, g);
@@ -863,13 +874,17 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
       const long lda = fresh(lda0);
       const int kb = min(PB, n - k), lane = fresh_lane(), li = lane & 15, lk = lane >> 4;
       const int ln = lane & (PB - 1), rhs = wave + 4 * (lane / PB);
-      T uc[PB], rd = T(0);
+      T uc[PB], d = T(1);
       if (wave < nrhs) {
 #pragma unroll
         for (int j = 0; j < PB; ++j)
           uc[j] = (ln < j && j < kb) ? A[(size_t)(k + j) * lda + k + ln] : T(0);
-        if (ln < kb) rd = T(1) / A[(size_t)(k + ln) * lda + k + ln];
+        if (ln < kb) d = A[(size_t)(k + ln) * lda + k + ln];
       }
+      /* a pivot can be any nonzero number: where the reciprocal of one in the
+       * block would over- or underflow, divide */
+      const T rd = T(1) / d, ad = d < T(0) ? -d : d, lo = T(4) * Lim<T>::safmin();
+      const bool plain = __ballot(!(ad >= lo && ad <= T(1) / lo)) == 0ull;
       acc_t acc[2] = {acc_t{0, 0, 0, 0}, acc_t{0, 0, 0, 0}};
       const T *xr = S.x + (size_t)min(li, nrhs - 1) * n;
       for (int j0 = k + PB + 16 * wave; j0 < n; j0 += 16 * (NT / 64)) {
@@ -903,13 +918,17 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
           g = S.x[(size_t)rhs * n + k + ln] -
               ((sp[0] + sp[MAXR * PB]) + (sp[2 * MAXR * PB] + sp[3 * MAXR * PB]));
         }
+        auto solve = [&](auto divide) {
 #pragma unroll
-        for (int j = PB - 1; j >= 0; --j) {        /* steps past kb change nothing */
-          const T x = g * rd;                      /* lane j's is x_j */
-          T xj = bcast(x, j);
-          if (nrhs > 4) xj = lane < PB ? xj : bcast(x, PB + j);
-          g = ln == j ? x : fma(-uc[j], xj, g);
-        }
+          for (int j = PB - 1; j >= 0; --j) {      /* steps past kb change nothing */
+            const T x = decltype(divide)::value ? g / d : quotient(g, d, rd);
+            T xj = bcast(x, j);                    /* lane j's is x_j */
+            if (nrhs > 4) xj = lane < PB ? xj : bcast(x, PB + j);
+            g = ln == j ? x : fma(-uc[j], xj, g);
+          }
+        };
+        if (plain) solve(std::false_type());
+        else solve(std::true_type());
         if (rhs < nrhs && ln < kb) S.x[(size_t)rhs * n + k + ln] = g;
       }
       __syncthreads();

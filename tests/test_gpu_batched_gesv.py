@@ -85,3 +85,34 @@ def test_gesv_above_the_one_row_orders():
     import torch
     X.use_torch_stream()
     _run(torch, [257, 40, 300], np.float64, 2)
+
+
+@pytest.mark.parametrize("dt,e", [(np.float64, -1060), (np.float64, 1000), (np.float32, -140),
+                                  (np.float32, 120)])
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("nrhs", [1, 8])
+def test_gesv_pivots_without_a_normal_reciprocal(dt, e, trans, nrhs):
+    """U of small integers times 2^e, its diagonal powers of two: the solution
+    is integers and every step exact, so it must come out bit for bit, though
+    1 / U(i, i) over- or underflows."""
+    import torch
+    X.use_torch_stream()
+    rng = np.random.default_rng(nrhs)
+    A0, B0, X0 = [], [], []
+    for n in (1, 7, 40, 100):
+        U = np.triu(rng.integers(-1, 2, (n, n)), 1) * (rng.random((n, n)) < 2.0 / n)
+        U = U + np.diag(rng.choice([1, 2, 4], n) * rng.choice([-1, 1], n))
+        x = rng.integers(-3, 4, (n, nrhs))
+        A0.append(np.ldexp(U.astype(np.float64), e).astype(dt))
+        B0.append(np.ldexp(((U.T if trans else U) @ x).astype(np.float64), e).astype(dt))
+        X0.append(x)
+    dev = lambda m: torch.tensor(np.ascontiguousarray(m.T), device="cuda")   # noqa: E731
+    As, Bs = [dev(a) for a in A0], [dev(b) for b in B0]
+    piv = [torch.zeros(len(a), dtype=torch.int32, device="cuda") for a in A0]
+    info = torch.full((len(A0),), -7, dtype=torch.int32, device="cuda")
+    with (X.gesv_t_batch if trans else X.gesv_batch)(As, piv, Bs, info) as plan:
+        plan.run()
+        torch.cuda.synchronize()
+    assert not info.any()
+    for b, x in zip(Bs, X0):
+        assert np.array_equal(b.cpu().numpy().T, x.astype(dt))
