@@ -615,33 +615,39 @@ __device__ void wg_gesv(int n, T *A, long lda, int *ipiv, int nrhs, T *B, long l
 }
 
 /* ---------------------------------------------------------------------- */
-/* Cholesky adjoint of one instance by one workgroup                       */
-/* ---------------------------------------------------------------------- */
-/* ---------------------------------------------------------------------- */
 /* LU factor + solve of one instance of order <= NT: one panel row a thread */
 /* ---------------------------------------------------------------------- */
 /* Right-looking, panels of PB = 32 columns held in registers, one row per
- * thread (lu_panel.h).  The columns right of the panel are taken in strips
- * of 16, each wholly one wavefront's, so a strip's steps need no barrier:
- * gather the 32 rows that come to the top, put the displaced top rows where
- * those came from, U12 = inv(L11) times the gathered rows, and the trailing
- * rows -= L21 U12, products on the matrix cores formed transposed
- * (D[column][row]: a lane's 16 neighbours run down a column of A; the U12
- * accumulators are the operand of the update as they stand).  The
- * right-hand sides are one more strip, in LDS, so the forward substitution
- * costs no pass of its own.  The columns left of a panel get their
- * interchanges once at the end, as one map per panel composed from the
- * later panels' maps.
+ * thread (lu_panel.h), as two halves of 16: after the first the top 16 rows'
+ * second half is solved for by one wavefront and every row below takes its
+ * products.  The columns right of the panel are taken in strips of 16, each
+ * wholly one wavefront's, so a strip's steps need no barrier: gather the 32
+ * rows that come to the top, put the displaced top rows where those came
+ * from, U12 by substitution in groups of four rows, and the trailing rows -=
+ * L21 U12, products on the matrix cores formed transposed (D[column][row]: a
+ * lane's 16 neighbours run down a column of A; the U12 accumulators are the
+ * operand of the update as they stand).  The right-hand sides are one more
+ * strip, in LDS, so the forward substitution costs no pass of its own.  The
+ * columns left of a panel get their interchanges once at the end, as one map
+ * per panel composed from the later panels' maps.
+ *
+ * Rounding: multipliers are divisions, the only inverses those of 4 x 4
+ * blocks, and products are summed apart, eight to sixteen at a time, before
+ * they meet an entry.  FP32, mean residual of the factors of order 32 / 100
+ * / 256: 1.32e-7 / 3.08e-7 / 6.5e-7 (LDS panels of 16 or 32 with
+ * substitutions, as above order 256: 1.32 / 3.17 / 7.4; reciprocals,
+ * panels of 32 and products with inv(L11): 1.41 / 4.30 / 9.2).
  *
  * Bound by the panel's chain (about 1 us a column, two workgroups to a
  * compute unit hiding each other's); the form it replaces at these orders kept
  * the panel in LDS, swapped rows one dependent load at a time in every
  * column, and updated through uncoalesced tiles.  FP64, 4000 of order
- * 8..256, one right-hand side: 8.9 -> 2.8 ms. */
+ * 8..256, one right-hand side, with the inputs' copies: 9.5 -> 2.9 ms. */
 constexpr int MAXPAN = NT / PB;
 
 template <typename T>
 struct RowsPanel {
+  static constexpr bool DIVIDE = true;
   int w, row0;
   int *ipiv;
   T *s_prow, *s_cand;
@@ -651,33 +657,33 @@ struct RowsPanel {
   __device__ void zero_pivot(int C) const { if (*s_zero == 0) *s_zero = row0 + C + 1; }
 };
 
-/* inv(L11), unit lower, L11 at s_l[c PLD + r]: every lane one column of the
- * inverse, the multipliers by readlane from the lanes that hold the rows;
- * to s_inv[l PLD + c] = inv(c, l) */
+/* The strict part of inv(D) for each 4 x 4 diagonal block D of L11 (unit
+ * lower, at s_l[c PLD + r]): row r's four entries at s_n[4 r].  Thread 4 e +
+ * c of the first 32 forms column c of block e. */
 template <typename T>
-__device__ __forceinline__ void unit_lower_inverse(const T *s_l, T *s_inv) {
-  const int ln = fresh_lane() & (PB - 1);
-  T v[PB], z[PB];
+__device__ __forceinline__ void unit_lower_inverse4(const T *s_l, T *s_n) {
+  const int r0 = (int)threadIdx.x & ~3, k = (int)threadIdx.x & 3;
+  T z[4];
 #pragma unroll
-  for (int c = 0; c < PB; ++c) {
-    v[c] = c < ln ? s_l[c * PLD + ln] : T(0);
-    z[c] = c == ln ? T(1) : T(0);
-  }
+  for (int c = 0; c < 4; ++c) z[c] = c == k ? T(1) : T(0);
 #pragma unroll
-  for (int j = 0; j < PB; ++j) {
-    /* ties step j's readlanes to z[j]: they depend on no step, and all 992
-     * scalars were read ahead and spilled */
-    asm volatile("" : "+v"(v[j]), "+v"(z[j]));
+  for (int j = 0; j < 3; ++j)
 #pragma unroll
-    for (int c = j + 1; c < PB; ++c) z[c] = fma(-z[j], bcast(v[j], c), z[c]);
-  }
+    for (int c = j + 1; c < 4; ++c) z[c] = fma(-s_l[(r0 + j) * PLD + r0 + c], z[j], z[c]);
 #pragma unroll
-  for (int c = 0; c < PB; ++c) s_inv[ln * PLD + c] = z[c];
+  for (int c = 0; c < 4; ++c) s_n[4 * (r0 + c) + k] = c > k ? z[c] : T(0);
 }
+
+/* An MFMA's 16 rows by the group of four that element e of the accumulators
+ * holds: lane group g's element e is row 4 e + g of a tile whose operand
+ * row i is row mfma_row(i). */
+template <typename T> __device__ __forceinline__ int mfma_row(int i);
+template <> __device__ __forceinline__ int mfma_row<double>(int i) { return i; }
+template <> __device__ __forceinline__ int mfma_row<float>(int i) { return 4 * (i & 3) + (i >> 2); }
 
 template <typename T>
 struct GesvLds {
-  T *l11, *inv;            /* PB x PLD each */
+  T *l11, *inv;            /* PB x PLD; 16 x 16 */
   T *part;                 /* 4 x MAXR x PB */
   T *x;                    /* n x nrhs */
   int *src, *dst;          /* PB each: row now at top j; where top row j went (-1: stays) */
@@ -692,7 +698,7 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
   typedef typename MF::acc_t acc_t;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int li = lane & 15;
+  const int li = lane & 15, lk = lane >> 4, mr = mfma_row<T>(li);
   const int nr_fwd = trans ? 0 : nrhs;             /* right-hand sides carried along */
   if (tid == 0) *st.s_zero = 0;
   for (int e = tid; e < n * nrhs; e += NT) S.x[e] = B[(size_t)(e / n) * ldb + e % n];
@@ -701,22 +707,84 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
   for (int k = 0; k < n; k += PB) {
     const int kb = min(PB, n - k), mp = n - k;
     const long lda = fresh(lda0);
-    /* ---- the panel ---- */
-    T a[PB];
+    /* ---- the panel, 16 columns and then 16 ---- */
+    T a[16], b[16];
     int pos = tid < mp ? tid : -1;
 #pragma unroll
-    for (int c = 0; c < PB; ++c)
+    for (int c = 0; c < 16; ++c) {
       a[c] = (c < kb && tid < mp) ? A[(size_t)(k + c) * lda + k + tid] : T(0);
-    st.w = kb; st.row0 = k; st.ipiv = ipiv + k;
-    atlmx::panel_segment<T, NT, PB, 32, false>(st, a, pos);
-    atlmx::panel_segment<T, NT, PB, 16, false>(st, a, pos);
+      b[c] = (16 + c < kb && tid < mp) ? A[(size_t)(k + 16 + c) * lda + k + tid] : T(0);
+    }
+    st.w = min(kb, 16); st.row0 = k; st.ipiv = ipiv + k;
+    atlmx::panel_segment<T, NT, 16, 16, false>(st, a, pos);
+    if (kb > 16) {
+      T *s_u = S.inv;                              /* the first pivot rows' second half */
+      if (pos >= 0 && pos < 16)
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+          s_u[16 * pos + c] = b[c];
+          S.l11[c * PLD + pos] = c < pos ? a[c] : T(0);
+        }
+      __syncthreads();
+      if (wave == 0) {
+        /* a column per lane, row j in x[0] at step j; the next step's
+         * multipliers are on their way during a step (rows past 15: unused) */
+        T x[16], lc[15], ln[15];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = s_u[16 * r + li];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) ln[r - 1] = S.l11[r];
+#pragma unroll 1
+        for (int j = 0; j < 16; ++j) {
+#pragma unroll
+          for (int r = 1; r < 16; ++r) lc[r - 1] = ln[r - 1];
+          const T *next = S.l11 + min(j + 1, 14) * (PLD + 1);
+#pragma unroll
+          for (int r = 1; r < 16; ++r) ln[r - 1] = next[r];
+          const T x0 = x[0];
+          if (lane < 16) s_u[16 * j + li] = x0;
+#pragma unroll
+          for (int r = 1; r < 16; ++r) x[r - 1] = fma(-lc[r - 1], x0, x[r]);
+        }
+      }
+      __syncthreads();
+      T sum[16];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) sum[c] = T(0);
+#pragma unroll 1
+      for (int j = 0; j < 16; j += 4) {            /* a[] comes round once */
+        T l[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          T u[16], p = s_u[16 * (j + q) + li];
+          asm volatile("" : "+v"(p));              /* one row's entries at a time */
+          atlmx::row_spread<T, 0>(u, p);
+          l[q] = a[q];
+#pragma unroll
+          for (int c = 0; c < 16; ++c) sum[c] = fma(l[q], u[c], sum[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < 12; ++c) a[c] = a[c + 4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[12 + q] = l[q];
+      }
+#pragma unroll
+      for (int c = 0; c < 16; ++c) b[c] = pos >= 16 ? b[c] - sum[c] : b[c];
+      if (pos >= 0 && pos < 16)
+#pragma unroll
+        for (int c = 0; c < 16; ++c) b[c] = s_u[16 * pos + c];
+      pos -= 16;                                   /* the top 16 rows, and no row, below zero */
+      st.w = kb - 16; st.row0 = k + 16; st.ipiv = ipiv + k + 16;
+      atlmx::panel_segment<T, NT, 16, 16, false>(st, b, pos);
+      pos += 16;
+    }
     if (tid < PB) S.dst[tid] = -1;
     __syncthreads();
     if (pos >= 0) {
       const long ldp = fresh(lda0);
 #pragma unroll
       for (int c = 0; c < PB; ++c) {
-        const T v = a[16 - 16 * (c / 16) + c % 16];
+        const T v = c < 16 ? a[c % 16] : b[c % 16];
         if (c < kb) A[(size_t)(k + c) * ldp + k + pos] = v;
         if (pos < PB) S.l11[c * PLD + pos] = (c < kb && c < pos) ? v : T(0);
       }
@@ -731,34 +799,38 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
     __syncthreads();
     const int ns = (n - k - kb + 15) / 16;         /* strips of A's columns */
     if (ns == 0 && nr_fwd == 0) break;
-    if (wave == 0) unit_lower_inverse(S.l11, S.inv);
+    if (tid < PB) unit_lower_inverse4(S.l11, S.inv);
     __syncthreads();
 
     /* ---- strips: columns j0.. of A, then the right-hand sides.  cp(c) is
      * column c's base; clamped columns are read but not written. ---- */
     auto strip = [&](auto cp, int nc) {
-      acc_t xv[2], tv[2], u[2];
+      acc_t xv[2], tv[2], u[2], sum[2] = {acc_t{0, 0, 0, 0}, acc_t{0, 0, 0, 0}};
 #pragma unroll
       for (int l = 0; l < 2; ++l)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int j = 16 * l + MF::drow(lane, e);
+          const int j = 16 * l + 4 * e + lk;
           auto col = cp(min(li, nc - 1));
           xv[l][e] = j < kb ? col[k + S.src[j]] : T(0);
           tv[l][e] = j < kb ? col[k + j] : T(0);
         }
-      /* U12 = inv(L11) X: u[c][col] as D[row][col], rows in the elements */
+      /* U12: four rows at a time, in element e of each lane group one: the
+       * gathered rows less the sum so far, times the block's inverse; then
+       * their products join the later rows' sums */
 #pragma unroll
-      for (int c = 0; c < 2; ++c) u[c] = acc_t{0, 0, 0, 0};
-#pragma unroll
-      for (int l = 0; l < 2; ++l)
+      for (int l = 0; l < 2; ++l) {
+        const T nv = S.inv[4 * (16 * l + mr) + lk];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int row = 16 * l + MF::drow(lane, e);
-#pragma unroll
-          for (int c = l; c < 2; ++c)
-            u[c] = MF::mma(S.inv[row * PLD + 16 * c + li], xv[l][e], u[c]);
+          const T x = xv[l][e] + sum[l][e];
+          const acc_t z = MF::mma((mr >> 2) == e ? nv : T(0), x, acc_t{0, 0, 0, 0});
+          u[l][e] = x + z[e];
+          const T *Lc = S.l11 + (16 * l + 4 * e + lk) * PLD + mr;
+          if (e < 3) sum[l] = MF::mma((mr >> 2) > e ? -Lc[16 * l] : T(0), u[l][e], sum[l]);
+          if (l == 0) sum[1] = MF::mma(-Lc[16], u[0][e], sum[1]);
         }
+      }
       __threadfence_block();                       /* every read above is done */
       if (li < nc) {
         auto col = cp(li);
@@ -766,7 +838,7 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
         for (int l = 0; l < 2; ++l)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const int j = 16 * l + MF::drow(lane, e);
+            const int j = 16 * l + 4 * e + lk;
             if (j < kb) {
               const int d = S.dst[j];
               if (d >= 0) col[k + d] = tv[l][e];
@@ -778,13 +850,13 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
       /* the rows below: D'[col][row] = sum over j of U(j, col) L21(row, j) */
       for (int r0 = k + PB; r0 < n; r0 += 32) {    /* then kb == PB */
         const int ra = min(r0 + li, n - 1), rb = min(r0 + 16 + li, n - 1);
-        acc_t d0 = acc_t{0, 0, 0, 0}, d1 = acc_t{0, 0, 0, 0}, c0, c1;
+        acc_t d0[4], d1[4], c0, c1;                /* sums of eight products each */
         T b0[2][4], b1[2][4];
 #pragma unroll
         for (int l = 0; l < 2; ++l)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const T *Lc = A + (size_t)(k + 16 * l + MF::drow(lane, e)) * lda;
+            const T *Lc = A + (size_t)(k + 16 * l + 4 * e + lk) * lda;
             b0[l][e] = Lc[ra];
             b1[l][e] = Lc[rb];
           }
@@ -798,16 +870,22 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
         for (int l = 0; l < 2; ++l)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            d0 = MF::mma(u[l][e], b0[l][e], d0);
-            d1 = MF::mma(u[l][e], b1[l][e], d1);
+            const int h = 2 * l + e / 2;
+            d0[h] = MF::mma(u[l][e], b0[l][e], e & 1 ? d0[h] : acc_t{0, 0, 0, 0});
+            d1[h] = MF::mma(u[l][e], b1[l][e], e & 1 ? d1[h] : acc_t{0, 0, 0, 0});
           }
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          c0 -= d0[h];
+          c1 -= d1[h];
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int c = MF::drow(lane, e);
           if (c < nc) {
             auto col = cp(c);
-            if (r0 + li < n) col[ra] = c0[e] - d0[e];
-            if (r0 + 16 + li < n) col[rb] = c1[e] - d1[e];
+            if (r0 + li < n) col[ra] = c0[e];
+            if (r0 + 16 + li < n) col[rb] = c1[e];
           }
         }
       }
@@ -885,7 +963,8 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
        * block would over- or underflow, divide */
       const T rd = T(1) / d, ad = d < T(0) ? -d : d, lo = T(4) * Lim<T>::safmin();
       const bool plain = __ballot(!(ad >= lo && ad <= T(1) / lo)) == 0ull;
-      acc_t acc[2] = {acc_t{0, 0, 0, 0}, acc_t{0, 0, 0, 0}};
+      acc_t acc[2][2];                             /* two sums: half the terms in each */
+      zero_tile(acc);
       const T *xr = S.x + (size_t)min(li, nrhs - 1) * n;
       for (int j0 = k + PB + 16 * wave; j0 < n; j0 += 16 * (NT / 64)) {
         T ua[2][4], b[4];
@@ -899,8 +978,8 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
         }
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
-          acc[0] = MF::mma(ua[0][s4], b[s4], acc[0]);
-          acc[1] = MF::mma(ua[1][s4], b[s4], acc[1]);
+          acc[0][s4 / 2] = MF::mma(ua[0][s4], b[s4], acc[0][s4 / 2]);
+          acc[1][s4 / 2] = MF::mma(ua[1][s4], b[s4], acc[1][s4 / 2]);
         }
       }
       if (li < nrhs) {
@@ -908,7 +987,8 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) sp[li * PB + 16 * c + MF::drow(lane, e)] = acc[c][e];
+          for (int e = 0; e < 4; ++e)
+            sp[li * PB + 16 * c + MF::drow(lane, e)] = acc[c][0][e] + acc[c][1][e];
       }
       __syncthreads();
       if (wave < nrhs) {
@@ -937,6 +1017,9 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
   for (int e = tid; e < n * nrhs; e += NT) B[(size_t)(e / n) * ldb + e % n] = S.x[e];
 }
 
+/* ---------------------------------------------------------------------- */
+/* Cholesky adjoint of one instance by one workgroup                       */
+/* ---------------------------------------------------------------------- */
 /* Given L (lower triangle of A after potrf; its strict upper triangle is
  * overwritten with zeros here), X = A^{-1} B and Bb = A^{-1} Xb (the solve's
  * adjoint), write to G the gradient of <Xb, X> with respect to the lower
@@ -1054,7 +1137,7 @@ __global__ __launch_bounds__(NT, 2) void gesv_rows_batched_kernel(BatchArgs<T> g
   GesvLds<T> S;
   S.l11 = (T *)smem;
   S.inv = S.l11 + PB * PLD;
-  S.part = S.inv + PB * PLD;
+  S.part = S.inv + 16 * 16;
   S.x = S.part + 4 * MAXR * PB;                        /* maxn x nrhs */
   S.src = s_src; S.dst = s_dst; S.map = s_map; S.fin = s_fin;
   RowsPanel<T> st;
@@ -1216,7 +1299,7 @@ hipError_t launch_gesv(const BatchArgs<T> &g, int maxn, int grid, int trans, hip
 template <typename T>
 hipError_t launch_gesv_rows(const BatchArgs<T> &g, int maxn, int grid, int trans,
                             hipStream_t s) {
-  const size_t lds = sizeof(T) * (2 * (size_t)PB * PLD + 4 * MAXR * PB + (size_t)maxn * g.nrhs);
+  const size_t lds = sizeof(T) * ((size_t)PB * PLD + 16 * 16 + 4 * MAXR * PB + (size_t)maxn * g.nrhs);
   if (maxn > NT || lds > 64 * 1024) return hipErrorInvalidValue;
   hipLaunchKernelGGL((gesv_rows_batched_kernel<T>), dim3(grid), dim3(NT), lds, s, g, trans);
   return hipGetLastError();

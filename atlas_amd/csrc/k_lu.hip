@@ -98,6 +98,7 @@ __device__ inline double take_f64(u64 *p, unsigned tag) {
 
 template <typename T>
 struct PanelState {
+  static constexpr bool DIVIDE = false;
   int w, G, g, row0, seq;
   int *ipiv, *info;
   PanelSlots S;

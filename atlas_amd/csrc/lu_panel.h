@@ -94,8 +94,9 @@ __device__ __forceinline__ void row_spread(T (&b)[16], T p) {
  * Two barriers a column; with several workgroups (MULTI) the wavefront that
  * holds the candidate does the exchange.  State: w, row0, ipiv, s_prow and
  * s_cand (MW entries each), s_key and s_pos (one per wavefront), s_piv,
- * first() (this workgroup records
- * the pivots), zero_pivot(column), and with MULTI exchange(). */
+ * first() (this workgroup records the pivots), zero_pivot(column), DIVIDE
+ * (the multipliers by division, not by the pivot's reciprocal as LAPACK
+ * scales a column), and with MULTI exchange(). */
 template <typename T, int NTH, int MW, int WA, bool MULTI, class State>
 __device__ __forceinline__ void panel_segment(const State &st, T (&a)[MW], int &pos) {
   constexpr int NW = NTH / 64;
@@ -149,7 +150,7 @@ __device__ __forceinline__ void panel_segment(const State &st, T (&a)[MW], int &
     for (int q = 0; q < WA / 16; ++q) pr[q] = st.s_prow[16 * q + (lane & 15)];
     const T pv = st.s_prow[0];
     const bool act = pos > C && pv != T(0);
-    const bool recip = (pv < T(0) ? -pv : pv) >= Lim<T>::safmin();   /* uniform */
+    const bool recip = !State::DIVIDE && (pv < T(0) ? -pv : pv) >= Lim<T>::safmin(); /* uniform */
     const T l = act ? (recip ? a0 * (T(1) / pv) : a0 / pv) : T(0);
     if (pv == T(0) && st.first() && tid == 0) st.zero_pivot(C);
     bool fin = __builtin_isfinite(l);

@@ -116,3 +116,56 @@ def test_gesv_pivots_without_a_normal_reciprocal(dt, e, trans, nrhs):
     assert not info.any()
     for b, x in zip(Bs, X0):
         assert np.array_equal(b.cpu().numpy().T, x.astype(dt))
+
+
+def _lu_by_16(A):
+    """batch of FP32 matrices: LU by divisions, substitutions and updates 16
+    columns at a time, every operation rounded (products fused); the factors
+    and the row order"""
+    f = np.float32
+    fma = lambda a, b, c: (a.astype(np.float64) * b + c).astype(f)     # noqa: E731
+    A = A.copy()
+    b, n, _ = A.shape
+    rows, idx = np.tile(np.arange(n), (b, 1)), np.arange(b)
+    for k in range(0, n, 16):
+        e = min(n, k + 16)
+        for j in range(k, e):
+            p = j + np.argmax(np.abs(A[:, j:, j]), axis=1)
+            for M in (A, rows):
+                M[idx, j], M[idx, p] = M[idx, p], M[idx, j]
+            A[:, j + 1:, j] /= A[:, j, j, None]
+            A[:, j + 1:, j + 1:e] = fma(-A[:, j + 1:, j, None], A[:, None, j, j + 1:e],
+                                        A[:, j + 1:, j + 1:e])
+        for j in range(k, e):
+            A[:, j + 1:e, e:] = fma(-A[:, j + 1:e, j, None], A[:, None, j, e:], A[:, j + 1:e, e:])
+        S = np.zeros_like(A[:, e:, e:])
+        for j in range(k, e):
+            S = fma(A[:, e:, j, None], A[:, None, j, e:], S)
+        A[:, e:, e:] -= S
+    return A, rows
+
+
+@pytest.mark.parametrize("n,count", [(8, 2000), (20, 1000), (32, 1000), (64, 400), (100, 300)])
+def test_gesv_rounding_no_larger_than_by_substitution(n, count):
+    """The mean residual of the FP32 factors over a batch against that of the
+    same batch by divisions and substitutions; 2% for the samples' spread."""
+    import torch
+    X.use_torch_stream()
+    A = np.random.default_rng(n).uniform(-1, 1, (count, n, n)).astype(np.float32)
+    dev = torch.tensor(np.ascontiguousarray(A.transpose(0, 2, 1)), device="cuda")
+    piv = torch.zeros(count, n, dtype=torch.int32, device="cuda")
+    info = torch.zeros(count, dtype=torch.int32, device="cuda")
+    with X.gesv_batch(list(dev), list(piv), [], info) as plan:
+        plan.run()
+        torch.cuda.synchronize()
+    assert not info.any()
+    F, p = dev.cpu().numpy().transpose(0, 2, 1), piv.cpu().numpy()
+    rows, idx = np.tile(np.arange(n), (count, 1)), np.arange(count)
+    for j in range(n):
+        rows[idx, j], rows[idx, p[:, j]] = rows[idx, p[:, j]], rows[idx, j]
+
+    def resid(F, rows):
+        P = np.take_along_axis(A, rows[:, :, None], 1).astype(np.float64)
+        E = P - (np.tril(F, -1).astype(np.float64) + np.eye(n)) @ np.triu(F).astype(np.float64)
+        return (np.linalg.norm(E, axis=(1, 2)) / np.linalg.norm(P, axis=(1, 2))).mean()
+    assert resid(F, rows) <= 1.02 * resid(*_lu_by_16(A))
