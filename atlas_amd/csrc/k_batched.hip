@@ -831,6 +831,39 @@ __device__ void wg_gesv_rows(int n, T *A, const long lda0, int *ipiv, int nrhs, 
           if (l == 0) sum[1] = MF::mma(-Lc[16], u[0][e], sum[1]);
         }
       }
+      /* the inverse's zeros times an infinity or a NaN would reach up to
+       * three rows above it: then row by row, below it alone */
+      bool odd = false;
+#pragma unroll
+      for (int l = 0; l < 2; ++l)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) odd |= !__builtin_isfinite(u[l][e]);
+      if (__ballot(odd)) {
+        const int ln = fresh_lane(), c = ln & 15, g = ln >> 4;
+        auto col = cp(min(c, nc - 1));
+#pragma unroll
+        for (int l = 0; l < 2; ++l)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int j = 16 * l + 4 * e + g;
+            u[l][e] = j < kb ? col[k + S.src[j]] : T(0);
+          }
+#pragma unroll
+        for (int l = 0; l < 2; ++l)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll 1
+            for (int q = 0; q < 4; ++q) {          /* row j, from lane group q */
+              const int j = 16 * l + 4 * e + q;
+              const T uj = __shfl(u[l][e], 16 * q + c);
+              const T *Lc = S.l11 + j * PLD + g;
+#pragma unroll
+              for (int r = 4 * l + e; r < 8; ++r) {
+                const T v = fma(-Lc[4 * r], uj, u[r / 4][r % 4]);
+                u[r / 4][r % 4] = 4 * r + g > j ? v : u[r / 4][r % 4];
+              }
+            }
+      }
       __threadfence_block();                       /* every read above is done */
       if (li < nc) {
         auto col = cp(li);

@@ -169,3 +169,43 @@ def test_gesv_rounding_no_larger_than_by_substitution(n, count):
         E = P - (np.tril(F, -1).astype(np.float64) + np.eye(n)) @ np.triu(F).astype(np.float64)
         return (np.linalg.norm(E, axis=(1, 2)) / np.linalg.norm(P, axis=(1, 2))).mean()
     assert resid(F, rows) <= 1.02 * resid(*_lu_by_16(A))
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_gesv_nonfinite_entry_stays_below_its_row(dt, bad):
+    """An entry right of the first panel, in the row that becomes pivot row j,
+    is not finite: its column's entries above row j, and every other column's
+    top 32 rows, are what they are without it, as a substitution leaves them."""
+    import torch
+    X.use_torch_stream()
+    n, tops = 100, [1, 2, 3, 6, 14, 15, 16, 19, 29, 31]
+    S = np.random.default_rng(4).uniform(-1, 1, (n, n)).astype(dt)
+
+    def run(mats):
+        As = [torch.tensor(np.ascontiguousarray(a.T), device="cuda") for a in mats]
+        piv = [torch.zeros(n, dtype=torch.int32, device="cuda") for _ in mats]
+        info = torch.zeros(len(mats), dtype=torch.int32, device="cuda")
+        with X.gesv_batch(As, piv, [], info) as plan:
+            plan.run()
+            torch.cuda.synchronize()
+        return [a.cpu().numpy().T for a in As], [p.cpu().numpy() for p in piv]
+    (R,), (p,) = run([S])
+    rows = np.arange(n)
+    for k, q in enumerate(p):
+        rows[[k, q]] = rows[[q, k]]
+    cols = [32 + (7 * j) % 60 for j in tops]
+    mats = []
+    for j, c in zip(tops, cols):
+        M = S.copy()
+        M[rows[j], c] = bad
+        mats.append(M)
+    F, piv = run(mats)
+    # the same sums in another order: c n u |L| |U|, both below 8 here
+    tol = 64 * n * np.finfo(dt).eps
+    for j, c, f, q in zip(tops, cols, F, piv):
+        assert np.array_equal(q[:32], p[:32])
+        keep = [i for i in range(n) if i != c]
+        assert np.abs(f[:32, keep] - R[:32, keep]).max() <= tol, (j, c)
+        assert np.abs(f[:j, c] - R[:j, c]).max() <= tol, (j, c)
+        assert not np.isfinite(f[j, c])
