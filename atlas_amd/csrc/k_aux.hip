@@ -49,13 +49,15 @@ template <> struct IvMfma<float> {
 };
 
 /* The doubling levels on the matrix cores.  Ls: the factor, lower, [i][j];
- * Xs: the inverse, zero but for its four 16x16 diagonal blocks on entry. */
+ * Xs: the inverse, zero but for its four 16x16 diagonal blocks on entry.
+ * Returns whether this lane formed an entry that is not finite. */
 template <typename T>
-__device__ __forceinline__ void tri_doubling_mfma(const T (*Ls)[TNB + 1], T (*Xs)[TNB + 1]) {
+__device__ __forceinline__ int tri_doubling_mfma(const T (*Ls)[TNB + 1], T (*Xs)[TNB + 1]) {
   typedef IvMfma<T> MF;
   typedef typename MF::acc_t acc_t;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane & 15, lk = lane >> 4;
+  int odd = 0;
   if (wave < 2) {                                  /* 16: pair at 32 wave */
     const int c0 = 32 * wave, r0 = c0 + 16;
     acc_t t = acc_t{0, 0, 0, 0}, x = acc_t{0, 0, 0, 0};
@@ -65,7 +67,10 @@ __device__ __forceinline__ void tri_doubling_mfma(const T (*Ls)[TNB + 1], T (*Xs
 #pragma unroll
     for (int e = 0; e < 4; ++e) x = MF::mma(Xs[r0 + li][r0 + MF::drow(lane, e)], t[e], x);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) Xs[r0 + MF::drow(lane, e)][c0 + li] = -x[e];
+    for (int e = 0; e < 4; ++e) {
+      Xs[r0 + MF::drow(lane, e)][c0 + li] = -x[e];
+      odd |= !__builtin_isfinite(x[e]);
+    }
   }
   __syncthreads();
   /* 32: wavefront w forms columns 16 (w & 1) of T and, from them, its 16x16
@@ -86,8 +91,11 @@ __device__ __forceinline__ void tri_doubling_mfma(const T (*Ls)[TNB + 1], T (*Xs
       x = MF::mma(Xs[32 + ib + li][32 + 16 * r + MF::drow(lane, e)], t[r][e], x);
   __syncthreads();
 #pragma unroll
-  for (int e = 0; e < 4; ++e) Xs[32 + ib + MF::drow(lane, e)][jb + li] = -x[e];
-  __syncthreads();
+  for (int e = 0; e < 4; ++e) {
+    Xs[32 + ib + MF::drow(lane, e)][jb + li] = -x[e];
+    odd |= !__builtin_isfinite(x[e]);
+  }
+  return odd;
 }
 
 template <typename T>
@@ -143,7 +151,7 @@ __global__ __launch_bounds__(256) void tri_inv_kernel(int lower, int unit, int n
     }
   }
   odd = __syncthreads_or(odd);
-  if (!odd) tri_doubling_mfma<T>(Ls, Xs);
+  if (!odd) odd = __syncthreads_or(tri_doubling_mfma<T>(Ls, Xs));
   /* doubling by loops: blocks of 2h from two blocks of h */
   if (odd)
   for (int h = 16; h < TNB; h *= 2) {

@@ -47,3 +47,22 @@ def test_trsm_nonfinite_entry_stays_below_its_row(bad):
     ref = np.linalg.solve(np.tril(A)[:40, :40], B[:40])
     assert np.allclose(Y[:40], ref, rtol=1e-11, atol=1e-13)
     assert not np.isfinite(Y[40]).any()
+
+
+@pytest.mark.parametrize("dt,tiny,big", [(np.float64, 1e-300, 1e200), (np.float32, 1e-30, 1e20)])
+@pytest.mark.parametrize("row", [20, 40])
+def test_trsm_overflow_in_the_inverse_stays_below_its_row(dt, tiny, big, row):
+    """A small diagonal entry and a large one below it overflow in the
+    block's inverse: the rows above the large entry do not depend on it."""
+    n = 64
+    A, _ = _tri(np.random.default_rng(3), n, X.Lower, X.NonUnit, dt)
+    A[5, 5], A[6:, 5], A[row, 5] = tiny, 0, big
+    B = np.asfortranarray(np.random.default_rng(4).uniform(-1, 1, (n, 300)).astype(dt))
+    B[5] = tiny
+    Y = X.trsm(X.Left, X.Lower, X.NoTrans, X.NonUnit, 1.0, A, B.copy(order="F"))
+    ref = np.linalg.solve(np.tril(A)[:row, :row].astype(np.float64), B[:row])
+    M = np.abs(np.tril(A)[:row, :row].astype(np.float64))
+    M[:, 5] = M[5] = 0
+    M[5, 5] = 1          # row 5 and column 5 stand apart
+    bound = 8 * (n + 1) * np.finfo(dt).eps * (np.abs(np.linalg.inv(M)) @ (M @ np.abs(ref))) + 1e-30
+    assert np.all(np.abs(Y[:row] - ref) <= bound)
