@@ -34,9 +34,11 @@ using namespace atlmx;
  * A[i rs + k cs], so that Upper (A = U^T U, L = U^T) is the same code.  What
  * bounds it: four times the one-wavefront factor of 32 columns.  128
  * columns, FP64: 87 us for one barrier-separated step per column, and 15 for
- * the inverses' launch; 71 for both with the tiles in memory; 46 so: 3 for
- * the load, 6.3 for each panel's factor, 2 to 4 for its products, 4 for the
- * store. */
+ * the inverses' launch; 71 for both with the tiles in memory; 49 so: 3 for
+ * the load, 7 for each panel's factor, 2 to 4 for its products, 4 for the
+ * store.  Tiles and column groups beyond the matrix are passed over: one of
+ * order 1 takes 6 us (5 in the form with a barrier per step, 13 with the
+ * whole block). */
 constexpr int TBLK = PB * PLD;
 constexpr int NTILE = (CNB / PB) * (CNB / PB + 1) / 2;
 
@@ -60,7 +62,8 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
   const int f = tid % PB, g = tid / PB;
   T in[NTILE][PB * PB / NT];                       /* every load before the first use */
 #pragma unroll
-  for (int i = 0, q = 0; i < CNB / PB; ++i)
+  for (int i = 0, q = 0; i < CNB / PB; ++i) {
+    if (i >= nt) break;
 #pragma unroll
     for (int j = 0; j <= i; ++j, ++q)
 #pragma unroll
@@ -70,13 +73,18 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
         in[q][h] = ar == ac ? T(1) : T(0);         /* beyond the matrix: the identity */
         if (ar < n && ac <= ar) in[q][h] = A[(long)ar * rs + (long)ac * cs];
       }
+  }
 #pragma unroll
-  for (int q = 0; q < NTILE; ++q)
+  for (int i = 0, q = 0; i < CNB / PB; ++i) {
+    if (i >= nt) break;                            /* rows of tiles beyond the matrix */
 #pragma unroll
-    for (int h = 0; h < PB * PB / NT; ++h) {
-      const int r = lower ? f : g + h * (NT / PB), c = lower ? g + h * (NT / PB) : f;
-      s_l[q * TBLK + c * PLD + r] = in[q][h];
-    }
+    for (int j = 0; j <= i; ++j, ++q)
+#pragma unroll
+      for (int h = 0; h < PB * PB / NT; ++h) {
+        const int r = lower ? f : g + h * (NT / PB), c = lower ? g + h * (NT / PB) : f;
+        s_l[q * TBLK + c * PLD + r] = in[q][h];
+      }
+  }
   __syncthreads();
   for (int p = 0; p < nt; ++p) {
     if (p) {
