@@ -228,17 +228,18 @@ __device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][
  * arithmetic on every column before it.  6.3 us. */
 constexpr int GRP0 = 4, GRP = 8;
 template <typename T, bool PLAIN, int G0, int W>
-__device__ __forceinline__ void block_group(T (&v)[PB], const T *s_d, int nb, int &fail,
-                                            bool &plain) {
+__device__ __forceinline__ void block_group(T (&v)[PB], T (&in)[GRP], const T *s_d, int nb,
+                                            int &fail, bool &plain) {
   if (G0 >= nb || (!PLAIN && fail)) return;        /* uniform */
   const int lane = fresh_lane();
   if (G0 > 0) {
 #pragma unroll
-    for (int c = G0; c < G0 + W; ++c) {
-      const T d = s_d[c * PLD + (lane & (PB - 1))];
-      v[c] += lane < PB ? d : T(0);
-    }
+    for (int c = 0; c < W; ++c) v[G0 + c] += lane < PB ? in[c] : T(0);
   }
+  /* the next group's entries, on their way during this one */
+#pragma unroll
+  for (int c = 0; c < GRP; ++c)
+    if (G0 + W + c < PB) in[c] = s_d[(G0 + W + c) * PLD + (lane & (PB - 1))];
 #pragma unroll
   for (int j = G0; j < G0 + W; ++j) {
     if (PLAIN || !fail) {
@@ -262,16 +263,17 @@ __device__ __forceinline__ int block_columns(T (&v)[PB], const T *s_d, int nb) {
   const int lane = fresh_lane();
   int fail = 0;
   bool plain = true;
+  T in[GRP];
 #pragma unroll
   for (int c = 0; c < PB; ++c) {
     v[c] = c == lane - PB ? T(1) : T(0);
     if (c < GRP0 && lane < PB) v[c] = s_d[c * PLD + lane];
   }
-  block_group<T, PLAIN, 0, GRP0>(v, s_d, nb, fail, plain);
-  block_group<T, PLAIN, GRP0, GRP - GRP0>(v, s_d, nb, fail, plain);
-  block_group<T, PLAIN, GRP, GRP>(v, s_d, nb, fail, plain);
-  block_group<T, PLAIN, 2 * GRP, GRP>(v, s_d, nb, fail, plain);
-  block_group<T, PLAIN, 3 * GRP, GRP>(v, s_d, nb, fail, plain);
+  block_group<T, PLAIN, 0, GRP0>(v, in, s_d, nb, fail, plain);
+  block_group<T, PLAIN, GRP0, GRP - GRP0>(v, in, s_d, nb, fail, plain);
+  block_group<T, PLAIN, GRP, GRP>(v, in, s_d, nb, fail, plain);
+  block_group<T, PLAIN, 2 * GRP, GRP>(v, in, s_d, nb, fail, plain);
+  block_group<T, PLAIN, 3 * GRP, GRP>(v, in, s_d, nb, fail, plain);
   return PLAIN ? !plain : fail;
 }
 

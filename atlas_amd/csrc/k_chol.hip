@@ -152,15 +152,25 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
         __builtin_amdgcn_s_sleep(1);
       tile_times_inv<T, 2>(w, s_i[p & 1]);
       const int nc = s_fail ? s_fail - 1 - p * PB : PB;
+      if (nc == PB) {
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int col = 16 * c + MF::drow(lane, e);
-          if (col < nc)
+          for (int r = 0; r < 2; ++r)
 #pragma unroll
-            for (int r = 0; r < 2; ++r) x[col * PLD + 16 * r + li] = w[c][r][e];
-        }
+            for (int e = 0; e < 4; ++e)
+              x[(16 * c + MF::drow(lane, e)) * PLD + 16 * r + li] = w[c][r][e];
+      } else {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int col = 16 * c + MF::drow(lane, e);
+            if (col < nc)
+#pragma unroll
+              for (int r = 0; r < 2; ++r) x[col * PLD + 16 * r + li] = w[c][r][e];
+          }
+      }
     }
     __syncthreads();
     if (s_fail) break;
