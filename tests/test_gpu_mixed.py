@@ -505,3 +505,25 @@ def test_dsgesv_lapack_stopping_test(torch):
     # the GPU met the test on its own FP64 residual; recomputing A x - b here
     # in another order adds up to ~n eps ||A|| ||x|| of rounding
     assert r <= np.abs(xs).max() * np.abs(A).sum(axis=1).max() * 2.0 ** -53 * (np.sqrt(n) + n)
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2, 3])
+def test_dsgesv_gives_a_hopeless_preconditioner_up_after_two_cycles(torch, seed):
+    """kappa 1e9 at n = 1000, two-sided Haar: neither FP32 factorization
+    preconditions it well enough.  A GMRES cycle is at most 100 steps; the
+    second that does not halve the residual ends it, for the two
+    factorizations tried, and the FP64 solve answers."""
+    n, kappa = 1000, 1e9
+    rng = np.random.default_rng(seed)
+    q = lambda: np.linalg.qr(rng.standard_normal((n, n)))[0]           # noqa: E731
+    A = (q() * kappa ** (-np.arange(n) / (n - 1))) @ q().T
+    b = rng.standard_normal((n, 1))
+    Y = torch.zeros(1, n, dtype=torch.float64, device="cuda")
+    X.set_refine_stop(True)
+    info, st = X.dsgesv_dev(_dev(torch, A, torch.float64), _dev(torch, b, torch.float64), Y)
+    X.set_refine_stop(False)
+    x = _host(Y)
+    assert info == 0
+    assert np.abs(b - A @ x).max() <= n * EPS64 * np.abs(A).sum(1).max() * np.abs(x).max()
+    if st.fallback:
+        assert st.inner_iterations <= 2 * 2 * 100
