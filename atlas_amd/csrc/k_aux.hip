@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void tri_inv_kernel(int lower, int unit, int n
   }
   /* (an upper half of Ls not yet written is read by no product below: every
    * L block there lies wholly below the diagonal) */
-  odd = __syncthreads_or(odd);
+  __syncthreads();
   /* the 16x16 diagonal sub-blocks, by substitution: lane (q, c) builds
    * column c of inv(L_qq) */
   if (tid < 64) {
