@@ -107,6 +107,7 @@ __device__ void wave_tile_update(T *C, long ldc, const T *X, long ldx, const T *
 constexpr int SB = 32;
 constexpr int RCH = 4;                             /* right-hand sides per pass */
 constexpr int RCT = 2;                             /* the transposed GEMV's accumulator set */
+constexpr int SOLVE_LDS = SB * (SB + 1) + 4 * RCH * SB;   /* s_blk and s_part */
 template <typename T>
 __device__ void wg_trsv(int n, int nrhs, const T *A, long lda, bool lower, bool trans, bool unit,
                         T *X, T *s_blk, T *s_part) {
@@ -483,7 +484,7 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
 /* ---------------------------------------------------------------------- */
 template <typename T, int NB>
 __device__ void wg_gesv(int n, T *A, long lda, int *ipiv, int nrhs, T *B, long ldb, int *info,
-                        T *s_p, T *s_a, T *s_b, T *s_x, T *s_v, int *s_i, bool trans) {
+                        T *s_p, T *s_t, T *s_x, T *s_v, int *s_i, bool trans) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int first0 = 0;                          /* first exactly-zero pivot, 1-based */
   for (int k = 0; k < n; k += NB) {
@@ -587,7 +588,7 @@ __device__ void wg_gesv(int n, T *A, long lda, int *ipiv, int nrhs, T *B, long l
   if (nrhs <= 0 || first0) return;
   /* ---- getrs in LDS (ATL_getrs.c:8-89): NoTrans: P b, L y = b (unit),
    * U x = y; Trans (A^T = U^T L^T P): U^T z = b, L^T w = z (unit), x = P^T w.
-   * The triangular solves stage through s_a, s_b (contiguous) ---- */
+   * The triangular solves stage through s_t ---- */
   __syncthreads();
   for (int e = tid; e < n * nrhs; e += NT) s_x[e] = B[(size_t)(e / n) * ldb + e % n];
   __syncthreads();
@@ -598,11 +599,11 @@ __device__ void wg_gesv(int n, T *A, long lda, int *ipiv, int nrhs, T *B, long l
     }
   }
   if (!trans) {
-    wg_trsv(n, nrhs, A, lda, true, false, true, s_x, s_a, s_a + SB * (SB + 1));
-    wg_trsv(n, nrhs, A, lda, false, false, false, s_x, s_a, s_a + SB * (SB + 1));
+    wg_trsv(n, nrhs, A, lda, true, false, true, s_x, s_t, s_t + SB * (SB + 1));
+    wg_trsv(n, nrhs, A, lda, false, false, false, s_x, s_t, s_t + SB * (SB + 1));
   } else {
-    wg_trsv(n, nrhs, A, lda, false, true, false, s_x, s_a, s_a + SB * (SB + 1));
-    wg_trsv(n, nrhs, A, lda, true, true, true, s_x, s_a, s_a + SB * (SB + 1));
+    wg_trsv(n, nrhs, A, lda, false, true, false, s_x, s_t, s_t + SB * (SB + 1));
+    wg_trsv(n, nrhs, A, lda, true, true, true, s_x, s_t, s_t + SB * (SB + 1));
   }
   if (trans && tid < nrhs) {                 /* x = P^T w: the swaps in reverse */
     for (int j = n - 1; j >= 0; --j) {
@@ -1142,9 +1143,8 @@ template <typename T, int NB>
 __global__ __launch_bounds__(NT) void gesv_batched_kernel(BatchArgs<T> g, int maxn, int trans) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   T *s_p = (T *)smem;                                  /* maxn x NB */
-  T *s_a = s_p + (size_t)maxn * NB;                    /* 16 x 64 */
-  T *s_b = s_a + 16 * TS;
-  T *s_x = s_b + 16 * TS;                              /* maxn x nrhs */
+  T *s_t = s_p + (size_t)maxn * NB;                    /* the solves' staging */
+  T *s_x = s_t + SOLVE_LDS;                            /* maxn x nrhs */
   __shared__ T s_v[4];
   __shared__ int s_i[5];
   __shared__ int s_item;
@@ -1156,7 +1156,7 @@ __global__ __launch_bounds__(NT) void gesv_batched_kernel(BatchArgs<T> g, int ma
     if (it >= g.count) return;
     const int i = g.order[it];
     wg_gesv<T, NB>(g.n[i], g.A[i], g.lda[i], g.ipiv[i], g.nrhs, g.B ? g.B[i] : nullptr,
-                   g.ldb ? g.ldb[i] : 1, &g.info[i], s_p, s_a, s_b, s_x, s_v, s_i, trans != 0);
+                   g.ldb ? g.ldb[i] : 1, &g.info[i], s_p, s_t, s_x, s_v, s_i, trans != 0);
   }
 }
 
@@ -1304,13 +1304,34 @@ __global__ __launch_bounds__(NT) void chol_adjoint_kernel(AdjArgs<T> g) {
   }
 }
 
+/* LDS of one workgroup, beside which the kernels keep at most 64 bytes of
+ * static words */
+constexpr size_t LDS_CAP = 160 * 1024 - 64;
+template <typename T>
+constexpr size_t posv_lds(size_t maxn, size_t nrhs, size_t blocks) {
+  return sizeof(T) * (blocks * PB * PLD + maxn * nrhs);
+}
+template <typename T>
+constexpr size_t gesv_lds(size_t maxn, size_t nb) {
+  return sizeof(T) * (maxn * nb + SOLVE_LDS + maxn * MAXR);
+}
+
+/* The largest orders of plans (0 Cholesky, 1 LU), with as many right-hand
+ * sides as a plan may have */
+template <typename T>
+constexpr int max_order(int kind) {
+  return sizeof(T) == 8 ? (kind == 0 ? 2270 : 768) : (kind == 0 ? 4830 : 1621);
+}
+static_assert(posv_lds<double>(max_order<double>(0), MAXR, 2) <= LDS_CAP &&
+              posv_lds<float>(max_order<float>(0), MAXR, 2) <= LDS_CAP &&
+              gesv_lds<double>(max_order<double>(1), 16) <= LDS_CAP &&
+              gesv_lds<float>(max_order<float>(1), 16) <= LDS_CAP, "the largest orders fit");
+
 template <typename T>
 hipError_t launch_posv(const BatchArgs<T> &g, int maxn, int grid, hipStream_t s) {
-  const size_t x = sizeof(T) * (size_t)maxn * g.nrhs, blk = sizeof(T) * PB * PLD;
-  const size_t cap = 160 * 1024 - 64;              /* less the static words */
-  const int blocks = 4 * blk + x <= cap ? 4 : 2;
-  const size_t lds = blocks * blk + x;
-  if (lds > cap) return hipErrorInvalidValue;
+  const int blocks = posv_lds<T>(maxn, g.nrhs, 4) <= LDS_CAP ? 4 : 2;
+  const size_t lds = posv_lds<T>(maxn, g.nrhs, blocks);
+  if (lds > LDS_CAP) return hipErrorInvalidValue;
   hipError_t e = hipFuncSetAttribute((const void *)posv_batched_kernel<T>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
@@ -1320,8 +1341,8 @@ hipError_t launch_posv(const BatchArgs<T> &g, int maxn, int grid, hipStream_t s)
 
 template <typename T, int NB>
 hipError_t launch_gesv(const BatchArgs<T> &g, int maxn, int grid, int trans, hipStream_t s) {
-  const size_t lds = sizeof(T) * ((size_t)maxn * NB + 2 * 16 * TS + (size_t)maxn * MAXR);
-  if (lds > 160 * 1024) return hipErrorInvalidValue;
+  const size_t lds = gesv_lds<T>(maxn, NB);
+  if (lds > LDS_CAP) return hipErrorInvalidValue;
   hipError_t e = hipFuncSetAttribute((const void *)gesv_batched_kernel<T, NB>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
@@ -1347,12 +1368,13 @@ hipError_t batch_factor(int kind, int nb, int count, const int *order, const int
   BatchArgs<T> g;
   g.count = count; g.order = order; g.n = n; g.A = A; g.lda = lda; g.ipiv = ipiv;
   g.nrhs = nrhs; g.B = B; g.ldb = ldb; g.info = info; g.counter = counter;
-  if (kind == 0) {
-    if (nb == 16 || nb == 32) return launch_posv<T>(g, maxn, grid, s);   /* one panel width */
-  } else if (kind == 1 || kind == 2) {      /* 2: solve with A^T */
+  if (kind == 0) return launch_posv<T>(g, maxn, grid, s);
+  if (kind == 1 || kind == 2) {             /* 2: solve with A^T */
     if (maxn <= NT) return launch_gesv_rows<T>(g, maxn, grid, kind == 2, s);
-    if (nb == 16) return launch_gesv<T, 16>(g, maxn, grid, kind == 2, s);
-    if (nb == 32) return launch_gesv<T, 32>(g, maxn, grid, kind == 2, s);
+    /* a width timed on another plan of the bucket may not fit this one's order */
+    if (nb == 32 && gesv_lds<T>(maxn, 32) <= LDS_CAP)
+      return launch_gesv<T, 32>(g, maxn, grid, kind == 2, s);
+    if (nb == 16 || nb == 32) return launch_gesv<T, 16>(g, maxn, grid, kind == 2, s);
   }
   return hipErrorInvalidValue;
 }
@@ -1489,16 +1511,6 @@ __global__ __launch_bounds__(64 * NW) void gemm_batched_mfma_kernel(GemmBatchArg
           }
         }
   }
-}
-
-/* Largest instance order whose LDS working set fits (panel width 16, the
- * smaller of the two the autotuner tries). */
-template <typename T>
-int max_order(int kind) {
-  const long cap = 160 * 1024 / (long)sizeof(T);
-  const long fixed = (kind == 0 ? 16L * 17 : 0L) + 2L * 16 * TS;
-  const long per_row = (kind == 0 ? 0L : 16L) + MAXR;
-  return (int)((cap - fixed) / per_row);
 }
 
 template <typename T>

@@ -92,3 +92,26 @@ def test_leading_dimensions_above_the_order(kind, dt, nrhs, above):
         assert np.array_equal(a, b), i
     if kind != "posv_adjoint":
         assert not plain[-2].any()
+
+
+def test_largest_lu_orders_and_a_width_from_a_smaller_plan():
+    """The largest orders run, with 8 right-hand sides; and an order whose
+    panel of 32 columns does not fit runs after a smaller one of its size
+    class has been timed."""
+    import torch
+    X.use_torch_stream()
+    L = X.lib()
+    for dt, dbl in ((np.float64, 1), (np.float32, 0)):
+        for sizes in ([L.atlmx_batch_max_order(1, dbl)], [300], [500]):
+            rng = np.random.default_rng(sizes[0])
+            A, B = rng.uniform(-1, 1, (sizes[0],) * 2), rng.uniform(-1, 1, (sizes[0], 8))
+            As, Bs = _Mats([A.astype(dt)], [0], torch), _Mats([B.astype(dt)], [0], torch)
+            piv = [torch.zeros(sizes[0], dtype=torch.int32, device="cuda")]
+            info = torch.full((1,), -7, dtype=torch.int32, device="cuda")
+            with X.gesv_batch(As.t, piv, Bs.t, info) as plan:
+                plan.run()
+                torch.cuda.synchronize()
+            x = Bs.get()[0].astype(np.float64)
+            r = np.abs(B.astype(dt) - A.astype(dt).astype(np.float64) @ x).max()
+            assert int(info) == 0
+            assert r <= 64 * sizes[0] * np.finfo(dt).eps * np.abs(A).sum(1).max() * np.abs(x).max()
