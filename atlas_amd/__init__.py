@@ -554,16 +554,16 @@ def gesv_t_batch(As, ipivs, Bs, info):
     return Batch(h, keep + (info,))
 
 
-def posv_adjoint_batch(Ls, Xs, Bbs, Gs, Ws):
+def posv_adjoint_batch(Ls, Xs, Bbs, Gs, Ws=None):
     """Plan the Cholesky adjoint: G_i = d<Xb, X>/d tril(A_i) from L_i
-    (factored A_i), X_i and Bb_i = A_i^{-1} Xb_i."""
+    (factored A_i), X_i and Bb_i = A_i^{-1} Xb_i.  Ws is not used."""
     L = lib()
     _setup_adjoint(L)
     pre = "d" if Ls[0].dtype.itemsize == 8 else "s"
     n = [a.shape[0] for a in Ls]
-    arrs = [_ptr_array(t) for t in (Ls, Xs, Bbs, Gs, Ws)]
+    arrs = [_ptr_array(t) for t in (Ls, Xs, Bbs, Gs)]
     keep = tuple(arrs) + (_ints(n),)
     h = getattr(L, "atlmx_%sposv_adjoint_batch_plan" % pre)(
-        len(Ls), keep[5], dptr(arrs[0]), keep[5], Xs[0].shape[0], dptr(arrs[1]), dptr(arrs[2]),
-        keep[5], dptr(arrs[3]), keep[5], dptr(arrs[4]))
+        len(Ls), keep[4], dptr(arrs[0]), keep[4], Xs[0].shape[0], dptr(arrs[1]), dptr(arrs[2]),
+        keep[4], dptr(arrs[3]), keep[4], None)
     return Batch(h, keep)

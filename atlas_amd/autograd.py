@@ -82,8 +82,7 @@ class CholeskySolve(torch.autograd.Function):
         _posv(Lw, Bb)                                   # L recomputed, Bb = A^{-1} Xb
         Xc = _cm(X)
         G = torch.empty_like(Lw)
-        W = torch.empty_like(Lw)
-        with posv_adjoint_batch(list(Lw), list(Xc), list(Bb), list(G), list(W)) as plan:
+        with posv_adjoint_batch(list(Lw), list(Xc), list(Bb), list(G)) as plan:
             plan.run()
         return G.transpose(-1, -2), Bb.transpose(-1, -2)
 

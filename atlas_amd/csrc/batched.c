@@ -264,7 +264,7 @@ static void autotune(atlmx_batch *p, const int *h_order, const int *h_n, const i
   }
   if (p->kind == BK_POSV) {
     /* one kernel, and as many workgroups as its registers let share a
-     * compute unit (212 in FP64, 157 in FP32): the timing below, on a sample
+     * compute unit (246 in FP64, 165 in FP32): the timing below, on a sample
      * of 512, had preferred one for orders up to 512 because its largest
      * instances alone run faster unshared (4000 of order 8..512: FP64 4.2 ms
      * with one, 2.9 with two; FP32 3.2 / 2.0 / 1.7 with one / two / three).

@@ -66,8 +66,8 @@ void NM(PFX, update_dev)(atlmx_ctx *c, int tb, int M, int N, int K, T alpha, con
  * updates) and the amm outer loops ATL_trsmL_LN_UT.c:11-110 that alternate
  * utrsm diagonal solves with GEMM updates.  Here the 64x64 diagonal blocks
  * are inverted in one launch, then per diagonal block one in-place GEMM
- * (X_k = op(inv A_kk) * B_k, a single 128-row tile, so it reads B_k before
- * writing it) and one GEMM update of the rest of B.  Left-side solves with
+ * (X_k = op(inv A_kk) * B_k, tiles that span the block's 64 rows, so each
+ * workgroup reads its part of B_k before writing it) and one GEMM update of the rest of B.  Left-side solves with
  * one column (or a few, within one diagonal block) run as one flag-chained
  * launch, and with up to ATLMX_TRSM_TAG_MAXRHS as one launch of work items
  * of two 64-row blocks by 16 columns chained the same way (matrix-core

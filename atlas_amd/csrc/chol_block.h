@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include "mfma16.h"
 
 namespace atlmx {
 
@@ -26,26 +27,6 @@ template <typename T> __device__ inline T dsqrt(T x);
 template <> __device__ inline double dsqrt<double>(double x) { return sqrt(x); }
 template <> __device__ inline float dsqrt<float>(float x) { return sqrtf(x); }
 
-typedef double td4 __attribute__((ext_vector_type(4)));
-typedef float tf4 __attribute__((ext_vector_type(4)));
-template <typename T> struct TMfma;
-template <> struct TMfma<double> {
-  typedef td4 acc_t;
-  __device__ static acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  /* v_mfma_f64_16x16x4f64: lane l, element r holds D[(l>>4) + 4r][l&15] */
-  __device__ static int drow(int lane, int r) { return (lane >> 4) + 4 * r; }
-};
-template <> struct TMfma<float> {
-  typedef tf4 acc_t;
-  __device__ static acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  /* v_mfma_f32_16x16x4f32: lane l, element r holds D[4(l>>4) + r][l&15] */
-  __device__ static int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
-
 constexpr int PB = 32;
 constexpr int PLD = PB + 1;
 
@@ -60,8 +41,10 @@ template <> struct Rng<float> {
 };
 
 /* sd = sqrt(d) and ri = 1 / sd (d > 0), each within an ulp: the hardware
- * reciprocal square root and two coupled Newton steps (one in FP32), a
- * shorter chain than the library's square root and division; PLAIN: d is in
+ * reciprocal square root and two coupled Newton steps (one in FP32; the
+ * iteration in Markstein, "Software division and square root using
+ * Goldschmidt's algorithms", RNC6, 2004), a shorter chain than the library's
+ * square root and division; PLAIN: d is in
  * the range where no step can over- or underflow.  Outside it, those. */
 template <typename T, bool PLAIN>
 __device__ inline void sqrt_inv(T d, T &sd, T &ri) {

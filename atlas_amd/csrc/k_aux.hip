@@ -6,6 +6,7 @@
 #include <float.h>
 #include <stdint.h>
 #include "kernels.h"
+#include "mfma16.h"
 
 namespace {
 
@@ -26,34 +27,17 @@ constexpr int TNB = ATLMX_TRI_NB;
  * as two products each on the matrix cores, the first one's accumulators
  * (element e of lane group g is row drow(e)) being the operand of the second
  * as they stand.  The products run over the triangles' zeros too, so a block
- * with an infinity or a NaN takes loops over the nonzero range instead.
+ * with an infinity or a NaN, or whose products overflow, takes loops over the
+ * nonzero range instead.
  * One or two blocks (a panel's): 23 -> 15 us; the loops, of one dependent LDS
  * read pair per term, had bound it.
  * ---------------------------------------------------------------------- */
-typedef double iv_d4 __attribute__((ext_vector_type(4)));
-typedef float iv_f4 __attribute__((ext_vector_type(4)));
-template <typename T> struct IvMfma;
-template <> struct IvMfma<double> {
-  typedef iv_d4 acc_t;
-  __device__ static acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  __device__ static int drow(int lane, int r) { return (lane >> 4) + 4 * r; }
-};
-template <> struct IvMfma<float> {
-  typedef iv_f4 acc_t;
-  __device__ static acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  __device__ static int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
-
 /* The doubling levels on the matrix cores.  Ls: the factor, lower, [i][j];
  * Xs: the inverse, zero but for its four 16x16 diagonal blocks on entry.
  * Returns whether this lane formed an entry that is not finite. */
 template <typename T>
 __device__ __forceinline__ int tri_doubling_mfma(const T (*Ls)[TNB + 1], T (*Xs)[TNB + 1]) {
-  typedef IvMfma<T> MF;
+  typedef atlmx::TMfma<T> MF;
   typedef typename MF::acc_t acc_t;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane & 15, lk = lane >> 4;

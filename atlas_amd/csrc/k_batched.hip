@@ -1390,27 +1390,9 @@ hipError_t batch_factor(int kind, int nb, int count, const int *order, const int
  * l>>4, column l&15); over the four sub-steps s4 the slots l>>4 = 0..3 take
  * k = 4 (l>>4) + s4, so the 16 k of a slice are each used once.  The
  * choice of NW is the autotuner's. */
-typedef double bd4 __attribute__((ext_vector_type(4)));
-typedef float bf4 __attribute__((ext_vector_type(4)));
-template <typename T> struct BMfma;
-template <> struct BMfma<double> {
-  typedef bd4 acc_t;
-  __device__ static acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  __device__ static int drow(int lane, int r) { return (lane >> 4) + 4 * r; }
-};
-template <> struct BMfma<float> {
-  typedef bf4 acc_t;
-  __device__ static acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  __device__ static int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
-
 template <typename T, int NW>
 __global__ __launch_bounds__(64 * NW) void gemm_batched_mfma_kernel(GemmBatchArgs<T> g) {
-  typedef BMfma<T> MF;
+  typedef TMfma<T> MF;
   typedef typename MF::acc_t acc_t;
   constexpr int NTH = 64 * NW;
   constexpr int KS = 16;                       /* K slice */

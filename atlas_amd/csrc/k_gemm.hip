@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "kernels.h"
+#include "mfma16.h"
 
 namespace {
 
@@ -33,13 +34,11 @@ constexpr int NT = 256;
 #endif
 constexpr int GROUP_M = ATLMX_GEMM_GROUP_M;
 
-typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef double d2 __attribute__((ext_vector_type(2)));
 
 template <typename T> struct Mfma;
-template <> struct Mfma<double> {
-  typedef d4 acc_t;
+template <> struct Mfma<double> : atlmx::TMfma<double> {
   typedef d2 vec_t;                 /* one 16-byte load */
   typedef d2 __attribute__((aligned(8))) uvec_t;   /* the same from any element address */
   static constexpr int VEC = 2;
@@ -47,14 +46,8 @@ template <> struct Mfma<double> {
   static constexpr int BKS = 16;    /* K slice of the small tiles */
   static constexpr int PADK = 2;    /* LDS row = 18 doubles = 144 B */
   static constexpr int PADR = 2;    /* [k][row] tiles: 130 doubles per k */
-  __device__ static acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  /* v_mfma_f64_16x16x4f64: lane l, element r holds D[(l>>4) + 4r][l&15] */
-  __device__ static int drow(int lane, int r) { return (lane >> 4) + 4 * r; }
 };
-template <> struct Mfma<float> {
-  typedef f4 acc_t;
+template <> struct Mfma<float> : atlmx::TMfma<float> {
   typedef f4 vec_t;
   typedef f4 __attribute__((aligned(4))) uvec_t;
   static constexpr int VEC = 4;
@@ -62,11 +55,6 @@ template <> struct Mfma<float> {
   static constexpr int BKS = 32;
   static constexpr int PADK = 4;    /* LDS row = 20 floats = 80 B */
   static constexpr int PADR = 4;    /* [k][row] tiles: 132 floats per k */
-  __device__ static acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  /* v_mfma_f32_16x16x4f32: lane l, element r holds D[4(l>>4) + r][l&15] */
-  __device__ static int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
 
 template <typename T>

@@ -49,8 +49,8 @@ constexpr int TALL_PARTS = 1024;   /* partial arg-maxes of the tall path */
 /* Record of one workgroup for one column parity: 64-bit words tag << 32 |
  * payload, [0] the candidate's position (INT_MAX: none), [1], [2] the low and
  * high halves of its |value| as a double's bits (0: none, or no nonzero
- * number), [RH + 2j], [RH + 2j + 1] the halves of entry j of the candidate
- * row, j >= the column. */
+ * number), [RH + 2j], [RH + 2j + 1] the halves of the candidate row's entry in
+ * the j-th column from the current one on. */
 constexpr int RH = 4;
 constexpr int RECW = RH + 2 * MAXW;
 using atlmx::u64;

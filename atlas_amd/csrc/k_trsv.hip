@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "kernels.h"
+#include "mfma16.h"
 
 namespace {
 
@@ -293,30 +294,12 @@ hipError_t launch_trsv_tag(int uplo, int trans, int n, int nrhs, const T *A, lon
 constexpr int RC = 16;
 constexpr int RB = 2;     /* 64-row blocks per work item */
 
-template <typename T> struct TMfma;
-template <> struct TMfma<double> {
-  typedef double acc_t __attribute__((ext_vector_type(4)));
-  __device__ static acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  /* v_mfma_f64_16x16x4f64: lane l, element r holds D[(l>>4) + 4r][l&15] */
-  __device__ static int drow(int lane, int r) { return (lane >> 4) + 4 * r; }
-};
-template <> struct TMfma<float> {
-  typedef float acc_t __attribute__((ext_vector_type(4)));
-  __device__ static acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  /* v_mfma_f32_16x16x4f32: lane l, element r holds D[4(l>>4) + r][l&15] */
-  __device__ static int drow(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
-
 template <typename T>
 __global__ __launch_bounds__(NT) void trsm_tag_kernel(int n, int nrhs, int lower, int trans,
                                                       const T *__restrict__ A, long lda,
                                                       const T *__restrict__ inv, T *X, long ldx,
                                                       int *ctl, unsigned long long *pub) {
-  typedef TMfma<T> MF;
+  typedef atlmx::TMfma<T> MF;
   typedef typename MF::acc_t acc_t;
   constexpr int W = Tag<T>::W;
   __shared__ int s_idx;

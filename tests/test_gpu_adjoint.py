@@ -132,8 +132,8 @@ def test_config_size_vs_reference(torch, dt, spd):
 
 @pytest.mark.parametrize("dt", ["f64", "f32"])
 def test_cholesky_solve_order_300(torch, dt):
-    """Orders above 256 take the adjoint kernel's global-scratch branch:
-    forward and both gradients against the numpy reference at n = 300."""
+    """Above order 256: forward and both gradients against the numpy
+    reference at n = 300."""
     from atlas_amd.autograd import CholeskySolve
     rng = np.random.default_rng(31)
     b, n, r = 4, 300, 3
