@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include "mfma16.h"
+#include "wave_argmax.h"
 
 namespace atlmx {
 
@@ -128,30 +129,49 @@ __device__ __forceinline__ int fresh_lane() {
   return l;
 }
 
-/* w <- w inv^T for a tile held as accumulators: out[c][r] = the sum over l of
- * inv(c, l) w(l, r), the inverse (lower) at s_inv[l PLD + c] in LDS.  The
- * products run over the inverse's zeros too, so where a sum is not finite
- * all are formed again over l <= c alone: an infinity or a NaN in column l
- * of the tile's row stays in that row, from column l on, as in a
- * substitution. */
-template <typename T, int RJ>
-__device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][RJ],
-                                               const T *s_inv) {
-  typename TMfma<T>::acc_t out[2][RJ];
+/* acc[c][r] += the sum over l <= c, in blocks of 16, of m(c, l) w(l, r), for
+ * a lower triangle m(c, l) at s_m[l PLD + c]; NEG: of -m(c, l) w(l, r) */
+template <typename T, int RJ, bool NEG>
+__device__ __forceinline__ void tri_times_tile(typename TMfma<T>::acc_t (&acc)[2][RJ],
+                                               const T *s_m,
+                                               const typename TMfma<T>::acc_t (&w)[2][RJ]) {
   const int lane = threadIdx.x & 63, li = lane & 15;
-  zero_tile(out);
 #pragma unroll
   for (int l = 0; l < 2; ++l)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int row = 16 * l + TMfma<T>::drow(lane, e);
 #pragma unroll
-      for (int c = l; c < 2; ++c) {                /* inv(c, l) = 0 above the diagonal */
-        const T a = s_inv[row * PLD + 16 * c + li];
+      for (int c = l; c < 2; ++c) {                /* zero above the diagonal */
+        const T m = s_m[row * PLD + 16 * c + li], a = NEG ? -m : m;
 #pragma unroll
-        for (int r = 0; r < RJ; ++r) out[c][r] = TMfma<T>::mma(a, w[l][r][e], out[c][r]);
+        for (int r = 0; r < RJ; ++r) acc[c][r] = TMfma<T>::mma(a, w[l][r][e], acc[c][r]);
       }
     }
+}
+
+/* w <- w inv^T for a tile held as accumulators: out[c][r] = the sum over l of
+ * inv(c, l) w(l, r), the inverse (lower) at s_inv[l PLD + c] in LDS.
+ *
+ * The product's error grows with the block's condition, which a
+ * substitution's does not (a Gaussian kernel matrix with 1e-10 added to its
+ * diagonal, FP64, order 100: a residual of 530 u against 0.9 u; with 1e-13
+ * the factorization broke down).  refine: the block L (at s_l) is not well
+ * conditioned, and the residual w - out L^T, times inv^T, is added once: as
+ * the error of the first product is at most sqrt(u) for a block that has a
+ * Cholesky factor, that leaves a substitution's (Higham, Accuracy and
+ * Stability, Theorem 12.3).
+ *
+ * The products run over the inverse's zeros too, so where a sum is not finite
+ * all are formed again over l <= c alone: an infinity or a NaN in column l
+ * of the tile's row stays in that row, from column l on, as in a
+ * substitution. */
+template <typename T, int RJ>
+__device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][RJ],
+                                               const T *s_inv, const T *s_l, bool refine) {
+  typename TMfma<T>::acc_t out[2][RJ];
+  zero_tile(out);
+  tri_times_tile<T, RJ, false>(out, s_inv, w);
   bool odd = false;
 #pragma unroll
   for (int c = 0; c < 2; ++c)
@@ -182,6 +202,20 @@ __device__ __forceinline__ void tile_times_inv(typename TMfma<T>::acc_t (&w)[2][
               for (int r = 0; r < RJ; ++r)
                 out[c][r][f] = col >= row ? fma(a, x[r], out[c][r][f]) : out[c][r][f];
             }
+        }
+  } else if (refine) {
+    typename TMfma<T>::acc_t d[2][RJ];
+    tri_times_tile<T, RJ, true>(w, s_l, out);
+    zero_tile(d);
+    tri_times_tile<T, RJ, false>(d, s_inv, w);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int r = 0; r < RJ; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const T v = out[c][r][e] + d[c][r][e];
+          out[c][r][e] = __builtin_isfinite(v) ? v : out[c][r][e];
         }
   }
 #pragma unroll
@@ -260,10 +294,35 @@ __device__ __forceinline__ int block_columns(T (&v)[PB], const T *s_d, int nb) {
   return PLAIN ? !plain : fail;
 }
 
+/* a positive number's upper 32 bits, and the number of those bits alone */
+__device__ __forceinline__ unsigned high_bits(double v) {
+  return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32);
+}
+__device__ __forceinline__ unsigned high_bits(float v) { return (unsigned)__float_as_int(v); }
+template <typename T> __device__ __forceinline__ T from_high_bits(unsigned b);
+template <> __device__ __forceinline__ double from_high_bits<double>(unsigned b) {
+  return __longlong_as_double((long long)((unsigned long long)b << 32));
+}
+template <> __device__ __forceinline__ float from_high_bits<float>(unsigned b) {
+  return __int_as_float((int)b);
+}
+
+/* refine: the largest column sum of |inv(L)| times the largest row norm of L
+ * (the root of A's largest diagonal entry) is above COND, about the condition
+ * from which a product with the inverse leaves a larger residual than a
+ * substitution (kernel matrices of order 48 to 256). */
+constexpr int COND = 16;
 template <typename T>
-__device__ __forceinline__ int block_factor(T (&v)[PB], const T *s_d, int nb) {
-  if (block_columns<T, true>(v, s_d, nb) == 0) return 0;
-  return block_columns<T, false>(v, s_d, nb);
+__device__ __forceinline__ int block_factor(T (&v)[PB], const T *s_d, int nb, bool &refine) {
+  const int lane = fresh_lane();
+  const T dg = s_d[(lane & (PB - 1)) * (PLD + 1)];
+  const T dmax = from_high_bits<T>(wave_umax(high_bits(dg > T(0) ? dg : T(0))));
+  const int fail = block_columns<T, true>(v, s_d, nb) ? block_columns<T, false>(v, s_d, nb) : 0;
+  T sum = T(0);
+#pragma unroll
+  for (int c = 0; c < PB; ++c) sum += fabs(v[c]);
+  refine = __ballot(lane >= PB && !(sum * sum * dmax <= T(COND * COND))) != 0ull;
+  return fail;
 }
 
 }  // namespace atlmx

@@ -271,7 +271,7 @@ __device__ __forceinline__ T quotient(T g, T d, T rd) {
  * order 512 1.1e-7 off against 5.5e-8 with the sum apart, 6.3e-8 before.) */
 /* s_blk: 4 blocks of PB x PLD elements, or 2 where LDS is short (split =
  * false: then wavefront 0 sums the diagonal tile alone); s_x: n x nrhs;
- * s_ctl: 3 */
+ * s_ctl: 4 */
 template <typename T>
 __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, int *info,
                         T *s_blk, bool split, T *s_x, int *s_ctl) {
@@ -322,21 +322,23 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
 
     if (wave == 0) {
       T v[PB];
-      const int fail = block_factor(v, s_d, kb);
+      bool refine;
+      const int fail = block_factor(v, s_d, kb, refine);
       const long lda = fresh(lda0);
       const int ln = fresh_lane();
-      if (ln < PB) {
-        if (!fail && ln < kb) {
+      if (!fail && ln < kb) {
 #pragma unroll
-          for (int c = 0; c < PB; ++c)
-            if (c <= ln) A[(size_t)(k + c) * lda + k + ln] = v[c];
-        }
-      } else {
-#pragma unroll
-        for (int c = 0; c < PB; ++c) s_inv[(ln - PB) * PLD + c] = v[c];
+        for (int c = 0; c < PB; ++c)
+          if (c <= ln) A[(size_t)(k + c) * lda + k + ln] = v[c];
       }
+      /* the rows' lanes L over the block, the columns' the inverse */
+      T *dst = ln < PB ? s_d + ln : s_inv + (ln - PB) * PLD;
+      const int step = ln < PB ? PLD : 1;
+#pragma unroll
+      for (int c = 0; c < PB; ++c) dst[c * step] = ln < c ? T(0) : v[c];
       if (ln == 0) {
         if (fail) s_ctl[2] = k + fail;
+        s_ctl[3] = refine;
         __hip_atomic_store(&s_ctl[0], epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
     }
@@ -371,7 +373,7 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
         while (__hip_atomic_load(&s_ctl[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < epoch)
           __builtin_amdgcn_s_sleep(1);
         if (s_ctl[2]) continue;
-        tile_times_inv<T, 2>(w, s_inv);
+        tile_times_inv<T, 2>(w, s_inv, s_d, s_ctl[3]);
         const long ldc = fresh(lda0);
 #pragma unroll
         for (int c = 0; c < 2; ++c)
@@ -397,7 +399,7 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
         while (__hip_atomic_load(&s_ctl[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < epoch)
           __builtin_amdgcn_s_sleep(1);
         if (s_ctl[2]) continue;
-        tile_times_inv<T, 1>(w, s_inv);
+        tile_times_inv<T, 1>(w, s_inv, s_d, s_ctl[3]);
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -1126,7 +1128,7 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 3) void posv_batched_kerne
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   T *s_blk = (T *)smem;                                /* blocks x PB x PLD */
   T *s_x = s_blk + blocks * PB * PLD;                  /* n x nrhs */
-  __shared__ int s_item, s_ctl[3];
+  __shared__ int s_item, s_ctl[4];
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) s_item = atomicAdd(g.counter, 1);

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
   constexpr int IB = 64;
   if (*info != 0) return;
   __shared__ T s_l[NTILE * TBLK], s_blk[4 * TBLK], s_i[2][TBLK];
-  __shared__ int s_ready, s_fail;
+  __shared__ int s_ready, s_fail, s_refine;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lk = lane >> 4;
@@ -116,7 +116,8 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
     if (wave == 0) {
       T v[PB];
       T *d = tile(p, p);
-      const int fail = block_factor(v, d, min(PB, n - p * PB));
+      bool refine;
+      const int fail = block_factor(v, d, min(PB, n - p * PB), refine);
       const int ln = fresh_lane();
       if (ln < PB) {
         /* on failure the columns before the failing one; so below */
@@ -130,6 +131,7 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
       }
       if (ln == 0) {
         if (fail) s_fail = p * PB + fail;
+        s_refine = refine;
         __hip_atomic_store(&s_ready, p + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
     } else if (p + wave < nt) {                    /* row tile p + wave */
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(NT) void potf2_kernel(int lower, int n, T *A, long 
             w[c][r][e] = x[(16 * c + MF::drow(lane, e)) * PLD + 16 * r + li] - acc[c][r][e];
       while (__hip_atomic_load(&s_ready, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < p + 1)
         __builtin_amdgcn_s_sleep(1);
-      tile_times_inv<T, 2>(w, s_i[p & 1]);
+      tile_times_inv<T, 2>(w, s_i[p & 1], tile(p, p), s_refine);
       const int nc = s_fail ? s_fail - 1 - p * PB : PB;
       if (nc == PB) {
 #pragma unroll

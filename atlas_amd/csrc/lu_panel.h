@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 #include <float.h>
+#include "wave_argmax.h"
 
 namespace atlmx {
 
@@ -21,20 +22,6 @@ template <> struct Lim<float> { __device__ static float safmin() { return FLT_MI
  * halves one after the other with 32-bit DPP maxima; the low half and the
  * positions are looked at only where the higher part ties.  key and pos
  * become the winner's, in every lane. */
-template <int CTRL, int RM>
-__device__ __forceinline__ unsigned dpp_umax(unsigned v) {
-  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RM, 0xf, false);
-  return v > o ? v : o;
-}
-__device__ __forceinline__ unsigned wave_umax(unsigned v) {
-  v = dpp_umax<0x111, 0xf>(v);
-  v = dpp_umax<0x112, 0xf>(v);
-  v = dpp_umax<0x114, 0xf>(v);
-  v = dpp_umax<0x118, 0xf>(v);
-  v = dpp_umax<0x142, 0xa>(v);
-  v = dpp_umax<0x143, 0xc>(v);
-  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
 __device__ __forceinline__ void wave_argmax_key(u64 &key, int &pos) {
   const unsigned hi = (unsigned)(key >> 32), lo = (unsigned)key;
   const unsigned mh = wave_umax(hi);

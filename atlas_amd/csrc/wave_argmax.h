@@ -51,6 +51,22 @@ __device__ __forceinline__ void wave_argmax(double &v, int &i, int &g) {
   g = __builtin_amdgcn_readlane(g, 63);
 }
 
+/* the largest of 64 unsigned values, to every lane, by the same network */
+template <int CTRL, int RM>
+__device__ __forceinline__ unsigned dpp_umax(unsigned v) {
+  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RM, 0xf, false);
+  return v > o ? v : o;
+}
+__device__ __forceinline__ unsigned wave_umax(unsigned v) {
+  v = dpp_umax<0x111, 0xf>(v);
+  v = dpp_umax<0x112, 0xf>(v);
+  v = dpp_umax<0x114, 0xf>(v);
+  v = dpp_umax<0x118, 0xf>(v);
+  v = dpp_umax<0x142, 0xa>(v);
+  v = dpp_umax<0x143, 0xc>(v);
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 }  // namespace atlmx
 
 #endif

@@ -152,3 +152,39 @@ def test_posv_rounding_no_larger_than_by_substitution(n, count):
     err = lambda F: (np.linalg.norm(F - L, axis=(1, 2)) / np.linalg.norm(L, axis=(1, 2))).mean()  # noqa: E731
     F = np.tril(dev.cpu().numpy().transpose(0, 2, 1)).astype(np.float64)
     assert err(F) <= 1.02 * err(_cholesky_by_16(A).astype(np.float64))
+
+
+def _kernel_matrix(rng, n, jitter, dt):
+    """Gaussian kernel of sorted points, nearly singular but for the jitter"""
+    x = np.sort(rng.uniform(0, 10, n))
+    A = (np.exp(-0.5 * (x[:, None] - x) ** 2) + jitter * np.eye(n)).astype(dt)
+    return np.tril(A) + np.tril(A, -1).T
+
+
+@pytest.mark.parametrize("dt,jitter", [(np.float64, 1e-6), (np.float64, 1e-10),
+                                       (np.float64, 1e-13), (np.float32, 1e-3),
+                                       (np.float32, 1e-5)])
+def test_posv_backward_stable_on_kernel_matrices(dt, jitter):
+    """|A - L L^T| <= 8 (n + 1) u |L| |L|^T whatever the condition of the
+    diagonal blocks (Higham, Accuracy and Stability, Theorem 10.3): a product
+    with a block's inverse alone misses it by its condition."""
+    import torch
+    X.use_torch_stream()
+    rng = np.random.default_rng(2)
+    A0 = [_kernel_matrix(rng, n, jitter, dt) for n in (33, 40, 64, 100, 128, 200, 256)]
+    As = [torch.tensor(a, device="cuda") for a in A0]
+    Bs = [torch.tensor(rng.uniform(-1, 1, (2, len(a))).astype(dt), device="cuda") for a in A0]
+    B0 = [b.cpu().numpy().T.astype(np.longdouble) for b in Bs]
+    info = torch.full((len(A0),), -7, dtype=torch.int32, device="cuda")
+    with X.posv_batch(As, Bs, info) as plan:
+        plan.run()
+        torch.cuda.synchronize()
+    assert not info.any()
+    u = np.finfo(dt).eps / 2
+    for a, t, b, b0 in zip(A0, As, Bs, B0):
+        n, A = len(a), a.astype(np.longdouble)
+        L, x = np.tril(t.cpu().numpy().T).astype(np.longdouble), b.cpu().numpy().T
+        assert np.all(np.abs(A - L @ L.T) <= 8 * (n + 1) * u * (np.abs(L) @ np.abs(L).T)), n
+        # two triangular solves on top of the factor's bound
+        bound = 24 * (n + 1) * u * (np.abs(L) @ np.abs(L).T) @ np.abs(x)
+        assert np.all(np.abs(b0 - A @ x.astype(np.longdouble)) <= bound), n

@@ -105,3 +105,19 @@ def test_potrf_failure_leaves_the_columns_before_it_factored(dt, uplo, n, col):
     # c n u kappa(S) |L|, kappa(S) < 8
     assert np.abs(np.tril(F.astype(np.float64) - L)[:, :col - 1]).max(initial=0) <= \
         64 * n * np.finfo(dt).eps
+
+
+@pytest.mark.parametrize("dt,jitter", [(np.float64, 1e-6), (np.float64, 1e-13), (np.float32, 1e-5)])
+@pytest.mark.parametrize("uplo", [X.Lower, X.Upper])
+@pytest.mark.parametrize("n", [33, 64, 100, 128])
+def test_potrf_block_backward_stable_on_kernel_matrices(dt, jitter, uplo, n):
+    """|A - L L^T| <= 8 (n + 1) u |L| |L|^T whatever the condition of the
+    32-column blocks: Gaussian kernel matrices, nearly singular."""
+    x = np.sort(np.random.default_rng(n).uniform(0, 10, n))
+    S = (np.exp(-0.5 * (x[:, None] - x) ** 2) + jitter * np.eye(n)).astype(dt)
+    S = np.tril(S) + np.tril(S, -1).T
+    A = np.asfortranarray(S)
+    assert X.potrf(A, uplo) == 0
+    L = (np.tril(A) if uplo == X.Lower else np.triu(A).T).astype(np.longdouble)
+    u = np.finfo(dt).eps / 2
+    assert np.all(np.abs(S - L @ L.T) <= 8 * (n + 1) * u * (np.abs(L) @ np.abs(L).T))
