@@ -69,8 +69,11 @@ __device__ inline void sqrt_inv(T d, T &sd, T &ri) {
 /* acc[ci][rj] += sum over j in [j0, j1) of Y(16 ci + c, j) X(16 rj + r, j):
  * lane (li, lk) reads Y(16 ci + li, j + lk) at y[ci][(j + lk) ys] and X
  * likewise.  j1 - j0 is a multiple of 4 U; the next U steps' operands are
- * loaded before the current steps' MFMAs. */
-template <typename T, int NC, int RJ, int U>
+ * loaded before the current steps' MFMAs.  MODE: SUM adds every product to
+ * acc; ADD and SUBTRACT sum the 4 U products of a step apart, so that a
+ * product rounds at that sum's size and acc once a step. */
+enum { SUM, ADD, SUBTRACT };
+template <typename T, int NC, int RJ, int U, int MODE = SUM>
 __device__ __forceinline__ void panel_acc(typename TMfma<T>::acc_t (&acc)[NC][RJ],
                                           const T *const (&y)[NC], long ys,
                                           const T *const (&x)[RJ], long xs, int j0, int j1) {
@@ -97,12 +100,25 @@ __device__ __forceinline__ void panel_acc(typename TMfma<T>::acc_t (&acc)[NC][RJ
       for (int r = 0; r < RJ; ++r) xa[u][r] = xc[u][r];
     }
     if (j + 4 * U < j1) load(j + 4 * U);
+    typename TMfma<T>::acc_t t[NC][RJ];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int r = 0; r < RJ; ++r) acc[c][r] = TMfma<T>::mma(ya[u][c], xa[u][r], acc[c][r]);
+        for (int r = 0; r < RJ; ++r) {
+          if (u == 0) t[c][r] = acc[c][r];
+          if (u == 0 && MODE != SUM) t[c][r] = typename TMfma<T>::acc_t{0, 0, 0, 0};
+          t[c][r] = TMfma<T>::mma(ya[u][c], xa[u][r], t[c][r]);
+        }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int r = 0; r < RJ; ++r) {
+        if (MODE == SUM) acc[c][r] = t[c][r];
+        else if (MODE == ADD) acc[c][r] += t[c][r];
+        else acc[c][r] -= t[c][r];
+      }
   }
 }
 

@@ -249,15 +249,16 @@ __device__ __forceinline__ T quotient(T g, T d, T rd) {
 /* Cholesky factor + solve of one instance by one workgroup                */
 /* ---------------------------------------------------------------------- */
 /* Left-looking in panels of PB = 32 columns.  Panel k's 32 x 32 row tiles
- * are each one wavefront's: A's tile less L(rows, 0:k) L(k.., 0:k)^T,
- * accumulated on the matrix cores from the finished columns, then times the
- * diagonal block's inverse, and written once -- no tile of the trailing
- * matrix is read and written again for every panel, as the right-looking
- * form did.  The right-hand sides are one more row tile, [A; B^T], so the
- * forward substitution costs no pass of its own.  Products are formed
- * transposed (D[column][row]): a lane's 16 neighbours run down a column of
- * A, and an accumulator is itself the operand of the product with the
- * inverse (its element e on lane group g is the k index drow(e) there).
+ * are each one wavefront's: A's tile less L(rows, 0:k) L(k.., 0:k)^T on the
+ * matrix cores from the finished columns, then times the diagonal block's
+ * inverse (tile_times_inv: refined where the block is not well conditioned),
+ * and written once -- no tile of the trailing matrix is read and written again
+ * for every panel, as the right-looking form did.  The right-hand sides are
+ * one more row tile, [A; B^T], so the forward substitution costs no pass of
+ * its own.  Products are formed transposed (D[column][row]): a lane's 16
+ * neighbours run down a column of A, and an accumulator is itself the operand
+ * of the product with the inverse (its element e on lane group g is the k
+ * index drow(e) there).
  *
  * What bounds an instance is the chain of panels: the diagonal tile (its
  * sum split over the four wavefronts), its factor and inverse by wavefront 0
@@ -265,10 +266,16 @@ __device__ __forceinline__ T quotient(T g, T d, T rd) {
  * tile meanwhile, and two workgroups share a compute unit (three in FP32).
  * Panels of 64 columns, which read the finished columns half as often, were
  * no faster (4000 of order 8..512: 3.02 against 2.85 ms).  FP64, 4000
- * instances of order 8..512, one right-hand side: 14.4 -> 2.9 ms; 512 of
- * order 256 with 8: 2.17 -> 0.31 ms.  (Starting the accumulators from A's
- * tile saves 32 registers but doubles the rounding error: FP32 factors of
- * order 512 1.1e-7 off against 5.5e-8 with the sum apart, 6.3e-8 before.) */
+ * instances of order 8..512, one right-hand side, with the inputs' copies:
+ * 15.8 -> 3.95 ms; 512 of order 256 with 8: 2.17 -> 0.31 ms.
+ *
+ * Rounding: 16 products at a time (8 in the diagonal tile) are summed apart
+ * and subtracted from A's entry; subtracted one by one, every product would
+ * round at the entry's size, and in one sum over all columns at the size it
+ * had before any.  FP32 factors of order 512: 1.1e-7 off, 6.1e-8 off, and
+ * 4.9e-8 so (updates 16 or 32 columns at a time with substitutions: 7.1e-8);
+ * eigenvalues from 1 to 1e-3, order 256: a residual of 1.92 u in one sum,
+ * 1.07 u so, 1.41 u with the updates. */
 /* s_blk: 4 blocks of PB x PLD elements, or 2 where LDS is short (split =
  * false: then wavefront 0 sums the diagonal tile alone); s_x: n x nrhs;
  * s_ctl: 4 */
@@ -295,7 +302,7 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
       acc_t acc[2][2];
       zero_tile(acc);
       const int w = split ? k / 4 : k;             /* a multiple of 8 */
-      panel_acc<T, 2, 2, 2>(acc, yp, lda, yp, lda, wave * w, wave * w + w);
+      panel_acc<T, 2, 2, 2, ADD>(acc, yp, lda, yp, lda, wave * w, wave * w + w);
       T *sp = s_blk + wave * BLK;
 #pragma unroll
       for (int c = 0; c < 2; ++c)
@@ -356,20 +363,15 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
         const int r0 = k + t * PB;                 /* then kb == PB */
         const int ra = r0 + li, rb = ra + 16;
         const T *xp[2] = {A + min(ra, n - 1), A + min(rb, n - 1)};
-        acc_t acc[2][2], w[2][2];
-        zero_tile(acc);
+        acc_t w[2][2];
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
           for (int r = 0; r < 2; ++r)
 #pragma unroll
-            for (int e = 0; e < 4; ++e)            /* A's tile on its way behind the sum */
+            for (int e = 0; e < 4; ++e)
               w[c][r][e] = xp[r][(size_t)(k + 16 * c + MF::drow(lane, e)) * lda];
-        panel_acc<T, 2, 2, UT>(acc, yp, lda, xp, lda, 0, k);
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-          for (int r = 0; r < 2; ++r) w[c][r] -= acc[c][r];
+        panel_acc<T, 2, 2, UT, SUBTRACT>(w, yp, lda, xp, lda, 0, k);
         while (__hip_atomic_load(&s_ctl[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < epoch)
           __builtin_amdgcn_s_sleep(1);
         if (s_ctl[2]) continue;
@@ -385,17 +387,20 @@ __device__ void wg_posv(int n, T *A, const long lda0, int nrhs, T *B, long ldb, 
           }
       } else {
         const T *xp[1] = {s_x + (size_t)min(li, nrhs - 1) * n};
-        acc_t acc[2][1], w[2][1];
-        zero_tile(acc);
-        panel_acc<T, 2, 1, UT>(acc, yp, lda, xp, 1, 0, k);
+        acc_t w[2][1];
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            /* columns beyond the matrix repeat its last row: dropped */
             const int j = 16 * c + MF::drow(lane, e);
-            w[c][0][e] = j < kb ? xp[0][k + j] - acc[c][0][e] : T(0);
+            w[c][0][e] = j < kb ? xp[0][k + j] : T(0);
           }
+        panel_acc<T, 2, 1, UT, SUBTRACT>(w, yp, lda, xp, 1, 0, k);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)              /* beyond the matrix: its last row again */
+            if (16 * c + MF::drow(lane, e) >= kb) w[c][0][e] = T(0);
         while (__hip_atomic_load(&s_ctl[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < epoch)
           __builtin_amdgcn_s_sleep(1);
         if (s_ctl[2]) continue;

@@ -188,3 +188,28 @@ def test_posv_backward_stable_on_kernel_matrices(dt, jitter):
         # two triangular solves on top of the factor's bound
         bound = 24 * (n + 1) * u * (np.abs(L) @ np.abs(L).T) @ np.abs(x)
         assert np.all(np.abs(b0 - A @ x.astype(np.longdouble)) <= bound), n
+
+
+def test_posv_rounding_on_a_graded_spectrum():
+    """Eigenvalues from 1 to 1e-3: the Schur complements shrink, and a sum
+    carried over all columns before it meets the entry rounds at the entry's
+    first size.  The residual against that of updates 16 columns at a time;
+    2% for the samples' spread."""
+    import torch
+    X.use_torch_stream()
+    n, count = 256, 12
+    rng = np.random.default_rng(8)
+    q = np.linalg.qr(rng.standard_normal((count, n, n)))[0]
+    A = ((q * 1e-3 ** (np.arange(n) / (n - 1))) @ q.transpose(0, 2, 1)).astype(np.float32)
+    A = np.tril(A) + np.tril(A, -1).transpose(0, 2, 1)
+    dev = torch.tensor(A, device="cuda")
+    info = torch.zeros(count, dtype=torch.int32, device="cuda")
+    with X.posv_batch(list(dev), [], info) as plan:
+        plan.run()
+        torch.cuda.synchronize()
+    assert not info.any()
+
+    def resid(F):
+        F = np.tril(F).astype(np.float64)
+        return np.linalg.norm(A - F @ F.transpose(0, 2, 1), axis=(1, 2)).mean()
+    assert resid(dev.cpu().numpy().transpose(0, 2, 1)) <= 1.02 * resid(_cholesky_by_16(A))
