@@ -209,3 +209,44 @@ def test_gesv_nonfinite_entry_stays_below_its_row(dt, bad):
         assert np.abs(f[:32, keep] - R[:32, keep]).max() <= tol, (j, c)
         assert np.abs(f[:j, c] - R[:j, c]).max() <= tol, (j, c)
         assert not np.isfinite(f[j, c])
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("trans", [False, True])
+def test_gesv_backward_stable_where_l11_is_ill_conditioned(dt, trans):
+    """Vandermonde and Gaussian kernel matrices: |P A - L U| <= 4 (n + 1) u
+    |L| |U| (Higham, Accuracy and Stability, Theorem 9.3, with the reciprocals
+    and 4 x 4 inverses) and the solve within twice that more; U12 as a product
+    with inv(L11) misses it by 1e5 here."""
+    import torch
+    X.use_torch_stream()
+    A0 = []
+    for n in (40, 64, 100, 200, 256):
+        x = np.sort(np.random.default_rng(n).uniform(0, 10, n))
+        A0 += [np.vander(np.linspace(-1, 1, n), n).astype(dt),
+               (np.exp(-0.5 * (x[:, None] - x) ** 2) + 1e-5 * np.eye(n)).astype(dt)]
+    B0 = [np.random.default_rng(1).uniform(-1, 1, (len(a), 2)).astype(dt) for a in A0]
+    dev = lambda m: torch.tensor(np.ascontiguousarray(m.T), device="cuda")   # noqa: E731
+    As, Bs = [dev(a) for a in A0], [dev(b) for b in B0]
+    piv = [torch.zeros(len(a), dtype=torch.int32, device="cuda") for a in A0]
+    info = torch.full((len(A0),), -7, dtype=torch.int32, device="cuda")
+    with (X.gesv_t_batch if trans else X.gesv_batch)(As, piv, Bs, info) as plan:
+        plan.run()
+        torch.cuda.synchronize()
+    u = np.finfo(dt).eps / 2
+    tiny = np.finfo(dt).tiny                       # products may underflow
+    for i, (a, t, p, b, b0) in enumerate(zip(A0, As, piv, Bs, B0)):
+        n, F = len(a), t.cpu().numpy().T.astype(np.longdouble)
+        P, rows = a.astype(np.longdouble), np.arange(n)
+        for k, q in enumerate(p.cpu().numpy()):
+            rows[[k, q]] = rows[[q, k]]
+        P = P[rows]
+        L, U = np.tril(F, -1) + np.eye(n), np.triu(F)
+        LU = np.abs(L) @ np.abs(U)
+        assert np.all(np.abs(P - L @ U) <= 4 * (n + 1) * u * LU + n * tiny), n
+        x, b0 = b.cpu().numpy().T.astype(np.longdouble), b0.astype(np.longdouble)
+        if int(info[i]) or not np.isfinite(x).all():   # FP32: numerically singular
+            continue
+        r = np.abs(b0 - P.T @ x[rows]) if trans else np.abs(b0[rows] - P @ x)
+        bound = LU.T @ np.abs(x[rows]) if trans else LU @ np.abs(x)
+        assert np.all(r <= 12 * (n + 1) * u * bound + n * tiny * (1 + np.abs(x).max())), n
