@@ -13,10 +13,10 @@
  * calling thread's stream.
  *
  * The autotuner times every candidate configuration of the LU above order
- * 256 and the GEMM -- panel width 16 or 32, one to three persistent workgroups per CU; for GEMM the kernel
- * (vector FMAs, or MFMA with one or four wavefronts per 64 x 64 tile) and
- * the workgroups per CU -- on a replica of up to AT_SAMPLE instances drawn evenly from the
- * ordered batch (well-conditioned synthetic data of the same sizes, so
+ * 256 (panel width 16 or 32, one to three persistent workgroups per CU) and of
+ * the GEMM (vector FMAs, or MFMA with one or four wavefronts per 64 x 64 tile,
+ * and the workgroups per CU) on a replica of up to AT_SAMPLE instances drawn
+ * evenly from the ordered batch (well-conditioned synthetic data of the same sizes, so
  * tuning never touches the caller's arrays), and keeps the fastest.
  * Results are cached for the process by (kind, precision, nrhs, size
  * buckets), so later plans of a similar shape skip the timing.

@@ -821,7 +821,12 @@ hipError_t launch_small_t(int ta, int tb, GemmArgs<T> &g, hipStream_t s) {
  * its own load latency, so few tiles or a long K take four (FP64 200^3,
  * 32-tile: 9.5 / 7.5 / 7.2 us with 1 / 2 / 4; 300 x 300 x 4000: 188 / 84 /
  * 63; was 645 in 128-tiles), and a full chip with a short K one (64-tile,
- * 8192 x 2048 x 64: 56 / 68 / 111). */
+ * 8192 x 2048 x 64: 56 / 68 / 111).  The lines were drawn from FP64 times and
+ * serve FP32 too, and they count a triangle-masked product's whole rectangle,
+ * of which about half the tiles are live: over 72 SYRK and 110 GEMM shapes of
+ * both precisions none was slower than the 128-tile alone (2%, the spread), but a masked
+ * product of 256 to 500 tiles (n = 2048) keeps the 128-tile where a smaller one
+ * may win. */
 inline double tile_use(long t) { return (double)t / (256.0 * ((t + 255) / 256)); }
 inline int gemm_tile(int M, int N, int K) {
   const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);

@@ -170,9 +170,11 @@ hipError_t atlmx_k_tslu_swap(float *S, long lds, int ebeg, int eend, int gbeg, i
  * Instance i = order[it] for it = 0.. (taken from *counter, zero on entry):
  * n[i], A[i] (lda[i]), ipiv[i] (kind 1, 0-based), nrhs <= ATLMX_BATCH_MAXRHS
  * right-hand sides B[i] (ldb[i]; B may be NULL with nrhs 0), info[i].
- * maxn bounds every n[i] (LDS sizing); nb: panel width 16 or 32; grid:
- * persistent workgroups. */
+ * maxn bounds every n[i] (LDS sizing); nb: panel width 16 or 32, for kind 1
+ * above order ATLMX_BATCH_ROWS (16 where 32 does not fit); grid: persistent
+ * workgroups. */
 #define ATLMX_BATCH_MAXRHS 8
+#define ATLMX_BATCH_ROWS 256  /* largest order of the LU with one panel row per thread */
 hipError_t atlmx_k_dbatch_factor(int kind, int nb, int count, const int *order, const int *n,
                                  double *const *A, const int *lda, int *const *ipiv, int nrhs,
                                  double *const *B, const int *ldb, int *info, int *counter,
@@ -182,8 +184,8 @@ hipError_t atlmx_k_sbatch_factor(int kind, int nb, int count, const int *order, 
                                  float *const *B, const int *ldb, int *info, int *counter,
                                  int maxn, int grid, hipStream_t s);
 /* kind 2 of atlmx_k_?batch_factor: LU as kind 1, then solve A^T X = B. */
-/* Largest order n[i] the factor kernels hold in LDS for kind (0 Cholesky,
- * 1 or 2 LU) and precision (dbl 1: FP64).  Host-only arithmetic. */
+/* Largest order n[i] of a plan of kind (0 Cholesky, 1 or 2 LU) and precision
+ * (dbl 1: FP64); the factor kernels hold it in LDS.  Host only. */
 int atlmx_k_batch_max_order(int kind, int dbl);
 /* Cholesky adjoint of the solve X = A^{-1} B per instance: L (potrf's lower
  * triangle; its strict upper triangle is zeroed), X, Bb = A^{-1} Xb (n x
@@ -204,7 +206,6 @@ hipError_t atlmx_k_sbatch_chol_adjoint(int count, const int *order, const int *n
  * tile_start[p] = first tile of instance order[p] (count + 1 entries).
  * variant: 0 vector FMAs (256 threads per tile), 1 MFMA with one
  * wavefront per tile, 2 MFMA with four wavefronts per tile. */
-#define ATLMX_BATCH_ROWS 256  /* largest order of the LU with one panel row per thread */
 #define ATLMX_BATCH_TILE 64
 hipError_t atlmx_k_dbatch_gemm(int count, int ta, int tb, const int *order, const int *m,
                                const int *n,

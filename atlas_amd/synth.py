@@ -2,10 +2,11 @@
 bench.py and the GPU tests).  Matrices are column-major float64 CUDA
 tensors held as their row-major transposes, like the rest of atlas_amd.
 
-* haar_system: A = U diag(sigma) V^T, U and V Haar-random orthogonal (QR of
+* haar_system: A = V^T U diag(sigma), U and V Haar-random orthogonal (QR of
   a seeded Gaussian, columns sign-fixed by diag(R)), sigma geometric from 1
-  down to 1/kappa; right-hand sides U[-1,1).  The product runs on the
-  library's own DGEMM.
+  down to 1/kappa: an orthogonal matrix with scaled columns, of condition
+  kappa; right-hand sides U[-1,1).  The product runs on the library's own
+  DGEMM.
 * uniform_matrix: U[-1,1) entries from numpy's PCG64 stream (identical on
   every machine), the LU configuration's input.
 * spd_matrix: B B^T / n + I with B standard normal (numpy stream), formed
@@ -31,9 +32,8 @@ def haar_system(n, kappa, nrhs, seed, torch, X):
     U *= sigma.unsqueeze(0)                       # U diag(sigma)
     A = torch.empty(n, n, dtype=torch.float64, device=dev)
     X.use_torch_stream()
-    # Column-major views of the row-major tensors: Vc = V^T, Uc = (U diag s)^T,
-    # and the matrix the library sees in A's storage is A^T = V diag(s) U^T
-    # = Vc^T Uc, whose condition number is kappa as well.
+    # torch.linalg.qr's Q lies column-major in memory, so the library sees V and
+    # U diag(s) themselves, and in A's storage V^T U diag(s).
     X.lib().atlmx_dgemm(X.Trans, X.NoTrans, n, n, n, 1.0, X.dptr(V), n, X.dptr(U), n, 0.0,
                         X.dptr(A), n)
     torch.cuda.synchronize()

@@ -1,10 +1,12 @@
 """Benchmark: FP64-accurate dgesv at n=16384 -- plain FP64 LU vs FP32 LU +
 FP64 iterative refinement -- plus DGEMM %peak, on one MI355X.
 
-Workload (the dense-solve configuration): A = U*diag(sigma)*V^T, n=16384,
-U and V Haar-random orthogonal (QR of a seeded Gaussian, signs fixed by
-diag(R)), sigma geometric from 1 down to 1/kappa (kappa=1e6), one
-right-hand side b ~ U[-1,1).  A step is one full solve of A x = b with the
+Workload (the dense-solve configuration): A = Q*diag(sigma), n=16384,
+Q = V^T U with U and V Haar-random orthogonal (QR of a seeded Gaussian, signs
+fixed by diag(R)), sigma geometric from 1 down to 1/kappa (kappa=1e6), one
+right-hand side b ~ U[-1,1).  The columns of A are orthogonal, so plain
+refinement converges; U*diag(sigma)*V^T of the same kappa needs GMRES and
+takes about twice as long.  A step is one full solve of A x = b with the
 inputs already resident in HBM:
   * plain FP64: copy A, clapack-style getrf + getrs on the GPU;
   * mixed: atlmx_dsgesv (FP32 LU on MFMA, FP64 residual/update/stop test).
@@ -35,7 +37,7 @@ def dgesv_flops(n, nrhs):
 
 
 def make_system(n, kappa, nrhs, seed, torch, X):
-    """A = U diag(sigma) V^T with Haar U, V (QR of Gaussian) and b ~ U[-1,1)."""
+    """A = Q diag(sigma), Q = V^T U with Haar U, V (QR of Gaussian), and b ~ U[-1,1)."""
     from atlas_amd import synth
     return synth.haar_system(n, kappa, nrhs, seed, torch, X)
 
@@ -674,7 +676,7 @@ def main():
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(tmp * 1e3, 3),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f64",
         "data": "synthetic",
-        "config": {"workload": "dgesv n=%d kappa=%g nrhs=%d, A=U diag(s) V^T Haar" %
+        "config": {"workload": "dgesv n=%d kappa=%g nrhs=%d, A=Q diag(s), Q=V^T U Haar" %
                    (n, args.kappa, nrhs), "n": n, "nrhs": nrhs, "kappa": args.kappa,
                    "factor_precision": "fp32" if ok_mp else "fp64"},
         "fp64_dgesv_gflops": round(g64, 2), "fp64_ms_per_step": round(t64 * 1e3, 3),

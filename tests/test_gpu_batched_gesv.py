@@ -3,8 +3,8 @@
 right-hand-side count, zero pivots in every part of a panel, the transposed
 solve, and a batch one order above, which takes the other kernel.  Pivots
 equal the oracle's; |P A - L U| <= gamma_n |L| |U| (Higham, Accuracy and
-Stability, Theorem 9.3, doubled for the product with inv(L11)); the solve by
-its normwise backward error, c n u with c the growth observed (<= 64)."""
+Stability, Theorem 9.3, doubled for the 4 x 4 inverses); the solve by its
+normwise backward error, c n u with c the growth observed (<= 64)."""
 import numpy as np
 import pytest
 
