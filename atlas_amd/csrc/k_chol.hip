@@ -35,7 +35,7 @@ using namespace atlmx;
  * bounds it: four times the one-wavefront factor of 32 columns.  128
  * columns, FP64: 87 us for one barrier-separated step per column, and 15 for
  * the inverses' launch; 71 for both with the tiles in memory; 49 so: 3 for
- * the load, 7 for each panel's factor, 2 to 4 for its products, 4 for the
+ * the load, 6.7 for each panel's factor, 2 to 4 for its products, 4 for the
  * store.  Tiles and column groups beyond the matrix are passed over: one of
  * order 1 takes 6 us (5 in the form with a barrier per step, 13 with the
  * whole block). */
